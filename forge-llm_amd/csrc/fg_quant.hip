@@ -1,4 +1,6 @@
-// Per-token activation quantisers (memory-bound pre-passes of the W8A8 GEMMs): one 256-thread workgroup per row.
+// Per-token and block activation quantisers (memory-bound pre-passes of the W8A8 GEMMs).  16-bit activations in rows of
+// whole 16-byte units take quant_rows_kernel / quant_row_blocks_kernel (one read of x, 16-byte accesses); fp32, ragged
+// or unaligned rows, static scales and tiles of several rows take the element-wise kernels.
 //
 // INT8 (forge/kernels/ref/gemm_int8.py:17-35): s = amax / 127 with IEEE division (1 where amax > 0 is false),
 //   q = clamp(round_half_even(x / s), -127, 127), x / s again IEEE-divided, so codes equal the CPU oracle's bit for
@@ -6,6 +8,8 @@
 // FP8 (forge/kernels/ref/gemm_fp8.py:43-85,130-150): optional fused RMSNorm y = x * (1 / sqrt(mean(x^2) + eps)) * w in
 //   fp32, s = amax(y) / 448 (IEEE; 1 where amax > 0 is false, so NaN rows get scale 1 as in the oracle), or a static
 //   device scale; q = e4m3fn(clamp(y / s, -448, 448)) with gfx950's round-to-nearest-even OCP fp8 conversion.
+#include <algorithm>
+
 #include "fg_device.h"
 
 namespace fg {
@@ -106,6 +110,266 @@ __global__ void __launch_bounds__(256) quant_fp8_rowwise_kernel(const void* __re
     const float c = __builtin_isnan(v) ? v : fminf(fmaxf(v, -448.f), 448.f);
     q[row * ldq + k] = f32_to_e4m3(c);
   }
+}
+
+// ------------------------------------------------------------------------------------------- 16-byte quantisers
+// What bounds these is the latency of one row for few rows and HBM for many.  The element-wise kernels above read x
+// twice (three times with the norm) in 2-byte accesses and divide with the ~12-instruction IEEE sequence: 20.6 us for 32
+// rows of 4096..14336, 79 us for 4096 x 8192 (1.3 TB/s), 24 us for 1024 x 4096 with the norm, and 45 us for 600 x 8192
+// in 1 x 128 blocks (a workgroup per block).  Here a row is read once, 8 values per lane and 16-byte load, and stays in
+// registers; the absolute maximum is a packed 16-bit integer maximum of the bit patterns (their order is the order of
+// magnitudes, a NaN above every number); and the quotient by the row's scale is exact with five multiply-adds.  The same
+// four calls: 4.8, 18.9 (5.3 TB/s), 9.5 and 7.3 us (kernel trace).
+
+// RN(a / b) from y = RN(1 / b): q0 = a y is within two units in the last place, one correction brings it within one,
+// and the second correction of a quotient that close is the correctly rounded one (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990, theorem on division with a fused multiply-add).
+// It holds while no intermediate leaves the normal range: the callers use it for 2^-60 <= b <= 2^60.  There a residual
+// can only lose bits for |a| < 2^-102, where the quotient is below 2^-42 and its code is zero either way.
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+  const float q0 = a * y;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-b, q0, a), y, q0);
+  return __builtin_fmaf(__builtin_fmaf(-b, q1, a), y, q1);
+}
+__device__ __forceinline__ bool div_by_ok(float b) { return b >= 0x1p-60f && b <= 0x1p60f; }
+
+template <bool BF16>
+__device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (BF16) {
+      f[2 * i] = __uint_as_float(w[i] << 16);
+      f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    } else {
+      f[2 * i] = f16_bits_to_f32((uint16_t)w[i]);
+      f[2 * i + 1] = f16_bits_to_f32((uint16_t)(w[i] >> 16));
+    }
+  }
+}
+
+// Largest magnitude among 8 packed 16-bit floats, folded into `m` (two bit patterns, one per half).
+__device__ __forceinline__ uint32_t absmax8(const uint4& u, uint32_t m) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 r = __builtin_bit_cast(u16x2, m);
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r = __builtin_elementwise_max(r, __builtin_bit_cast(u16x2, w[i] & 0x7fff7fffu));
+  return __builtin_bit_cast(uint32_t, r);
+}
+
+// Codes of 8 values as they lie in memory.  `fast`: div_by applies (finite values, a scale in its range).
+template <bool FP8>
+__device__ __forceinline__ uint2 encode8(const float (&v)[8], float scale, float y, bool fast) {
+  float c[8];
+  if (fast) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float q = div_by(v[i], scale, y);
+      // the corrections turn -0 into +0; an e4m3 code keeps the sign of a zero
+      c[i] = FP8 ? __builtin_copysignf(fminf(fmaxf(q, -448.f), 448.f), v[i]) : fminf(fmaxf(q, -127.f), 127.f);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float q = __fdiv_rn(v[i], scale);
+      if (FP8)
+        c[i] = __builtin_isnan(q) ? q : fminf(fmaxf(q, -448.f), 448.f);
+      else
+        c[i] = __builtin_isnan(q) ? 0.f : fminf(fmaxf(q, -127.f), 127.f);
+    }
+  }
+  uint32_t w[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float* d = c + 4 * h;
+    if (FP8) {
+      if (fast) {
+        int p = __builtin_amdgcn_cvt_pk_fp8_f32(d[0], d[1], 0, false);
+        p = __builtin_amdgcn_cvt_pk_fp8_f32(d[2], d[3], p, true);
+        w[h] = (uint32_t)p;
+      } else {
+        w[h] = (uint32_t)f32_to_e4m3(d[0]) | (uint32_t)f32_to_e4m3(d[1]) << 8 | (uint32_t)f32_to_e4m3(d[2]) << 16 |
+               (uint32_t)f32_to_e4m3(d[3]) << 24;
+      }
+    } else {
+      // |d| <= 127: adding 1.5 * 2^23 rounds to the nearest integer, ties to even, and leaves it in the low byte
+      uint32_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(d[i] + 12582912.f);
+      w[h] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u),
+                                   __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), 0x05040100u);
+    }
+  }
+  return make_uint2(w[0], w[1]);
+}
+
+__device__ __forceinline__ void load8_f(const void* p, int dt, int64_t i, float (&f)[8]) {
+  if (dt == FG_F32) {
+    const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
+    const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i + 4);
+    f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
+    f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
+  } else {
+    const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + i);
+    if (dt == FG_BF16) unpack8<true>(u, f);
+    else unpack8<false>(u, f);
+  }
+}
+
+template <bool BF16>
+__device__ __forceinline__ float pattern_f(uint32_t b) {
+  return BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32((uint16_t)b);
+}
+__device__ __forceinline__ bool pattern_nan(bool bf16, uint32_t b) { return b > (bf16 ? 0x7f80u : 0x7c00u); }
+
+// One workgroup per row; thread t holds the row's 16-byte units t, t + T, .. (C of them at most, T threads).
+template <int C, bool BF16, bool FP8, bool RMS>
+__global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                          uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ s,
+                                                          int K, const void* __restrict__ rms_w, int wdt, float eps) {
+  __shared__ uint32_t red[2][16];
+  const int64_t row = blockIdx.x;
+  const int T = blockDim.x, units = K / 8, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = T >> 6;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
+  uint4 u[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int k = threadIdx.x + c * T;
+    u[c] = k < units ? xr[k] : make_uint4(0, 0, 0, 0);
+  }
+  float rs = 1.f;
+  if (RMS) {
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float f[8];
+      unpack8<BF16>(u[c], f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(f[i], f[i], ss);
+    }
+    ss = wave_sum(ss);
+    if (waves > 1) {
+      if (lane == 0) red[0][wave] = __float_as_uint(ss);
+      __syncthreads();
+      ss = 0.f;
+      for (int w = 0; w < waves; ++w) ss += __uint_as_float(red[0][w]);
+    }
+    rs = __fdiv_rn(1.f, __fsqrt_rn(__fdiv_rn(ss, (float)K) + eps));
+  }
+  auto normed = [&](int c, float (&f)[8]) {
+    unpack8<BF16>(u[c], f);
+    if (RMS) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] *= rs;
+      const int k = threadIdx.x + c * T;
+      if (rms_w && k < units) {
+        float g[8];
+        load8_f(rms_w, wdt, (int64_t)k * 8, g);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] *= g[i];
+      }
+    }
+  };
+  uint32_t m = 0;  // bit pattern of the largest magnitude (16-bit without the norm, fp32 with it)
+  if (RMS) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float f[8];
+      normed(c, f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) m = max(m, __float_as_uint(f[i]) & 0x7fffffffu);
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < C; ++c) m = absmax8(u[c], m);
+    m = max(m & 0xffffu, m >> 16);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, kWave));
+  if (waves > 1) {
+    if (lane == 0) red[1][wave] = m;
+    __syncthreads();
+    for (int w = 0; w < waves; ++w) m = max(m, red[1][w]);
+  }
+  const bool nan = RMS ? m > 0x7f800000u : pattern_nan(BF16, m);
+  const float amax = RMS ? __uint_as_float(m) : pattern_f<BF16>(m);
+  const float top = FP8 ? 448.f : 127.f;
+  // torch.amax propagates NaN and `NaN > 0` is false: such rows take scale 1
+  const float scale = (!nan && amax > 0.f) ? __fdiv_rn(amax, top) : 1.f;
+  if (threadIdx.x == 0) s[row] = scale;
+  const bool fast = !nan && div_by_ok(scale);
+  const float y = __fdiv_rn(1.f, scale);
+  uint2* qr = reinterpret_cast<uint2*>(q + row * ldq);
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int k = threadIdx.x + c * T;
+    if (k < units) {
+      float f[8];
+      normed(c, f);
+      qr[k] = encode8<FP8>(f, scale, y, fast);
+    }
+  }
+}
+
+// FP8 in 1 x bk blocks: L = bk / 8 lanes (a power of two up to 64) hold one block, so a wavefront covers 64 / L of them
+// and the amax needs no LDS.
+template <bool BF16>
+__global__ void __launch_bounds__(256) quant_row_blocks_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                               uint8_t* __restrict__ q, int64_t ldq,
+                                                               float* __restrict__ s, int64_t lds, int M, int K,
+                                                               int kb, int log_l) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t block = (uint32_t)(t >> log_l), row = block / (uint32_t)kb, b = block - row * (uint32_t)kb;
+  const int l = (int)(t & ((1 << log_l) - 1)), k = (int)((b << log_l) + l) * 8;
+  const bool in = row < (uint32_t)M && k < K;
+  const uint4 u = in ? *reinterpret_cast<const uint4*>(x + (int64_t)row * ldx + k) : make_uint4(0, 0, 0, 0);
+  uint32_t m = absmax8(u, 0);
+  m = max(m & 0xffffu, m >> 16);
+  for (int off = (1 << log_l) >> 1; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, kWave));
+  const bool nan = pattern_nan(BF16, m);
+  const float amax = pattern_f<BF16>(m);
+  const float scale = (!nan && amax > 0.f) ? __fdiv_rn(amax, 448.f) : 1.f;
+  const bool fast = !nan && div_by_ok(scale);
+  if (!in) return;
+  if (l == 0) s[(int64_t)row * lds + b] = scale;
+  float f[8];
+  unpack8<BF16>(u, f);
+  *reinterpret_cast<uint2*>(q + (int64_t)row * ldq + k) = encode8<true>(f, scale, __fdiv_rn(1.f, scale), fast);
+}
+
+// Whether x and q can be accessed in 16- and 8-byte units: 16-bit values in whole units, aligned rows.
+static bool quant_vec_ok(const void* x, int64_t ldx, int xdt, const void* q, int64_t ldq, int64_t K) {
+  return (xdt == FG_BF16 || xdt == FG_F16) && K % 8 == 0 && ldx % 8 == 0 && ldq % 8 == 0 &&
+         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 8 == 0;
+}
+
+// Threads per row and units per thread: one unit per thread while the rows are too few to fill the CUs (up to two
+// workgroups each; a row's latency counts), else about four (rows in flight count).  Rows past 65536 columns do not
+// fit: returns 0.
+static int quant_rows_plan(int64_t M, int64_t K, int* C) {
+  const int64_t units = K / 8, per = M <= 2 * device_cus() ? 1 : 4;
+  const int64_t t = std::min<int64_t>(1024, ((units + per - 1) / per + kWave - 1) / kWave * kWave);
+  const int64_t c = (units + t - 1) / t;
+  *C = c <= 1 ? 1 : (c <= 2 ? 2 : (c <= 4 ? 4 : 8));
+  return c > 8 ? 0 : (int)t;
+}
+
+template <bool FP8, bool RMS>
+static hipError_t launch_quant_rows(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s, int M,
+                                    int K, int T, int C, const void* rms_w, int wdt, float eps, hipStream_t st) {
+  auto go = [&](auto c_tag, auto bf_tag) {
+    hipLaunchKernelGGL((quant_rows_kernel<decltype(c_tag)::value, decltype(bf_tag)::value, FP8, RMS>), dim3(M), dim3(T),
+                       0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, K, rms_w, wdt, eps);
+    return hipGetLastError();
+  };
+  auto pick = [&](auto bf_tag) {
+    if (C == 1) return go(std::integral_constant<int, 1>{}, bf_tag);
+    if (C == 2) return go(std::integral_constant<int, 2>{}, bf_tag);
+    if (C == 4) return go(std::integral_constant<int, 4>{}, bf_tag);
+    return go(std::integral_constant<int, 8>{}, bf_tag);
+  };
+  return xdt == FG_BF16 ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 // One workgroup per [block_m x block_k] tile: amax over the tile, one scale, then the codes.
@@ -222,6 +486,16 @@ hipError_t launch_quant_fp8_block(const void* x, int64_t ldx, int xdt, uint8_t* 
   const int kb = (K + bk - 1) / bk, mb = (M + bm - 1) / bm;
   const int64_t tiles = (int64_t)kb * mb, per_tile = (int64_t)min(bm, M) * min(bk, K);
   const int64_t cus = device_cus();
+  // one row per block, in units a power of two of lanes holds: 16-byte accesses, several blocks per wavefront
+  if (bm == 1 && !static_scale && bk >= 8 && bk <= 512 && (bk & (bk - 1)) == 0 && tiles < (1LL << 31) &&
+      quant_vec_ok(x, ldx, xdt, q, ldq, K)) {
+    const int log_l = __builtin_ctz((unsigned)bk) - 3;
+    const unsigned grid = (unsigned)(((tiles << log_l) + 255) / 256);
+    auto k = xdt == FG_BF16 ? quant_row_blocks_kernel<true> : quant_row_blocks_kernel<false>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, lds, M, K, kb,
+                       log_l);
+    return hipGetLastError();
+  }
   // one workgroup per tile while the tiles cover the CUs or are small; else parts of 64 Ki elements, up to 4 rounds
   int64_t parts = 1;
   if (tiles < cus && per_tile > 65536) parts = min((per_tile + 65535) / 65536, (4 * cus + tiles - 1) / tiles);
@@ -250,6 +524,11 @@ hipError_t launch_quant_fp8_block(const void* x, int64_t ldx, int xdt, uint8_t* 
 
 hipError_t launch_quant_int8(const void* x, int64_t ldx, int xdt, int8_t* q, int64_t ldq, float* s, int M, int K,
                              hipStream_t st) {
+  int C = 0;
+  const int T = quant_vec_ok(x, ldx, xdt, q, ldq, K) ? quant_rows_plan(M, K, &C) : 0;
+  if (T)
+    return launch_quant_rows<false, false>(x, ldx, xdt, reinterpret_cast<uint8_t*>(q), ldq, s, M, K, T, C, nullptr, 0,
+                                           0.f, st);
   hipLaunchKernelGGL(quant_int8_rowwise_kernel, dim3(M), dim3(256), 0, st, x, ldx, xdt, q, ldq, s, K);
   return hipGetLastError();
 }
@@ -257,6 +536,12 @@ hipError_t launch_quant_int8(const void* x, int64_t ldx, int xdt, int8_t* q, int
 hipError_t launch_quant_fp8(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s, int M, int K,
                             const float* static_scale, const void* rms_w, int wdt, float eps, int fuse,
                             hipStream_t st) {
+  int C = 0;
+  const int T = !static_scale && quant_vec_ok(x, ldx, xdt, q, ldq, K) && reinterpret_cast<uintptr_t>(rms_w) % 16 == 0
+                    ? quant_rows_plan(M, K, &C)
+                    : 0;
+  if (T && fuse) return launch_quant_rows<true, true>(x, ldx, xdt, q, ldq, s, M, K, T, C, rms_w, wdt, eps, st);
+  if (T) return launch_quant_rows<true, false>(x, ldx, xdt, q, ldq, s, M, K, T, C, nullptr, 0, 0.f, st);
   hipLaunchKernelGGL(quant_fp8_rowwise_kernel, dim3(M), dim3(256), 0, st, x, ldx, xdt, q, ldq, s, K, static_scale,
                      rms_w, wdt, eps, fuse);
   return hipGetLastError();
