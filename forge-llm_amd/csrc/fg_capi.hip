@@ -156,6 +156,8 @@ hipError_t launch_fp8_gemm_blocked(const uint8_t* a, int64_t lda, const float* s
                                    const uint8_t* b, int64_t ldb, const float* sb, int64_t sb_sn, int64_t sb_sk,
                                    int sb_div, const void* bias, int bdt, void* y, int64_t ldy, int ydt, int M, int N,
                                    int K, hipStream_t s);
+hipError_t launch_gather(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int M, int K,
+                         hipStream_t s);
 hipError_t launch_quant_int8(const void* x, int64_t ldx, int xdt, int8_t* q, int64_t ldq, float* s, int M, int K,
                              hipStream_t st);
 hipError_t launch_quant_fp8(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s, int M, int K,
@@ -170,12 +172,15 @@ namespace fg {
 
 namespace {
 thread_local char g_kernel[160];
+thread_local bool g_gathered;  // the launch to come reads x as fg_w4_gather_columns left it
 }
 
 void note_kernel(const char* fmt, ...) {
+  const int at = g_gathered ? snprintf(g_kernel, sizeof(g_kernel), "gather_columns + ") : 0;
+  g_gathered = false;
   va_list ap;
   va_start(ap, fmt);
-  vsnprintf(g_kernel, sizeof(g_kernel), fmt, ap);
+  vsnprintf(g_kernel + at, sizeof(g_kernel) - at, fmt, ap);
   va_end(ap);
 }
 
@@ -192,6 +197,7 @@ int fail(int code, const char* fmt, ...) {
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
   g_err = buf;
+  fg::g_gathered = false;
   return code;
 }
 
@@ -692,6 +698,19 @@ int fg_w4a16_gemv_sz8(const void* x, int64_t ldx, int x_dtype, const int32_t* qw
                                            bias, bias_dtype, y, ldy, (int)M, (int)N, (int)K, gs, G == 1,
                                            static_cast<hipStream_t>(stream)),
                     "fg_w4a16_gemv_sz8 launch");
+}
+
+int fg_w4_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int64_t M, int64_t K,
+                         fg_stream_t stream) {
+  if (M < 0 || K <= 0 || M >= kMaxDim || K >= kMaxDim) return fail(FG_EINVAL, "fg_w4_gather_columns: bad sizes");
+  if (M == 0) return FG_OK;
+  if (!x || !perm || !out) return fail(FG_EINVAL, "fg_w4_gather_columns: null tensor");
+  if (ldx < K || ldo < (K + 7) / 8 * 8 || ldo % 8 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0)
+    return fail(FG_EINVAL, "fg_w4_gather_columns: out needs 16-byte aligned rows of at least K rounded up to 8");
+  const int rc = hip_status(fg::launch_gather(x, ldx, perm, out, ldo, (int)M, (int)K, static_cast<hipStream_t>(stream)),
+                            "fg_w4_gather_columns launch");
+  fg::g_gathered = rc == FG_OK;
+  return rc;
 }
 
 int fg_w4_dequant(const int32_t* qweight, int64_t ldq, const void* scales, int scale_dtype, int64_t lds,

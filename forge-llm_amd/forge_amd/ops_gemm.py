@@ -388,6 +388,15 @@ def _w4_operands(packed: PackedW4, capturing: bool) -> _W4Operands:
     return _W4Operands(sorted_[0], perm=sorted_[1])
 
 
+def _gather_columns(x2: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
+    """``x2[:, perm]``, in rows that start on 16 bytes: the activations in a sorted act-order weight's column order."""
+    m, k = x2.shape
+    out = torch.empty((m, (k + 7) // 8 * 8), dtype=x2.dtype, device=x2.device)
+    _check(_lib.lib().fg_w4_gather_columns(_lib.ptr(x2), _ld(x2), _lib.ptr(perm), _lib.ptr(out), out.stride(0), m, k,
+                                           _lib.stream_of(x2)), "fg_w4_gather_columns")
+    return out[:, :k]
+
+
 def _w4_call(x2: torch.Tensor, ops_: _W4Operands, bias: torch.Tensor | None, y: torch.Tensor,
              cfg: _lib.W4Config | None) -> None:
     L = _lib.lib()
@@ -443,6 +452,27 @@ def _w4_cdna4_call(x2: torch.Tensor, p: PackedW4, bias: torch.Tensor | None, y: 
         _lib.stream_of(x2)), "fg_w4a16_gemm_cdna4")
 
 
+def _w4_dispatch(x2: torch.Tensor, packed: PackedW4, b: torch.Tensor | None, y: torch.Tensor,
+                 config: dict[str, Any] | None) -> None:
+    """One call on a weight whose columns lie in group order, through the copies kept beside it where they serve it."""
+    m = x2.shape[0]
+    copy = (_cdna4_copy(packed) if packed.layout.kind == KIND_PORTABLE
+            and CDNA4_COPY_ROWS[0] <= m <= CDNA4_COPY_ROWS[1] else None)
+    blocks = (_sz8_copy(packed) if packed.layout.kind == KIND_PORTABLE and m <= SZ8_ROWS and config is None
+              and forced_impl() is None else None)
+    if blocks is not None and _w4_sz8_call(x2, packed, blocks, b, y):
+        pass
+    elif copy is not None and _cdna4_fits(copy, m, config):
+        _w4_cdna4_call(x2, copy, b, y)
+    elif _cdna4_fits(packed, m, config):
+        _w4_cdna4_call(x2, packed, b, y)
+    else:
+        if packed.layout.kind == KIND_CDNA4:
+            _warn_once("cdna4_copy", "a cdna4_mfma W4 weight met a call its kernel does not take (more than 64 rows, "
+                                     "a forced impl, or its shape): a portable_row copy serves it and is kept")
+        _w4_call(x2, _w4_operands(packed, _capturing(x2)), b, y, _w4_config(config))
+
+
 def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = None, *,
                  config: dict[str, Any] | None = None, deterministic: bool = True) -> torch.Tensor:
     """``y = x @ dequant(W)^T (+ bias)`` for bf16 / fp16 ``x [..., K]`` on a gfx950 GPU; returns ``x.dtype``.
@@ -467,21 +497,14 @@ def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = 
     y = torch.empty((m, packed.n), dtype=x.dtype, device=x.device)
     if m:
         b = None if bias is None else bias.contiguous()
-        copy = (_cdna4_copy(packed) if packed.layout.kind == KIND_PORTABLE
-                and CDNA4_COPY_ROWS[0] <= m <= CDNA4_COPY_ROWS[1] else None)
-        blocks = (_sz8_copy(packed) if packed.layout.kind == KIND_PORTABLE and m <= SZ8_ROWS and config is None
-                  and forced_impl() is None else None)
-        if blocks is not None and _w4_sz8_call(x2, packed, blocks, b, y):
-            pass
-        elif copy is not None and _cdna4_fits(copy, m, config):
-            _w4_cdna4_call(x2, copy, b, y)
-        elif _cdna4_fits(packed, m, config):
-            _w4_cdna4_call(x2, packed, b, y)
+        if packed.g_idx is None or packed.layout.kind == KIND_CDNA4:
+            _w4_dispatch(x2, packed, b, y, config)
         else:
-            if packed.layout.kind == KIND_CDNA4:
-                _warn_once("cdna4_copy", "a cdna4_mfma W4 weight met a call its kernel does not take (more than 64 rows, "
-                                         "a forced impl, or its shape): a portable_row copy serves it and is kept")
-            _w4_call(x2, _w4_operands(packed, _capturing(x2)), b, y, _w4_config(config))
+            ops_ = _w4_operands(packed, _capturing(x2))
+            if ops_.perm is not None:  # regular act order: x in the sorted weight's column order, then any kernel
+                _w4_dispatch(_gather_columns(x2, ops_.perm), ops_.weight, b, y, config)
+            else:
+                _w4_call(x2, ops_, b, y, _w4_config(config))
     _done("w4a16_linear")
     return y.reshape(*x.shape[:-1], packed.n)
 
@@ -932,28 +955,35 @@ class KernelW4A16Linear(_PackedLinear):
 
     def prepare(self) -> KernelW4A16Linear:
         """Host-synchronising preparation (repack, act-order sort) done now, so forward never syncs; runs after
-        ``load_state_dict`` and ``.to()``.  On the GPU a portable_row weight also gets a CDNA4-layout copy for 3..64-row
-        calls (``CDNA4_COPY_ROWS``) and its scales / zero words blocked by 8 channels for 1..2-row calls
-        (``SZ8_ROWS``); the state dict stays portable_row (``FORGE_W4_CDNA4_COPY=0`` / ``FORGE_W4_SZ8_COPY=0`` turn
-        the copies off)."""
+        ``load_state_dict`` and ``.to()``.  On the GPU a portable_row weight (of a regular act-order weight: its
+        column-sorted form) also gets a CDNA4-layout copy for 3..64-row calls (``CDNA4_COPY_ROWS``) and its scales /
+        zero words blocked by 8 channels for 1..2-row calls (``SZ8_ROWS``); the state dict stays portable_row
+        (``FORGE_W4_CDNA4_COPY=0`` / ``FORGE_W4_SZ8_COPY=0`` turn the copies off)."""
+        weight = self.packed()
         if self.g_idx is not None or self.layout.kind != KIND_PORTABLE:
             try:
-                prepare_w4(self.packed())
+                prepare_w4(weight)
             except (ConfigError, RuntimeError) as e:  # forward prepares lazily outside capture
                 log.debug("W4 prepare deferred: %s", e)
-        else:
-            if self._cdna4_copy_wanted():
-                try:
-                    prepare_w4(self.packed(), CDNA4_W4)
-                except (ConfigError, RuntimeError) as e:
-                    log.debug("W4 CDNA4 copy not made: %s", e)
-            if os.environ.get("FORGE_W4_SZ8_COPY", "1") != "0":
-                prepare_w4_sz8(self.packed())
+                return self
+            if self.g_idx is None or self.layout.kind == KIND_CDNA4:
+                return self
+            sorted_ = cached_group_sort(_layout_copy(weight, PORTABLE_W4), compute=False)
+            if not sorted_:
+                return self
+            weight = sorted_[0]
+        if self._cdna4_copy_wanted():
+            try:
+                prepare_w4(weight, CDNA4_W4)
+            except (ConfigError, RuntimeError) as e:
+                log.debug("W4 CDNA4 copy not made: %s", e)
+        if os.environ.get("FORGE_W4_SZ8_COPY", "1") != "0":
+            prepare_w4_sz8(weight)
         return self
 
     def _cdna4_copy_wanted(self) -> bool:
-        """A portable_row weight on the GPU in a shape the CDNA4-layout kernels take."""
-        return (os.environ.get("FORGE_W4_CDNA4_COPY", "1") != "0" and self.qweight.is_cuda and self.g_idx is None
+        """A weight on the GPU in a shape the CDNA4-layout kernels take."""
+        return (os.environ.get("FORGE_W4_CDNA4_COPY", "1") != "0" and self.qweight.is_cuda
                 and self.in_features % 128 == 0 and (self.group_size <= 0 or self.group_size % 128 == 0)
                 and self.scales.dtype in (torch.float16, torch.bfloat16))
 

@@ -160,6 +160,14 @@ int fg_w4a16_gemv_sz8(const void* x, int64_t ldx, int x_dtype, const int32_t* qw
                       void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t n_groups,
                       fg_stream_t stream);
 
+/* Column gather out[m, c] = x[m, perm[c]] of 16-bit activations x [M, K] (row stride ldx): puts x in the column order
+ * of a sorted act-order weight (the role of the gather inside the reference's kernels, forge/kernels/triton/
+ * gemm_w4_fast.py), after which the entry points above take it without a perm.  perm int32 [K], entries in 0..K-1.
+ * out: row stride ldo >= K rounded up to 8, ldo % 8 == 0, 16-byte aligned; columns K .. roundup(K, 8) - 1 of its rows
+ * are written too.  out must not overlap x. */
+int fg_w4_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int64_t M, int64_t K,
+                         fg_stream_t stream);
+
 /* Dense dequantisation out[n,k] = (q - z) * s computed in fp32 and rounded once to out_dtype (FG_F32|FG_F16|FG_BF16).
  * Replaces forge/kernels/triton/gemm_w4_dequant.py:143-191 (w4_dequant) and PackedW4.dequantize
  * (forge/kernels/layouts/w4.py:137-140 -> dequantize_parts :294-305). */

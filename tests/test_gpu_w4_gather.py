@@ -1,0 +1,44 @@
+"""The column gather in front of act-order weights: every element in place, and the whole call against the oracle in the
+kernels it now reaches."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from forge_amd import layouts as L
+from forge_amd import ops_gemm as ops
+from oracle import gemm as og
+from tests._util import assert_close, gen, oracle_packed, to_f32, w4_parts, x_act
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# direct form up to 64 rows and past 32768 columns; LDS form with 1, 2, 4 and 8 units per thread; K off the 8-column unit
+@pytest.mark.parametrize("m,k", [(1, 8), (64, 4096), (65, 1), (65, 4093), (65, 4096), (70, 8192), (66, 14336),
+                                 (65, 32768), (65, 32776), (1500, 520)])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_gather_moves_every_element(m, k, pad):
+    x = torch.randint(-30000, 30000, (m, k + pad), generator=gen(k), dtype=torch.int16).view(torch.bfloat16)
+    x = x.to(DEV)[:, :k]
+    perm = torch.randperm(k, generator=gen(m)).to(torch.int32).to(DEV)
+    out = ops._gather_columns(x, perm)
+    assert torch.equal(out.view(torch.int16), x[:, perm.long()].view(torch.int16)) and out.stride(0) % 8 == 0
+
+
+# the GEMV on blocked scales, the CDNA4 copies, the prefill kernels, and (K % 64 != 0) the tiled kernel
+@pytest.mark.parametrize("m,n,k,gs,kernel", [(1, 1024, 2048, 128, "w4_gemv_split"), (16, 1024, 2048, 128, "w4_frag"),
+                                             (100, 1024, 2048, 64, "w4_big"), (300, 1032, 2048, 128, "w4_pc"),
+                                             (9, 520, 1056, 32, "w4_mfma")])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_act_order_module_reaches_the_policy_kernels(m, n, k, gs, kernel, xdt):
+    q, s, z = w4_parts(n, k, gs, False, seed=m)
+    g_idx = (torch.arange(k) // gs)[torch.randperm(k, generator=gen(k))].to(torch.int32)
+    mod = ops.make_packed_linear("w4a16", packed=L.pack_w4(q, s, z, gs, g_idx=g_idx).to(DEV))
+    x = x_act(m, k, xdt, seed=m + 1)
+    y = mod(x.to(DEV))
+    assert ops.last_kernel().startswith(f"gather_columns + {kernel}"), ops.last_kernel()
+    ref = og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, gs, g_idx))
+    assert_close(y.cpu(), ref, "bfloat16" if xdt == torch.bfloat16 else "float16", what=f"act-order {kernel}")
+    mod.scales.mul_(2)  # the copies of the sorted weight follow the weight's own tensors
+    assert_close(mod(x.to(DEV)).cpu(), 2 * ref, "bfloat16" if xdt == torch.bfloat16 else "float16", what="scaled")
