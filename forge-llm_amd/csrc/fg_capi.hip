@@ -131,6 +131,11 @@ hipError_t launch_fp8_gemm(const uint8_t* a, int64_t lda, const float* sa, int64
                            int64_t ldb, const float* sb, int64_t sb_sn, const void* bias, int bdt, void* y,
                            int64_t ldy, int ydt, int M, int N, int K, int tile, hipStream_t s);
 bool mm_big_ok(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t K);
+bool mm_tail_ok(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t K);
+hipError_t launch_fp8_gemm_blk(const uint8_t* a, int64_t lda, const float* sa, int64_t sa_sm, int64_t sa_sk,
+                               const uint8_t* b, int64_t ldb, const float* sb, int64_t sb_sn, int64_t sb_sk, int sb_div,
+                               const void* bias, int bdt, void* y, int64_t ldy, int ydt, int M, int N, int K, int bm,
+                               int bn, hipStream_t s);
 bool w8_skinny_ok(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K);
 hipError_t launch_int8_gemm_skinny(const int8_t* a, int64_t lda, const float* sa, int64_t sa_len, const int8_t* b,
                                    int64_t ldb, const float* sb, int64_t sb_len, const void* bias, int bdt, void* y,
@@ -138,7 +143,7 @@ hipError_t launch_int8_gemm_skinny(const int8_t* a, int64_t lda, const float* sa
 hipError_t launch_fp8_gemm_skinny(const uint8_t* a, int64_t lda, const float* sa, int64_t sa_sm, const uint8_t* b,
                                   int64_t ldb, const float* sb, int64_t sb_sn, const void* bias, int bdt, void* y,
                                   int64_t ldy, int ydt, int M, int N, int K, hipStream_t s);
-int64_t mm_big_tiles(int64_t M, int64_t N);
+void mm_pick_tile(int64_t M, int64_t N, bool blk, bool wide, int* bm, int* bn);
 hipError_t launch_int8_gemm_big(const int8_t* a, int64_t lda, const float* sa, int64_t sa_len, const int8_t* b,
                                 int64_t ldb, const float* sb, int64_t sb_len, const void* bias, int bdt, void* y,
                                 int64_t ldy, int ydt, int M, int N, int K, hipStream_t s);
@@ -163,6 +168,8 @@ hipError_t launch_quant_int8(const void* x, int64_t ldx, int xdt, int8_t* q, int
 hipError_t launch_quant_fp8(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s, int M, int K,
                             const float* static_scale, const void* rms_w, int wdt, float eps, int fuse,
                             hipStream_t st);
+hipError_t launch_quant_fp8_row_blocks(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s,
+                                       int64_t lds, int64_t ldk, int M, int K, int bk, hipStream_t st);
 hipError_t launch_quant_fp8_block(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s,
                                   int64_t lds, int M, int K, int bm, int bk, const float* static_scale,
                                   hipStream_t st);
@@ -215,50 +222,45 @@ constexpr int64_t kMaxDim = (int64_t)1 << 31;
 // kernel's conditions hold (K % 128 == 0, 16-byte aligned operands with 16-byte multiple leading dimensions), with
 // tile_n (32, 64, 128; 128 only for 128-row tiles) or mm_ring_bn choosing the width, else the register-staged tiled
 // kernel with square tiles.  Tile 16 selects the skinny kernel (M <= 64, K % 256 == 0, same alignment;
-// register-resident split-K).  Returns the tile (16, 64, 128, 256) and sets *ring when the ring kernel runs; -1 for a
-// configuration the operands do not allow, -2 for a tile_m outside 0 / 16 / 64 / 128 / 256.
-int mm_tile(int64_t M, int64_t N, int64_t K, bool int8, const void* a, int64_t lda, const void* b, int64_t ldb,
-            const fg_mm_config* cfg, bool* ring) {
+// register-resident split-K).  The automatic choice takes the 256-row and ring kernels for any K of whole 16-byte units.
+// Returns the tile rows (16, 64, 128, 192, 256) and sets *ring to the tile width when the ring kernel runs (0: another);
+// -1 for a configuration the operands do not allow, -2 for a tile_m outside 0 / 16 / 64 / 128 / 256.
+int mm_tile(int64_t M, int64_t N, int64_t K, bool int8, const void* a, int64_t lda, const void* b, int64_t ldb, int ydt,
+            const fg_mm_config* cfg, int* ring) {
   const bool big_ok = fg::mm_big_ok(a, lda, b, ldb, K);
   const bool skinny_ok = fg::w8_skinny_ok(a, lda, b, ldb, M, N, K);
-  *ring = false;
+  *ring = 0;
   if (cfg && cfg->tile_m) {
     const int t = cfg->tile_m, tn = cfg->tile_n;
     if (t != 16 && t != 64 && t != 128 && t != 256) return -2;
     if ((t == 256 && !big_ok) || (t == 16 && !skinny_ok)) return -1;
     if (t == 64 || t == 128) {
       if (tn && (!big_ok || (t == 64 && tn != 32 && tn != 64 && tn != 128) || (t == 128 && tn != 128))) return -1;
-      *ring = big_ok;
+      if (big_ok) *ring = tn ? tn : fg::mm_ring_bn(M, N, t);
     }
     return t;
   }
-  if (big_ok) {
-    // Measured on the configs' shapes (us, bf16 output, random operands):
-    //  * the skinny kernel for M <= 16 at K >= 16384 (int8 K=28672, N=8192: 45 / 56 at M = 1 / 16 against 58 / 60 for
-    //    the ring kernel), and for M <= 32 where the ring's 64 x 32 tiles would not cover the CUs (int8 K=14336,
-    //    N=4096: 15.3 / 22.6 / 26.0 at M = 4 / 24 / 32 against 29.6-30.1; fp8 K=N=4096: 6.8 / 9.0 against 9.6 / 9.8 at
-    //    M = 4 / 24, level at 32, behind from 48); with the CUs covered the ring kernel is ahead from M = 1 (int8 K=8192,
-    //    N=10240: 20 against 27; fp8 N=8192 at M=16: 17 against 19; int8 N=57344: 96 against 112; K=4096, N=14336 or
-    //    28672: 15.8 / 27.8 against 19.1 / 32.7 at M = 4), and at M = 32..64 everywhere (int8 K=28672, M=64: 63
-    //    against 139);
-    //  * the 256-row kernel once its tiles number 5/8 of the CUs, whatever M (int8 M=1024, K=8192, N=10240: 160 tiles,
-    //    113 against 130 for 128-row ring tiles; K=8192, M=160..224, N=57344: 224 tiles, 146-150 against 180-186
-    //    int8 and 150-156 against 168-180 fp8; M=300..448, N=28672: 118-128 against 131-177; M=640, N=14336: 168
-    //    tiles, 102 against 120); at 112-128 tiles the ring is ahead (fp8 M=1024, K=N=8192, 89 against 117; int8
-    //    K=28672, N=8192, 297 against 353; K=8192, N=28672, M=160..224, 110-124 against 88-96);
-    //  * below that the ring kernel: 128-row tiles once they number 5/8 of the CUs (fp8 M=512: 256 tiles, 47 against
-    //    62 for 64 x 128) unless 64 x 128 tiles fit one per CU (int8 K=8192, N=10240, M=160..192: 240 tiles, 34-35
-    //    against 41; M=224: 320 tiles, 57 against 43), else 64-row tiles (fp8 M=256: 33 against 65 for the
-    //    register-staged 64 x 64 tiles).
-    const int64_t tiles = fg::mm_big_tiles(M, N), cus = fg::device_cus();
-    if (skinny_ok && ((M <= 16 && K >= 16384) || (M <= 32 && (N + 31) / 32 < cus))) return 16;
-    if (8 * tiles >= 5 * cus) return 256;
-    *ring = true;
-    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), t64 = ((M + 63) / 64) * ((N + 127) / 128);
-    return (M > 64 && 8 * t128 >= 5 * cus && t64 > cus) ? 128 : 64;
+  if (big_ok || fg::mm_tail_ok(a, lda, b, ldb, K)) {
+    // The skinny kernel, whose split-K gives few output tiles many wavefronts, for few rows: M <= 16 at K >= 16384
+    // (int8 K=28672, N=8192: 45 / 56 us at M = 1 / 16 against 58 / 60 for the ring kernel), and where 64 x 32 tiles
+    // would leave CUs idle (us, skinny / best ring tile): up to 8 rows if they cover them just once (int8 K=N=8192,
+    // M=4 15.9 / 19.4), up to 16 rows below that (K=14336, N=4096 20.4 / 29.0; K=4096, N=6144 11.4 / 11.3), up to 32
+    // while they cover half (K=14336, N=4096 25.9 / 29.3, K=N=4096 9.8 / 10.8, but N=6144 14.1 / 11.7).
+    const int64_t t32 = (N + 31) / 32, cus = fg::device_cus();
+    if (skinny_ok && ((M <= 16 && K >= 16384) || (M <= 8 && t32 <= cus) || (M <= 16 && t32 < cus) ||
+                      (M <= 32 && 2 * t32 <= cus)))
+      return 16;
+    // INT8 at 33..64 rows over outputs that 256-column tiles spread over 5/8 of the CUs stays on the 256-row kernel, as
+    // tests/test_gpu_w8a8_ring.py states it; 64 x 128 tiles would be ahead there (K=8192, N=57344, M=64: 105 against
+    // 132), as they are for FP8 and fewer rows, which take them.
+    if (int8 && M > 32 && M <= 64 && 8 * ((N + 255) / 256) >= 5 * cus) return 256;
+    int bm, bn;
+    fg::mm_pick_tile(M, N, false, int8 && (ydt == FG_BF16 || ydt == FG_F16), &bm, &bn);
+    if (bn < 256) *ring = bn;
+    return bm;
   }
-  // Unaligned operands or K % 128 != 0: the skinny kernel where it applies and was measured faster, else the
-  // register-staged tiles (64-row while 128-row tiles would leave fewer than two per CU).
+  // Unaligned operands: the skinny kernel where it applies and was measured faster, else the register-staged tiles
+  // (64-row while 128-row tiles would leave fewer than two per CU).
   if (skinny_ok && N < 32768 && (M <= 16 || N < 16384) && !(int8 && M > 32 && K < 16384)) return 16;
   const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
   return (M <= 64 || N <= 64 || tiles128 < 512) ? 64 : 128;
@@ -870,17 +872,16 @@ int fg_int8_gemm(const int8_t* a, int64_t lda, const float* sa, int64_t sa_len, 
     return hip_status(fg::launch_int8_gemv(a, lda, sa, sa_len, b, ldb, sb, sb_len, bias, bias_dtype, y, ldy, y_dtype,
                                            (int)M, (int)N, (int)K, static_cast<hipStream_t>(stream)),
                       "fg_int8_gemm launch");
-  bool ring;
-  const int tile = mm_tile(M, N, K, true, a, lda, b, ldb, cfg, &ring);
+  int ring;
+  const int tile = mm_tile(M, N, K, true, a, lda, b, ldb, y_dtype, cfg, &ring);
   if (tile == -2) return fail(FG_EINVAL, "fg_int8_gemm: tile_m must be 0, 16, 64, 128 or 256, got %d", cfg->tile_m);
   if (tile < 0)
     return fail(FG_EUNSUPPORTED, "fg_int8_gemm: tile_m=256 needs K %% 128 == 0, tile_m=16 M <= 64 and K %% 256 == 0, "
                                  "both 16-byte aligned operands; tile_n (32, 64, 128 for tile_m=64, 128 for "
                                  "tile_m=128) the same");
   if (ring) {
-    const int bn = cfg && cfg->tile_n ? cfg->tile_n : fg::mm_ring_bn(M, N, tile);
     return hip_status(fg::launch_int8_gemm_ring(a, lda, sa, sa_len, b, ldb, sb, sb_len, bias, bias_dtype, y, ldy,
-                                                y_dtype, (int)M, (int)N, (int)K, tile, bn,
+                                                y_dtype, (int)M, (int)N, (int)K, tile, ring,
                                                 static_cast<hipStream_t>(stream)),
                       "fg_int8_gemm launch");
   }
@@ -911,17 +912,16 @@ int fg_fp8_gemm(const uint8_t* a, int64_t lda, const float* sa, int64_t sa_sm, i
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (scale_mode == 0 || scale_mode == 1) {
     if (scale_mode == 0) sa_sm = sb_sn = 0;
-    bool ring;
-    const int tile = mm_tile(M, N, K, false, a, lda, b, ldb, cfg, &ring);
+    int ring;
+    const int tile = mm_tile(M, N, K, false, a, lda, b, ldb, y_dtype, cfg, &ring);
     if (tile == -2) return fail(FG_EINVAL, "fg_fp8_gemm: tile_m must be 0, 16, 64, 128 or 256, got %d", cfg->tile_m);
     if (tile < 0)
       return fail(FG_EUNSUPPORTED, "fg_fp8_gemm: tile_m=256 needs K %% 128 == 0, tile_m=16 M <= 64 and K %% 256 == 0, "
                                    "both 16-byte aligned operands; tile_n (32, 64, 128 for tile_m=64, 128 for "
                                    "tile_m=128) the same");
     if (ring) {
-      const int bn = cfg && cfg->tile_n ? cfg->tile_n : fg::mm_ring_bn(M, N, tile);
-      return hip_status(fg::launch_fp8_gemm_ring(a, lda, sa, sa_sm, b, ldb, sb, sb_sn, bias, bias_dtype, y, ldy,
-                                                 y_dtype, (int)M, (int)N, (int)K, tile, bn, s),
+        return hip_status(fg::launch_fp8_gemm_ring(a, lda, sa, sa_sm, b, ldb, sb, sb_sn, bias, bias_dtype, y, ldy,
+                                                 y_dtype, (int)M, (int)N, (int)K, tile, ring, s),
                         "fg_fp8_gemm launch");
     }
     if (tile == 16)
@@ -939,6 +939,13 @@ int fg_fp8_gemm(const uint8_t* a, int64_t lda, const float* sa, int64_t sa_sm, i
   if (scale_mode == 2) {
     if (block != 128) return fail(FG_EUNSUPPORTED, "fg_fp8_gemm: block scales need block=128, got %d", block);
     if (sb_div != 1 && sb_div != 128) return fail(FG_EINVAL, "fg_fp8_gemm: sb_div must be 1 or the block");
+    if (fg::mm_tail_ok(a, lda, b, ldb, K)) {
+      int bm, bn;
+      fg::mm_pick_tile(M, N, true, false, &bm, &bn);
+      return hip_status(fg::launch_fp8_gemm_blk(a, lda, sa, sa_sm, sa_sk, b, ldb, sb, sb_sn, sb_sk, sb_div, bias,
+                                                bias_dtype, y, ldy, y_dtype, (int)M, (int)N, (int)K, bm, bn, s),
+                        "fg_fp8_gemm launch");
+    }
     return hip_status(fg::launch_fp8_gemm_blocked(a, lda, sa, sa_sm, sa_sk, b, ldb, sb, sb_sn, sb_sk, sb_div, bias,
                                                   bias_dtype, y, ldy, y_dtype, (int)M, (int)N, (int)K, s),
                       "fg_fp8_gemm launch");
@@ -985,6 +992,21 @@ int fg_quant_fp8_block(const void* x, int64_t ldx, int x_dtype, uint8_t* q, int6
   return hip_status(fg::launch_quant_fp8_block(x, ldx, x_dtype, q, ldq, s, lds, (int)M, (int)K, block_m, block_k,
                                                static_scale, static_cast<hipStream_t>(stream)),
                     "fg_quant_fp8_block launch");
+}
+
+int fg_quant_fp8_row_blocks(const void* x, int64_t ldx, int x_dtype, uint8_t* q, int64_t ldq, float* s, int64_t s_row,
+                            int64_t s_block, int64_t M, int64_t K, int32_t block, fg_stream_t stream) {
+  if (M < 0 || K <= 0 || M >= kMaxDim || K >= kMaxDim || block <= 0)
+    return fail(FG_EINVAL, "fg_quant_fp8_row_blocks: bad sizes");
+  if (M == 0) return FG_OK;
+  if (!x || !q || !s) return fail(FG_EINVAL, "fg_quant_fp8_row_blocks: null tensor");
+  if (!is_float_dt(x_dtype)) return fail(FG_EINVAL, "fg_quant_fp8_row_blocks: bad x dtype");
+  if (ldx < K || ldq < K || s_row < 1 || s_block < 1)
+    return fail(FG_EINVAL, "fg_quant_fp8_row_blocks: leading dimensions too small");
+  if (M >= 65536) return fail(FG_EINVAL, "fg_quant_fp8_row_blocks: too many blocks");
+  return hip_status(fg::launch_quant_fp8_row_blocks(x, ldx, x_dtype, q, ldq, s, s_row, s_block, (int)M, (int)K, block,
+                                                    static_cast<hipStream_t>(stream)),
+                    "fg_quant_fp8_row_blocks launch");
 }
 
 }  // extern "C"

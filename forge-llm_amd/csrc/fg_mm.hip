@@ -10,8 +10,8 @@
 // column hit 16 distinct bank quads.  Tiles are ordered so that each XCD (workgroups are dealt round-robin over the
 // 8 XCDs) works on a compact block of output tiles that shares A and B slices in its own L2.
 //
-// Used for outputs that do not fill the 256 x 256 kernel of fg_mm_big.hip (small M or N, K not a multiple of 128,
-// unaligned operands) and for the K-blocked FP8 scale mode.
+// Used for operands that the kernels of fg_mm_big.hip cannot read in 16-byte units (or when a configuration asks for its
+// tiles at such a K).
 #include "fg_mm.h"
 
 namespace fg {
@@ -162,7 +162,10 @@ static hipError_t launch_mm(const uint8_t* A, int64_t lda, const uint8_t* B, int
   const bool aligned = (lda % 16 == 0) && (ldb % 16 == 0) && (K % 16 == 0) &&
                        ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 == 0);
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  auto k = aligned ? mm_kernel<Mma, TM, TN, true, Epi> : mm_kernel<Mma, TM, TN, false, Epi>;
+  auto k = mm_kernel<Mma, TM, TN, false, Epi>;
+  if constexpr (!Epi::kBlocked) {  // aligned operands with K-blocked scales run in mm_blk_kernel
+    if (aligned) k = mm_kernel<Mma, TM, TN, true, Epi>;
+  }
   if (shm > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);

@@ -317,8 +317,8 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __rest
 template <bool BF16>
 __global__ void __launch_bounds__(256) quant_row_blocks_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                uint8_t* __restrict__ q, int64_t ldq,
-                                                               float* __restrict__ s, int64_t lds, int M, int K,
-                                                               int kb, int log_l) {
+                                                               float* __restrict__ s, int64_t lds, int64_t ldk, int M,
+                                                               int K, int kb, int log_l) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const uint32_t block = (uint32_t)(t >> log_l), row = block / (uint32_t)kb, b = block - row * (uint32_t)kb;
   const int l = (int)(t & ((1 << log_l) - 1)), k = (int)((b << log_l) + l) * 8;
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(256) quant_row_blocks_kernel(const uint16_t* _
   const float scale = (!nan && amax > 0.f) ? __fdiv_rn(amax, 448.f) : 1.f;
   const bool fast = !nan && div_by_ok(scale);
   if (!in) return;
-  if (l == 0) s[(int64_t)row * lds + b] = scale;
+  if (l == 0) s[(int64_t)row * lds + b * ldk] = scale;
   float f[8];
   unpack8<BF16>(u, f);
   *reinterpret_cast<uint2*>(q + (int64_t)row * ldq + k) = encode8<true>(f, scale, __fdiv_rn(1.f, scale), fast);
@@ -375,8 +375,9 @@ static hipError_t launch_quant_rows(const void* x, int64_t ldx, int xdt, uint8_t
 // One workgroup per [block_m x block_k] tile: amax over the tile, one scale, then the codes.
 __global__ void __launch_bounds__(256) quant_fp8_block_kernel(const void* __restrict__ x, int64_t ldx, int xdt,
                                                               uint8_t* __restrict__ q, int64_t ldq,
-                                                              float* __restrict__ s, int64_t lds, int M, int K,
-                                                              int bm, int bk, const float* __restrict__ static_scale) {
+                                                              float* __restrict__ s, int64_t lds, int64_t ldk, int M,
+                                                              int K, int bm, int bk,
+                                                              const float* __restrict__ static_scale) {
   __shared__ float red[8];
   __shared__ int nan_flag;
   const int r0 = blockIdx.y * bm, c0 = blockIdx.x * bk;
@@ -399,7 +400,7 @@ __global__ void __launch_bounds__(256) quant_fp8_block_kernel(const void* __rest
     if (has_nan) nan_flag = 1;
     amax = block_reduce(amax, true, red);
     scale = (!nan_flag && amax > 0.f) ? __fdiv_rn(amax, 448.f) : 1.f;
-    if (threadIdx.x == 0) s[(int64_t)blockIdx.y * lds + blockIdx.x] = scale;
+    if (threadIdx.x == 0) s[(int64_t)blockIdx.y * lds + blockIdx.x * ldk] = scale;
   }
   for (int64_t t = threadIdx.x; t < n; t += blockDim.x) {
     const int r = (int)(t / cols), c = (int)(t - (int64_t)r * cols);
@@ -480,28 +481,44 @@ __global__ void __launch_bounds__(256) quant_fp8_tile_encode_kernel(const void* 
   }
 }
 
+// One row per block, 16-byte accesses, several blocks per wavefront: units a power of two of lanes holds.
+static bool quant_row_blocks_ok(const void* x, int64_t ldx, int xdt, const void* q, int64_t ldq, int64_t M, int64_t K,
+                                int64_t bk) {
+  return bk >= 8 && bk <= 512 && (bk & (bk - 1)) == 0 && M * ((K + bk - 1) / bk) < (1LL << 31) &&
+         quant_vec_ok(x, ldx, xdt, q, ldq, K);
+}
+
+// Blocks of 1 x bk, scale of (row, block) at s[row * lds + block * ldk].
+hipError_t launch_quant_fp8_row_blocks(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s,
+                                       int64_t lds, int64_t ldk, int M, int K, int bk, hipStream_t st) {
+  const int kb = (K + bk - 1) / bk;
+  if (quant_row_blocks_ok(x, ldx, xdt, q, ldq, M, K, bk)) {
+    const int log_l = __builtin_ctz((unsigned)bk) - 3;
+    const unsigned grid = (unsigned)((((int64_t)M * kb << log_l) + 255) / 256);
+    auto k = xdt == FG_BF16 ? quant_row_blocks_kernel<true> : quant_row_blocks_kernel<false>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, lds, ldk, M, K,
+                       kb, log_l);
+  } else {
+    hipLaunchKernelGGL(quant_fp8_block_kernel, dim3(kb, M), dim3(256), 0, st, x, ldx, xdt, q, ldq, s, lds, ldk, M, K, 1,
+                       bk, nullptr);
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_quant_fp8_block(const void* x, int64_t ldx, int xdt, uint8_t* q, int64_t ldq, float* s,
                                   int64_t lds, int M, int K, int bm, int bk, const float* static_scale,
                                   hipStream_t st) {
   const int kb = (K + bk - 1) / bk, mb = (M + bm - 1) / bm;
   const int64_t tiles = (int64_t)kb * mb, per_tile = (int64_t)min(bm, M) * min(bk, K);
   const int64_t cus = device_cus();
-  // one row per block, in units a power of two of lanes holds: 16-byte accesses, several blocks per wavefront
-  if (bm == 1 && !static_scale && bk >= 8 && bk <= 512 && (bk & (bk - 1)) == 0 && tiles < (1LL << 31) &&
-      quant_vec_ok(x, ldx, xdt, q, ldq, K)) {
-    const int log_l = __builtin_ctz((unsigned)bk) - 3;
-    const unsigned grid = (unsigned)(((tiles << log_l) + 255) / 256);
-    auto k = xdt == FG_BF16 ? quant_row_blocks_kernel<true> : quant_row_blocks_kernel<false>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, lds, M, K, kb,
-                       log_l);
-    return hipGetLastError();
-  }
+  if (bm == 1 && !static_scale && quant_row_blocks_ok(x, ldx, xdt, q, ldq, M, K, bk))
+    return launch_quant_fp8_row_blocks(x, ldx, xdt, q, ldq, s, lds, 1, M, K, bk, st);
   // one workgroup per tile while the tiles cover the CUs or are small; else parts of 64 Ki elements, up to 4 rounds
   int64_t parts = 1;
   if (tiles < cus && per_tile > 65536) parts = min((per_tile + 65535) / 65536, (4 * cus + tiles - 1) / tiles);
   if (parts == 1) {
-    hipLaunchKernelGGL(quant_fp8_block_kernel, dim3(kb, mb), dim3(256), 0, st, x, ldx, xdt, q, ldq, s, lds, M, K, bm,
-                       bk, static_scale);
+    hipLaunchKernelGGL(quant_fp8_block_kernel, dim3(kb, mb), dim3(256), 0, st, x, ldx, xdt, q, ldq, s, lds,
+                       (int64_t)1, M, K, bm, bk, static_scale);
     return hipGetLastError();
   }
   const dim3 grid(kb, mb, (unsigned)parts);

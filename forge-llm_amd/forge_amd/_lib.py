@@ -79,6 +79,7 @@ SIGNATURES = {
     "fg_quant_int8_rowwise": ([P, I64, INT, P, I64, P, I64, I64, P], INT),
     "fg_quant_fp8_rowwise": ([P, I64, INT, P, I64, P, I64, I64, P, P, INT, F32_, I32_, P], INT),
     "fg_quant_fp8_block": ([P, I64, INT, P, I64, P, I64, I64, I64, I32_, I32_, P, P], INT),
+    "fg_quant_fp8_row_blocks": ([P, I64, INT, P, I64, P, I64, I64, I64, I64, I32_, P], INT),
     "fg_version": ([], ctypes.c_char_p),
     "fg_last_error": ([], ctypes.c_char_p),
     "fg_last_kernel": ([], ctypes.c_char_p),

@@ -619,8 +619,9 @@ def prepare_fp8_scales(sx: torch.Tensor, sw: torch.Tensor, m: int, n: int, k: in
     per tensor; 1: per token and / or per channel; 2: either side K-blocked (1 x ``block`` activations,
     ``block`` x ``block`` or per-channel-per-block weights).  Sizes that do not fit raise ValueError."""
     kb = -(-k // block)
-    a = _act_side(sx.float().contiguous(), m, kb)
-    b = _weight_side(sw.float().contiguous(), n, kb, block)
+    # a 2-D scale is read through its strides as it lies; the others as one dense vector
+    a = _act_side(sx.float() if sx.dim() == 2 else sx.float().contiguous(), m, kb)
+    b = _weight_side(sw.float() if sw.dim() == 2 else sw.float().contiguous(), n, kb, block)
     if a.scalar and b.scalar:
         return 0, a.t, b.t, (0, 0, 0, 0), block
     if not (a.blocked or b.blocked):
@@ -642,6 +643,22 @@ def _fp8_block_quant(x2: torch.Tensor, bm: int, bk: int, static: torch.Tensor | 
             _lib.ptr(x2), _ld(x2), _lib.dtype_code(x2.dtype), _lib.ptr(q), _ld(q), _lib.ptr(s_out), kb, m, k, bm, bk,
             _lib.ptr(None if static is None else s), _lib.stream_of(x2)), "fg_quant_fp8_block")
     return q, s
+
+
+def _fp8_gemm_blocks(x: torch.Tensor, block: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """``quantize_act_fp8(x, granularity="block")`` for a GEMM to read: the same codes and scales, the ``[M, KB]`` scales
+    of one K block next to each other in memory (600 x 8192 x 8192: 79 us against 72 in the GEMM)."""
+    _on_gpu(x, "quantize_act_fp8")
+    x2 = _as_rows(x)
+    m, k = x2.shape
+    q = torch.empty((m, k), dtype=torch.float8_e4m3fn, device=x2.device)
+    s = torch.empty((-(-k // block), m), dtype=torch.float32, device=x2.device)
+    if m:
+        _check(_lib.lib().fg_quant_fp8_row_blocks(
+            _lib.ptr(x2), _ld(x2), _lib.dtype_code(x2.dtype), _lib.ptr(q), _ld(q), _lib.ptr(s), 1, m, m, k, block,
+            _lib.stream_of(x2)), "fg_quant_fp8_row_blocks")
+    _done("quantize_act_fp8")
+    return q.reshape(x.shape), s.t()
 
 
 def _fp8_row_quant(x2: torch.Tensor, static: torch.Tensor | None, rms_weight: torch.Tensor | None,
@@ -765,7 +782,10 @@ def fp8_linear(x: torch.Tensor, w_fp8: torch.Tensor, w_scale: torch.Tensor, bias
             gran = "per_tensor"
         else:
             gran = "per_token"
-        xq, sx = quantize_act_fp8(x, granularity=gran, block=block, scale=x_scale)
+        if gran == "block" and x_scale is None and x.is_floating_point():
+            xq, sx = _fp8_gemm_blocks(x, block)
+        else:
+            xq, sx = quantize_act_fp8(x, granularity=gran, block=block, scale=x_scale)
     _on_gpu(xq, "fp8_linear")
     if xq.dtype != torch.float8_e4m3fn or w_fp8.dtype != torch.float8_e4m3fn:
         raise HardwareUnsupported("fp8_linear: the gfx950 kernels take float8_e4m3fn operands (no e5m2)")

@@ -249,6 +249,12 @@ int fg_quant_fp8_block(const void* x, int64_t ldx, int x_dtype, uint8_t* q, int6
                        int64_t M, int64_t K, int32_t block_m, int32_t block_k, const float* static_scale,
                        fg_stream_t stream);
 
+/* fg_quant_fp8_block with 1 x block tiles and a dynamic scale (block_m = 1, static_scale = NULL): the same codes and
+ * scales, the scale of (row, block) at s[row * s_row + block * s_block].  With s_row = 1 the scales of a K block lie
+ * next to each other, as fg_fp8_gemm reads them fastest (sa_sm = 1, sa_sk = s_block). */
+int fg_quant_fp8_row_blocks(const void* x, int64_t ldx, int x_dtype, uint8_t* q, int64_t ldq, float* s, int64_t s_row,
+                            int64_t s_block, int64_t M, int64_t K, int32_t block, fg_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------------------------
  * Library information.  fg_device_ok replaces the capability gate triton_usable (forge/kernels/ops_gemm.py:159-175):
  * returns 1 when `device` is a gfx950 GPU this build can run on, else 0 (message in fg_last_error).
