@@ -126,16 +126,24 @@ def check(status: int, what: str) -> None:
         raise KernelLaunchError(f"{what} failed (status {status}): {last_error()}", status=status)
 
 
-def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# the current stream's handle without building a torch.cuda.Stream (1.4 us a call), where this torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def stream_of(t: torch.Tensor) -> int:
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def require_device(t: torch.Tensor, op: str) -> None:
     """Raise unless ``t`` lives on a gfx950 GPU this library can run on (checked once per device)."""
+    if t.is_cuda and _DEVICE_OK.get(t.get_device()):
+        return
     if not t.is_cuda:
         raise HardwareUnsupported(f"{op}: forge_amd runs on MI355X (gfx950) GPUs only; got a {t.device.type} tensor "
                                   "(there is no CPU path in this build)")

@@ -63,13 +63,30 @@ _ONCE_LOCK = threading.Lock()
 
 
 # ================================================================================================ switches
+def _env_reader(name: str) -> Callable[[], str]:
+    """A function that reads environment variable ``name`` ("" when unset) as it is now.  Every op asks for several:
+    ``os.environ.get`` encodes the name and decodes the value each time (0.8 us), the mapping behind it holds both as
+    bytes."""
+    data, key = getattr(os.environ, "_data", None), os.fsencode(name)
+    if not isinstance(data, dict):
+        return lambda: os.environ.get(name, "")
+    def read() -> str:
+        value = data.get(key)
+        return "" if value is None else os.fsdecode(value)
+    return read
+
+
+_FORCE_REF, _KERNEL_DEBUG, _W4_IMPL = (_env_reader(v) for v in ("FORGE_FORCE_REF", "FORGE_KERNEL_DEBUG",
+                                                               "FORGE_W4_IMPL"))
+
+
 def force_ref() -> bool:
     """``FORGE_FORCE_REF=1``: the caller asks for the torch oracle, which this build does not ship (ops raise)."""
-    return os.environ.get("FORGE_FORCE_REF", "0") == "1"
+    return _FORCE_REF() == "1"
 
 
 def kernel_debug() -> bool:
-    return os.environ.get("FORGE_KERNEL_DEBUG", "0") == "1"
+    return _KERNEL_DEBUG() == "1"
 
 
 def kernel_strict() -> bool:
@@ -110,12 +127,13 @@ def _warn_once(key: str, message: str) -> None:
 def _ld(t: torch.Tensor) -> int:
     """Row stride handed to the C ABI.  torch calls a one-row tensor contiguous whatever its dim-0 stride, which
     can then be smaller than the row; the row length is the safe stride there."""
-    return int(t.stride(0)) if t.shape[0] > 1 else int(t.shape[1])
+    rows, cols = t.shape
+    return t.stride(0) if rows > 1 else cols
 
 
 def _as_rows(x: torch.Tensor) -> torch.Tensor:
     """``x [..., K]`` as ``[M, K]`` with unit stride along K and rows that do not overlap (copied only if not)."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if x2.stride(-1) == 1 and (x2.shape[0] <= 1 or x2.stride(0) >= x2.shape[1]):
         return x2
     return x2.contiguous()
@@ -150,7 +168,8 @@ def _on_gpu(t: torch.Tensor, op: str) -> None:
         raise HardwareUnsupported(f"{op}: FORGE_FORCE_REF=1 asks for the torch reference path, which forge_amd does "
                                   "not include (run the reference implementation for that)")
     _lib.require_device(t, op)
-    _SELFTEST.ensure(t)
+    if not _SELFTEST.passed(t.get_device()):
+        _SELFTEST.ensure(t)
 
 
 # ================================================================================================ device self-test
@@ -166,6 +185,9 @@ class _SelfTest:
     def __init__(self) -> None:
         self._state: dict[int, str] = {}  # device -> "running" | "ok"
         self._lock = threading.Lock()
+
+    def passed(self, dev: int) -> bool:
+        return self._state.get(dev) == "ok"
 
     def ensure(self, t: torch.Tensor) -> None:
         if os.environ.get("FORGE_AMD_SELFTEST", "1") == "0":
@@ -266,11 +288,14 @@ def forced_impl() -> str | None:
     """``FORGE_W4_IMPL`` = gemv | mfma | prefill | dequant_gemm | generic (the reference's dot / dequant_matmul / legacy
     map to mfma / dequant_gemm / generic; dequant_gemm names the prefill kernels, which fuse the dequantisation into
     the MFMA tiles); anything else means the policy."""
-    return _W4_IMPLS.get(os.environ.get("FORGE_W4_IMPL", "").strip().lower())
+    value = _W4_IMPL()
+    return _W4_IMPLS.get(value.strip().lower()) if value else None
 
 
 def _w4_config(config: dict[str, Any] | None) -> _lib.W4Config | None:
     """The C launch knobs of a W4A16 / W8A16 ``config`` dict (None = the built-in per-shape policy)."""
+    if not config and forced_impl() is None:
+        return None
     c = dict(config or {})
     if c.get("impl") not in _W4_IMPLS:
         raise ConfigError(f"unknown W4A16 impl {c.get('impl')!r}: use gemv, mfma, prefill or generic")
@@ -287,11 +312,20 @@ def _cfg_ref(cfg: Any) -> Any:
     return None if cfg is None else _lib.ctypes.byref(cfg)
 
 
+def _stamp(packed: PackedW4) -> tuple:
+    """What changes whenever one of ``packed``'s tensors is replaced or written."""
+    q, s, z, g = packed.qweight, packed.scales, packed.zeros, packed.g_idx
+    stamp = (q.data_ptr(), q._version, s.data_ptr(), s._version)
+    if z is not None:
+        stamp += (z.data_ptr(), z._version)
+    return stamp if g is None else (*stamp, None, g.data_ptr(), g._version)
+
+
 def _layout_copy(packed: PackedW4, lay: Layout) -> PackedW4:
     """``packed`` in ``lay``: itself, or a repacked copy kept in ``packed.meta`` until its tensors change."""
     if packed.layout.id == lay.id:
         return packed
-    stamp = tuple((t.data_ptr(), t._version) for t in packed.tensors().values())
+    stamp = _stamp(packed)
     copies = packed.meta.setdefault("hip.layout_copies", {})
     hit = copies.get(lay.id)
     if hit is None or hit[0] != stamp:
@@ -324,8 +358,6 @@ SZ8_ROWS = 2
 _SZ8_KEY = "hip.sz8"  # p.meta entry: (tensor stamp, scales8, zeros8)
 
 
-def _stamp(packed: PackedW4) -> tuple:
-    return tuple((t.data_ptr(), t._version) for t in packed.tensors().values())
 
 
 def prepare_w4_sz8(packed: PackedW4) -> bool:
@@ -372,14 +404,16 @@ class _W4Operands:
     g_idx: torch.Tensor | None = None
 
 
-def _w4_operands(packed: PackedW4, capturing: bool) -> _W4Operands:
+def _w4_operands(packed: PackedW4, x: torch.Tensor) -> _W4Operands:
     """What the portable-row kernels read: the portable weight, plus either the sorted weight and its column
     permutation (regular act order) or the per-column ``g_idx`` (irregular act order, or a cold cache under
     capture)."""
     p = _layout_copy(packed, PORTABLE_W4)
     if p.g_idx is None:
         return _W4Operands(p)
-    sorted_ = cached_group_sort(p, compute=not capturing)
+    sorted_ = cached_group_sort(p, compute=False)
+    if sorted_ is MISSING_SORT and not _capturing(x):
+        sorted_ = cached_group_sort(p, compute=True)
     if sorted_ is MISSING_SORT:
         _warn_once("w4_capture", "act-order W4 weight met graph capture unprepared (call prepare_w4 first): the "
                                  "per-column g_idx kernel serves it")
@@ -436,7 +470,7 @@ def _cdna4_copy(packed: PackedW4) -> PackedW4 | None:
     hit = copies.get(CDNA4_W4.id) if copies else None
     if hit is None:
         return None
-    return hit[1] if hit[0] == tuple((t.data_ptr(), t._version) for t in packed.tensors().values()) else None
+    return hit[1] if hit[0] == _stamp(packed) else None
 
 
 def _w4_cdna4_call(x2: torch.Tensor, p: PackedW4, bias: torch.Tensor | None, y: torch.Tensor) -> None:
@@ -456,21 +490,23 @@ def _w4_dispatch(x2: torch.Tensor, packed: PackedW4, b: torch.Tensor | None, y: 
                  config: dict[str, Any] | None) -> None:
     """One call on a weight whose columns lie in group order, through the copies kept beside it where they serve it."""
     m = x2.shape[0]
-    copy = (_cdna4_copy(packed) if packed.layout.kind == KIND_PORTABLE
-            and CDNA4_COPY_ROWS[0] <= m <= CDNA4_COPY_ROWS[1] else None)
-    blocks = (_sz8_copy(packed) if packed.layout.kind == KIND_PORTABLE and m <= SZ8_ROWS and config is None
-              and forced_impl() is None else None)
-    if blocks is not None and _w4_sz8_call(x2, packed, blocks, b, y):
-        pass
-    elif copy is not None and _cdna4_fits(copy, m, config):
-        _w4_cdna4_call(x2, copy, b, y)
+    if packed.layout.kind == KIND_PORTABLE:
+        if m <= SZ8_ROWS:
+            blocks = _sz8_copy(packed) if config is None and forced_impl() is None else None
+            if blocks is not None and _w4_sz8_call(x2, packed, blocks, b, y):
+                return
+        elif CDNA4_COPY_ROWS[0] <= m <= CDNA4_COPY_ROWS[1]:
+            copy = _cdna4_copy(packed)
+            if copy is not None and _cdna4_fits(copy, m, config):
+                _w4_cdna4_call(x2, copy, b, y)
+                return
     elif _cdna4_fits(packed, m, config):
         _w4_cdna4_call(x2, packed, b, y)
-    else:
-        if packed.layout.kind == KIND_CDNA4:
-            _warn_once("cdna4_copy", "a cdna4_mfma W4 weight met a call its kernel does not take (more than 64 rows, "
-                                     "a forced impl, or its shape): a portable_row copy serves it and is kept")
-        _w4_call(x2, _w4_operands(packed, _capturing(x2)), b, y, _w4_config(config))
+        return
+    elif packed.layout.kind == KIND_CDNA4:
+        _warn_once("cdna4_copy", "a cdna4_mfma W4 weight met a call its kernel does not take (more than 64 rows, "
+                                 "a forced impl, or its shape): a portable_row copy serves it and is kept")
+    _w4_call(x2, _w4_operands(packed, x2), b, y, _w4_config(config))
 
 
 def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = None, *,
@@ -500,13 +536,13 @@ def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = 
         if packed.g_idx is None or packed.layout.kind == KIND_CDNA4:
             _w4_dispatch(x2, packed, b, y, config)
         else:
-            ops_ = _w4_operands(packed, _capturing(x2))
+            ops_ = _w4_operands(packed, x2)
             if ops_.perm is not None:  # regular act order: x in the sorted weight's column order, then any kernel
                 _w4_dispatch(_gather_columns(x2, ops_.perm), ops_.weight, b, y, config)
             else:
                 _w4_call(x2, ops_, b, y, _w4_config(config))
     _done("w4a16_linear")
-    return y.reshape(*x.shape[:-1], packed.n)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], packed.n)
 
 
 def w4_dequant(packed: PackedW4, dtype: torch.dtype = torch.float32) -> torch.Tensor:
@@ -558,7 +594,7 @@ def w8a16_linear(x: torch.Tensor, packed: PackedW8, bias: torch.Tensor | None = 
             packed.k, packed.group_size, packed.num_groups, _cfg_ref(cfg), _lib.ptr(ws), ws_bytes,
             _lib.stream_of(x2)), "fg_w8a16_gemm")
     _done("w8a16_linear")
-    return y.reshape(*x.shape[:-1], packed.n)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], packed.n)
 
 
 # ================================================================================================ FP8
@@ -618,6 +654,9 @@ def prepare_fp8_scales(sx: torch.Tensor, sw: torch.Tensor, m: int, n: int, k: in
     ``(mode, sa, sb, (sa_m, sa_k, sb_n, sb_k), sb_div)`` with element strides (0 broadcasts).  Mode 0: both scales
     per tensor; 1: per token and / or per channel; 2: either side K-blocked (1 x ``block`` activations,
     ``block`` x ``block`` or per-channel-per-block weights).  Sizes that do not fit raise ValueError."""
+    if (sx.dim() == 1 and sw.dim() == 1 and sx.dtype == sw.dtype == torch.float32 and sx.numel() == m
+            and sw.numel() == n > 1 and sx.is_contiguous() and sw.is_contiguous()):
+        return 1, sx, sw, (int(m > 1), 0, 1, 0), block  # per token and per channel, as the quantisers write them
     kb = -(-k // block)
     # a 2-D scale is read through its strides as it lies; the others as one dense vector
     a = _act_side(sx.float() if sx.dim() == 2 else sx.float().contiguous(), m, kb)
@@ -658,7 +697,7 @@ def _fp8_gemm_blocks(x: torch.Tensor, block: int) -> tuple[torch.Tensor, torch.T
             _lib.ptr(x2), _ld(x2), _lib.dtype_code(x2.dtype), _lib.ptr(q), _ld(q), _lib.ptr(s), 1, m, m, k, block,
             _lib.stream_of(x2)), "fg_quant_fp8_row_blocks")
     _done("quantize_act_fp8")
-    return q.reshape(x.shape), s.t()
+    return q if x.dim() == 2 else q.reshape(x.shape), s.t()
 
 
 def _fp8_row_quant(x2: torch.Tensor, static: torch.Tensor | None, rms_weight: torch.Tensor | None,
@@ -722,7 +761,7 @@ def quantize_act_fp8(x: torch.Tensor, *, granularity: str = "per_token", block: 
     else:
         raise ConfigError(f"unknown granularity {granularity!r}")
     _done("quantize_act_fp8")
-    return q.reshape(x.shape), s
+    return q if x.dim() == 2 else q.reshape(x.shape), s
 
 
 def quantize_weight_fp8(w: torch.Tensor, granularity: str = "per_channel",
@@ -797,8 +836,9 @@ def fp8_linear(x: torch.Tensor, w_fp8: torch.Tensor, w_scale: torch.Tensor, bias
     y = torch.empty((m, n), dtype=odt, device=xq.device)
     if m:
         try:
-            mode, sa, sb, (sam, sak, sbn, sbk), sb_div = prepare_fp8_scales(sx.to(a.device), sw.to(a.device), m, n, k,
-                                                                            block)
+            dev = a.device
+            mode, sa, sb, (sam, sak, sbn, sbk), sb_div = prepare_fp8_scales(
+                sx if sx.device == dev else sx.to(dev), sw if sw.device == dev else sw.to(dev), m, n, k, block)
         except ValueError as e:
             raise ConfigError(str(e)) from e
         wq = _unit_stride(w_fp8)
@@ -808,7 +848,7 @@ def fp8_linear(x: torch.Tensor, w_fp8: torch.Tensor, w_scale: torch.Tensor, bias
             block, _lib.ptr(b), _code_or_zero(b), _lib.ptr(y), y.stride(0), _lib.dtype_code(odt), m, n, k,
             _cfg_ref(_mm_config(config)), _lib.stream_of(a)), "fg_fp8_gemm")
     _done("fp8_linear")
-    return y.reshape(*xq.shape[:-1], n)
+    return y if xq.dim() == 2 else y.reshape(*xq.shape[:-1], n)
 
 
 # ================================================================================================ INT8
@@ -825,7 +865,7 @@ def quantize_act_int8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         _check(_lib.lib().fg_quant_int8_rowwise(_lib.ptr(x2), _ld(x2), _lib.dtype_code(x2.dtype), _lib.ptr(q), _ld(q),
                                                 _lib.ptr(s), m, k, _lib.stream_of(x2)), "fg_quant_int8_rowwise")
     _done("quantize_act_int8")
-    return q.reshape(x.shape), s
+    return q if x.dim() == 2 else q.reshape(x.shape), s
 
 
 def int8_gemm(xq: torch.Tensor, sx: torch.Tensor | None, wq: torch.Tensor, sw: torch.Tensor | None,
@@ -855,7 +895,7 @@ def int8_gemm(xq: torch.Tensor, sx: torch.Tensor | None, wq: torch.Tensor, sw: t
             _lib.ptr(a), _ld(a), _lib.ptr(sa), 0 if raw else sa.numel(), _lib.ptr(w), _ld(w), _lib.ptr(sb),
             0 if raw else sb.numel(), _lib.ptr(b), _code_or_zero(b), _lib.ptr(y), y.stride(0),
             _lib.dtype_code(out_dtype), m, n, k, _cfg_ref(_mm_config(config)), _lib.stream_of(a)), "fg_int8_gemm")
-    return y.reshape(*xq.shape[:-1], n)
+    return y if xq.dim() == 2 else y.reshape(*xq.shape[:-1], n)
 
 
 def int8_linear(x: torch.Tensor, w_int8: torch.Tensor, w_scale: torch.Tensor, bias: torch.Tensor | None = None, *,
@@ -904,7 +944,8 @@ class _PackedLinear(nn.Module):
         raise NotImplementedError
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self._linear(x, None if self.bias is None else self.bias.to(x.dtype))
+        bias = self.bias
+        return self._linear(x, None if bias is None else bias.to(x.dtype))
 
     @classmethod
     def from_shape(cls, in_features: int, out_features: int, bias: bool = False, dtype: torch.dtype | None = None,
@@ -970,8 +1011,9 @@ class KernelW4A16Linear(_PackedLinear):
         return cls.from_packed(pack_w4(q, s, z, group_size, layout), b)
 
     def packed(self) -> PackedW4:
-        return PackedW4(self.qweight, self.scales, self.zeros, self.layout, self.out_features, self.in_features,
-                        self.group_size, self.g_idx, self._meta)
+        buf = self._buffers  # past nn.Module.__getattr__, which looks a buffer up in four dicts (every forward)
+        return PackedW4(buf["qweight"], buf["scales"], buf["zeros"], self.layout, self.out_features, self.in_features,
+                        self.group_size, buf["g_idx"], self._meta)
 
     def prepare(self) -> KernelW4A16Linear:
         """Host-synchronising preparation (repack, act-order sort) done now, so forward never syncs; runs after
@@ -1054,7 +1096,8 @@ class KernelW8A16Linear(_PackedLinear):
         return cls.from_packed(pack_w8(q, s, group_size), b)
 
     def packed(self) -> PackedW8:
-        return PackedW8(self.qweight, self.scales, PORTABLE_W8, self.out_features, self.in_features, self.group_size)
+        buf = self._buffers
+        return PackedW8(buf["qweight"], buf["scales"], PORTABLE_W8, self.out_features, self.in_features, self.group_size)
 
     def dequantize(self, dtype: torch.dtype | None = None) -> torch.Tensor:
         return self.packed().dequantize(dtype or torch.float32)
