@@ -294,7 +294,7 @@ int fg_device_ok(int device) {
 
 namespace {
 
-// Rows of x from which the policy takes the prefill kernel (64/128/256-row tiles, split-K) over the skinny MFMA
+// Rows of x from which the policy takes the prefill kernels (64/128/256-row tiles, split-K) over the skinny MFMA
 // kernel: measured on the Llama-3-8B shapes, the skinny kernel wins up to 32 rows (and to 64 rows for N, K <= 4096),
 // the prefill kernel from 48 rows (gate+up at M = 64: 1.10 against 0.60 TB/s).
 constexpr int64_t kPrefillMinM = 33;
@@ -312,10 +312,11 @@ bool ring_policy(const fg_w4_config* cfg, int64_t M, int64_t N, int64_t K) {
 // the all-rounder), 2 / 4 / 5 as in the launch switch; 1 (skinny) when `skinny_first`.  tile_n = 256 / 128 / 64
 // forces ping-pong / producer-consumer / all-rounder.  Otherwise from 256 rows: the ping-pong kernel once its tiles
 // come near one per CU (>= 160 of 256 x 256), else the producer / consumer kernel (graph replays over four distinct
-// weights, us, ping-pong / producer-consumer / all-rounder: M = 512 qkv 53.0 / 50.4 / 60.5, o_proj 48.1 / 36.9 / 40.9,
+// weights, us, ping-pong / producer-consumer with 256-row tiles / all-rounder: M = 512 qkv 53.0 / 50.4 / 60.5, o_proj 48.1 / 36.9 / 40.9,
 // gate+up 114.6 / 138.6 / 135.1, down 87.4 / 75.0 / 96.9; M = 2048 qkv 108.9 / 135.2 / 131.0, o_proj 98.3 / 78.4 /
 // 93.4, gate+up 449.5 / 501.7 / 502.3, down 234.8 / 232.5 / 297.4; M = 8192 qkv 367 / 434 / 413, o_proj 246 / 294 /
-// 273, gate+up 1624 / 1916 / 1799, down 779 / 894 / 878); below 256 rows the all-rounder.
+// 273, gate+up 1624 / 1916 / 1799, down 779 / 894 / 878).  Below 256 rows the producer / consumer kernel, whose row tiles
+// follow M (w4_pc_plan), ahead of the all-rounder on every shape measured; that one where neither's conditions hold.
 constexpr int64_t kPpMinTiles = 160;
 int64_t pp_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
 int prefill_kernel(int tile_n, int64_t M, int64_t N, bool pp, bool pc, bool big, bool skinny_first) {
@@ -324,7 +325,7 @@ int prefill_kernel(int tile_n, int64_t M, int64_t N, bool pp, bool pc, bool big,
   if (tile_n == 64 && big) return 2;
   if (skinny_first) return 1;
   if (M >= 256 && pp && pp_tiles(M, N) >= kPpMinTiles) return 5;
-  if (M >= 256 && pc) return 4;
+  if (pc) return 4;
   return big ? 2 : 0;
 }
 
@@ -346,7 +347,7 @@ int w8_pp_split(int64_t M, int64_t N) {
 // (the ping-pong kernel falls back to the producer / consumer kernel, W4 only, and both to the all-rounder).
 size_t prefill_workspace_bytes(int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool w4) {
   const bool pp = tile_n == 256 || (tile_n == 0 && M >= 256 && pp_tiles(M, N) >= kPpMinTiles);
-  const bool pc = w4 && (tile_n == 128 || tile_n == 256 || (tile_n == 0 && M >= 256));
+  const bool pc = w4 && tile_n != 64;
   size_t b = fg::w4_big_workspace_bytes((int)M, (int)N, (int)K, split_k, !w4);
   if (pp) b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k));
   if (!w4 && tile_n == 0 && w8_pp_split(M, N) > 1)
@@ -386,6 +387,8 @@ int plan_w4(int64_t M, int64_t N, int64_t K, int32_t group_size, bool x_aligned,
   const bool mfma_ok = !has_g_idx && q_aligned && x_aligned && (K % 8 == 0);
   // the prefill kernel's shape conditions (an act-order perm, known only at launch, sends the call to MFMA instead)
   const bool prefill_ok = mfma_ok && (K % 64 == 0) && (gs % 32 == 0 || G == 1);
+  // the producer / consumer kernel alone also takes K % 64 == 32 (by the automatic choice)
+  const bool pc_shape = mfma_ok && (K % 32 == 0) && (gs % 32 == 0 || G == 1);
   // FG_W4_DEQUANT_GEMM (the reference's dequant_matmul) names the prefill kernels: they dequantise tiles into LDS and
   // feed them to bf16 / fp16 MFMA, the two steps of that route fused
   int use = impl == FG_W4_DEQUANT_GEMM ? FG_W4_PREFILL : impl;
@@ -416,7 +419,7 @@ int plan_w4(int64_t M, int64_t N, int64_t K, int32_t group_size, bool x_aligned,
     if (wm > p->ws_bytes) p->ws_bytes = wm;
     // the launch picks among the skinny, prefill and tiled MFMA kernels once the operand addresses are known (an
     // act-order perm or misaligned operands rule some out): size the workspace for either split-K kernel
-    if (prefill_ok) {
+    if (prefill_ok || (pc_shape && impl == FG_W4_AUTO)) {
       const size_t wb = prefill_workspace_bytes(cfg ? cfg->tile_n : 0, M, N, K, p->splits, true);
       if (wb > p->ws_bytes) p->ws_bytes = wb;
     }
@@ -529,7 +532,7 @@ int w4a16_run(const void* x, int64_t ldx, int x_dtype, const int32_t* qweight, i
       kern = prefill_kernel(cfg ? cfg->tile_n : 0, M, N, pp, pc, big,
                             auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096);
     else
-      kern = skinny ? 1 : ((auto_impl && big) ? 2 : 0);
+      kern = skinny ? 1 : ((auto_impl && pc) ? 4 : ((auto_impl && big) ? 2 : 0));
     if (ring_policy(cfg, M, N, K) && perm == nullptr &&
         fg::w4_ring_ok(true, x, ldx, qweight, ldq, scales, scale_dtype, lds, zeros, zeros ? ldz : 0, (int)M, N, K, gs,
                        G) &&

@@ -1,11 +1,11 @@
-// W4A16 prefill for large M x N with producer and consumer wavefronts: y[M,N] = x[M,K] @ dequant(W)[N,K]^T (+bias).
+// W4A16 prefill with producer and consumer wavefronts: y[M,N] = x[M,K] @ dequant(W)[N,K]^T (+bias).
 //
-// A workgroup owns a 256 x 128 output tile and walks K in 64-column slices through a three-stage LDS ring.  Its eight
-// wavefronts split the work by role, one of each role per SIMD (wavefronts 0-3 on SIMDs 0-3, 4-7 likewise):
-//   * consumers (wavefronts 0-3, a 2 x 2 grid of 128 x 64 tiles): read A and B fragments from LDS and run
+// A workgroup owns a BM x 128 output tile (BM = 256, 128 or 64; below 256 rows) and walks K in 64-column slices through
+// a three-stage LDS ring.  Its eight wavefronts split the work by role, one of each role per SIMD (wavefronts 0-3 on SIMDs 0-3, 4-7 likewise):
+//   * consumers (wavefronts 0-3, a 2 x 2 grid of BM/2 x 64 tiles): read A and B fragments from LDS and run
 //     v_mfma_f32_16x16x32_{bf16,f16}; they issue no global memory instruction;
 //   * producers (wavefronts 4-7): every global access of the slice is a direct-to-LDS load (global_load_lds, no
-//     registers): the 256 x 64 tile of x (eight 1 KiB loads per producer), the 128 x 64 tile of packed int4 weights
+//     registers): the BM x 64 tile of x (BM / 32 1 KiB loads per producer), the 128 x 64 tile of packed int4 weights
 //     (one 1 KiB load per producer: its own 32 rows), and the scales and zero-point words of those 32 rows (one 4-byte
 //     per lane load); then each producer lane reads back its 16 bytes of packed weights (32 columns of one row),
 //     dequantises them -- (q - z) * s in fp32, exactly the oracle's value (q * s + (-z * s) is exact and the fma
@@ -24,15 +24,17 @@
 // (loads complete in issue order); the direct-to-LDS loads are invisible to the compiler's wait analysis, so those
 // waits are explicit.  Packed weights and scales get two slices (~2 us at full rate) to arrive, x two as well.
 //
-// LDS per stage: x 256 rows x 128 B (16-byte unit c of row r at c ^ (r & 7): conflict-free fragment reads), weight
+// LDS per stage: x BM rows x 128 B (16-byte unit c of row r at c ^ (r & 7): conflict-free fragment reads), weight
 // rows 128 x 128 B (same swizzle), packed-weight staging 4 KiB (producer p's lane l at p * 1024 + 16 l), scale and
-// zero staging 1 KiB (producer p: 32 fp16 scales at p * 256, its 4 zero words at p * 256 + 64).  Three stages:
-// 162816 bytes.
+// zero staging 1 KiB (producer p: 32 fp16 scales at p * 256, its 4 zero words at p * 256 + 64, and 128 bytes further the
+// same of the group of the slice's second 32 columns).  Three stages: 162816 bytes at BM = 256, 113664 and 89088 below.
 //
 // Split-K (gridDim.y > 1): each split covers `kchunk` columns and writes fp32 partials [S, M, N] to the caller's
 // workspace; w4_splitk_reduce_kernel (fg_w4_mfma.hip) sums them in a fixed order and adds the bias.
 //
-// Requirements (w4_pc_ok): K % 64 == 0, group a multiple of 64 (or one group), N % 8 == 0, 16-bit scales with an even
+// A K that ends inside a slice (K % 64 == 32; TAIL) reads zeros in place of x past K.
+//
+// Requirements (w4_pc_ok): K % 32 == 0, group a multiple of 32 (or one group), N % 8 == 0, 16-bit scales with an even
 // row stride, 16-byte aligned x (ldx % 8 == 0) and qweight (ldq % 4 == 0), 4-byte aligned scales, no act-order perm.
 // Rows past M and channels past N read row M - 1 / channel N - 1 and are not stored.
 #include <algorithm>
@@ -46,18 +48,23 @@ typedef _Float16 f16x8_pc_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_pc_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_pc_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_pc_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_pc_t __attribute__((ext_vector_type(2)));
 
-constexpr int kPcBM = 256, kPcBN = 128, kPcBK = 64, kPcRow = 128, kPcThreads = 512;
-constexpr int kPcXBytes = kPcBM * kPcRow;                      // x rows
+constexpr int kPcBN = 128, kPcBK = 64, kPcRow = 128, kPcThreads = 512;
 constexpr int kPcWBytes = kPcBN * kPcRow;                      // dequantised weight rows
 constexpr int kPcQBytes = kPcBN * kPcBK / 2;                   // packed weights of the slice
 constexpr int kPcSBytes = 4 * 256;                             // scales and zero words
-constexpr int kPcStage = kPcXBytes + kPcWBytes + kPcQBytes + kPcSBytes;
-constexpr int kPcLds = 3 * kPcStage;
-static_assert(kPcLds <= 160 * 1024, "the ring exceeds the LDS");
+constexpr int pc_x_bytes(int bm) { return bm * kPcRow; }       // x rows
+constexpr int pc_stage(int bm) { return pc_x_bytes(bm) + kPcWBytes + kPcQBytes + kPcSBytes; }
+constexpr int pc_lds(int bm) { return 3 * pc_stage(bm); }
+static_assert(pc_lds(256) <= 160 * 1024, "the ring exceeds the LDS");
 // direct-to-LDS loads one producer issues per slice: x rows, packed weights, scales + zero words
-constexpr int kPcXI = kPcXBytes / 1024 / 4, kPcQI = 1, kPcSI = 1;
-static_assert(kPcXI == 8, "eight x loads per producer and slice");
+constexpr int pc_xi(int bm) { return pc_x_bytes(bm) / 1024 / 4; }
+constexpr int kPcQI = 1, kPcSI = 1;
+static_assert(pc_xi(256) == 8, "eight x loads per producer and slice");
+
+// What a TAIL launch reads in place of the 16-byte x units past K: zeros, so the weights they meet do not matter.
+static __device__ __align__(16) const uint16_t g_pc_zero[8] = {};
 
 struct PcArgs {
   const uint16_t* x;
@@ -74,8 +81,8 @@ struct PcArgs {
   int64_t ldy;
   int M, N, K;
   int kchunk;        // columns per K split (a multiple of 64)
-  uint32_t gdiv;     // 64-column slices per group (0: one group)
-  uint32_t gmul;     // slice / gdiv = umulhi(slice, gmul) (gdiv > 1)
+  uint32_t gdiv;     // 32-column chunks per group (0: one group)
+  uint32_t gmul;     // chunk / gdiv = umulhi(chunk, gmul) (gdiv > 1)
   int hasz, sbf16, bdt;
 };
 
@@ -106,8 +113,10 @@ __device__ __forceinline__ uint4 pc_frag(const uint8_t* rp, int r16, int lane, i
   return *reinterpret_cast<const uint4*>(rp + c * 16);
 }
 
-template <bool XBF16>
-__global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) w4_pc_kernel(const PcArgs a) {
+template <int BM, bool XBF16, bool TAIL>
+__device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
+  constexpr int kPcBM = BM, kPcXBytes = pc_x_bytes(BM), kPcStage = pc_stage(BM), kPcXI = pc_xi(BM);
+  constexpr int TM = BM / 32;  // 16-row blocks of a consumer
   extern __shared__ __align__(16) uint8_t smem[];
   const int ntm = (a.M + kPcBM - 1) / kPcBM, ntn = (a.N + kPcBN - 1) / kPcBN;
   int tm, tn;
@@ -115,14 +124,20 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
   const int m0 = tm * kPcBM, n0 = tn * kPcBN;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kbeg = blockIdx.y * a.kchunk;
-  const int nk = (min(a.K, kbeg + a.kchunk) - kbeg) / kPcBK;
+  const int nk = (min(a.K, kbeg + a.kchunk) - kbeg + (TAIL ? kPcBK - 1 : 0)) / kPcBK;
 
   if (wave < 4) {
     // ------------------------------------------------------------------------------------------- consumers
+    // Below 256 rows the weights are the MFMA's first operand: a lane's four results are four consecutive channels of one
+    // row of x (row lane % 16 of the block, channels 4 (lane / 16) .. + 3), stored as one unit, which shortens a split
+    // launch's partial stores (K=N=2048, M=384 with four splits 24.0 -> 22.0 us).  With 256 rows x comes first (rows 4
+    // (lane / 16) .. + 3 of channel lane % 16): the other order measured 3-5% slower at row counts that leave most of the
+    // last tile empty (K=14336, N=4096, M=300 62.1 -> 64.4).
+    constexpr bool kWFirst = BM < 256;
     const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15;
-    f32x4_pc_t acc[8][4];
+    f32x4_pc_t acc[TM][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_pc_t{0.f, 0.f, 0.f, 0.f};
     asm volatile("s_barrier" ::: "memory");  // slice 0 is in stage 0
@@ -130,66 +145,86 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
     // around the barrier: k-step 0 of slice t + 1 is read right after the barrier that ends slice t, while the last
     // eight MFMAs of slice t (whose fragments are already in registers) run, so a consumer -- the only MFMA issuer of
     // its SIMD -- does not sit out the LDS latency at the top of every slice.
-    uint4 fa0[8], fb0[4], fa1[8], fb1[4];
-    auto read_ks = [&](const uint8_t* st, int s, uint4 (&fa)[8], uint4 (&fb)[4]) __attribute__((always_inline)) {
-      const uint8_t* sA = st + (wm * 128 + r16) * kPcRow;
+    uint4 fa0[TM], fb0[4], fa1[TM], fb1[4];
+    auto read_ks = [&](const uint8_t* st, int s, uint4 (&fa)[TM], uint4 (&fb)[4]) __attribute__((always_inline)) {
+      const uint8_t* sA = st + (wm * (BM / 2) + r16) * kPcRow;
       const uint8_t* sB = st + kPcXBytes + (wn * 64 + r16) * kPcRow;
 #pragma unroll
       for (int j = 0; j < 4; ++j) fb[j] = pc_frag(sB + j * 16 * kPcRow, r16, lane, s);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) fa[i] = pc_frag(sA + i * 16 * kPcRow, r16, lane, s);
+      for (int i = 0; i < TM; ++i) fa[i] = pc_frag(sA + i * 16 * kPcRow, r16, lane, s);
     };
-    auto mfma_rows = [&](int i0, int i1, const uint4 (&fa)[8], const uint4 (&fb)[4]) __attribute__((always_inline)) {
+    auto mfma_rows = [&](int i0, int i1, const uint4 (&fa)[TM], const uint4 (&fb)[4]) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = i0; i < i1; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = pc_mfma<XBF16>(fa[i], fb[j], acc[i][j]);
+        for (int j = 0; j < 4; ++j) acc[i][j] = kWFirst ? pc_mfma<XBF16>(fb[j], fa[i], acc[i][j]) : pc_mfma<XBF16>(fa[i], fb[j], acc[i][j]);
     };
     const uint8_t* st = smem;
     read_ks(st, 0, fa0, fb0);
     for (int t = 0; t < nk; ++t) {
       read_ks(st, 1, fa1, fb1);
-      mfma_rows(0, 8, fa0, fb0);
-      mfma_rows(0, 6, fa1, fb1);
+      mfma_rows(0, TM, fa0, fb0);
+      mfma_rows(0, TM - 2, fa1, fb1);
       // this stage's fragments are in registers before the barrier lets the producers refill it
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       st = st == smem + 2 * kPcStage ? smem : st + kPcStage;
       read_ks(st, 0, fa0, fb0);  // slice t + 1 (past the last slice: a stage no one writes any more, unused)
       __builtin_amdgcn_sched_barrier(0);
-      mfma_rows(6, 8, fa1, fb1);
+      mfma_rows(TM - 2, TM, fa1, fb1);
       __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_barrier" ::: "memory");  // the producers' last loads have drained: the ring is free
 
-    const int mw = m0 + wm * 128, nw = n0 + wn * 64;
+    const int mw = m0 + wm * (BM / 2), nw = n0 + wn * 64, n4 = 4 * (lane >> 4);
     if (gridDim.y > 1) {  // fp32 partials of this split
+      // a unit of four lies in one row, 16-byte aligned
+      const bool v4 = kWFirst && a.N % 4 == 0 && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0;
+      float* const part = a.ws + (int64_t)blockIdx.y * a.M * a.N;
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j) {
+          const int m = mw + i * 16 + (kWFirst ? r16 : n4), n = nw + j * 16 + (kWFirst ? n4 : r16);
+          if (v4) {
+            if (m < a.M && n < a.N) *reinterpret_cast<f32x4_pc_t*>(part + (int64_t)m * a.N + n) = acc[i][j];
+          } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int m = mw + i * 16 + 4 * (lane >> 4) + e, n = nw + j * 16 + (lane & 15);
-            if (m < a.M && n < a.N) a.ws[((int64_t)blockIdx.y * a.M + m) * a.N + n] = acc[i][j][e];
+            for (int e = 0; e < 4; ++e) {
+              const int me = m + (kWFirst ? 0 : e), ne = n + (kWFirst ? e : 0);
+              if (me < a.M && ne < a.N) part[(int64_t)me * a.N + ne] = acc[i][j][e];
+            }
           }
+        }
       return;
     }
     // 16-bit output through a per-wavefront LDS slab of 16 rows x 64 columns, stored as 16-byte row segments
     constexpr int SP = 64 + 8;
     uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * 16 * SP;
-    float cb[4];
+    float cb[4][kWFirst ? 4 : 1];  // bias of the lane's channels
 #pragma unroll
-    for (int j = 0; j < 4; ++j) cb[j] = a.bias ? load_f(a.bias, a.bdt, min(nw + j * 16 + (lane & 15), a.N - 1)) : 0.f;
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < (kWFirst ? 4 : 1); ++e)
+        cb[j][e] = a.bias ? load_f(a.bias, a.bdt, min(nw + j * 16 + (kWFirst ? n4 + e : r16), a.N - 1)) : 0.f;
     const bool vec_ok = (a.ldy % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) % 16) == 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j) {
+        uint32_t h[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float v = a.bias ? acc[i][j][e] + cb[j] : acc[i][j][e];
-          slab[(4 * (lane >> 4) + e) * SP + j * 16 + (lane & 15)] = XBF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
+          const float v = a.bias ? acc[i][j][e] + cb[j][kWFirst ? e : 0] : acc[i][j][e];
+          h[e] = XBF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
         }
+        if constexpr (kWFirst) {
+          *reinterpret_cast<uint2*>(slab + r16 * SP + j * 16 + n4) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) slab[(n4 + e) * SP + j * 16 + r16] = (uint16_t)h[e];
+        }
+      }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's slab writes are done before it reads them
 #pragma unroll
       for (int u0 = 0; u0 < 16 * 64 / 8; u0 += 64) {
@@ -214,49 +249,58 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
 
   // --------------------------------------------------------------------------------------------- producers
   const int p = wave - 4;
-  // x: load i of producer p fills tile rows (8 p + i) * 8 .. + 8; lane l writes position l % 8 of row
-  // (8 p + i) * 8 + l / 8, i.e. global unit (l % 8) ^ (l / 8) (the row's swizzle key is l / 8)
+  // x: load i of producer p fills tile rows (XI p + i) * 8 .. + 8; lane l writes position l % 8 of row
+  // (XI p + i) * 8 + l / 8, i.e. global unit (l % 8) ^ (l / 8) (the row's swizzle key is l / 8)
   const int lrow = lane >> 3, lcol = ((lane & 7) ^ (lane >> 3)) * 8;
   const uint16_t* xr[kPcXI];
 #pragma unroll
-  for (int i = 0; i < kPcXI; ++i) xr[i] = a.x + (int64_t)min(m0 + (8 * p + i) * 8 + lrow, a.M - 1) * a.ldx + lcol;
+  for (int i = 0; i < kPcXI; ++i) xr[i] = a.x + (int64_t)min(m0 + (kPcXI * p + i) * 8 + lrow, a.M - 1) * a.ldx + lcol;
   // packed weights: lane l owns tile row 32 p + l / 2, columns 32 (l % 2) .. + 32 of each slice (16 bytes)
   const int wr = 32 * p + (lane >> 1), wh = lane & 1;
-  const int32_t* wq = a.qw + (int64_t)min(n0 + wr, a.N - 1) * a.ldq + 4 * wh;
-  // scales and zero words of the producer's 32 channels: lanes 0-15 read scale pairs, lanes 16-19 zero words, the
-  // rest repeat lane 0's pair (every lane of a direct-to-LDS load writes its 4 bytes)
+  const int32_t* wq = a.qw + (int64_t)min(n0 + wr, a.N - 1) * a.ldq;
+  // scales and zero words of the producer's 32 channels, of the group of the slice's first 32 columns in lanes 0-31 and
+  // of its second 32 in lanes 32-63 (the same group when the group size is a multiple of 64): lanes 0-15 of each half
+  // read scale pairs, lanes 16-19 zero words, the rest repeat lane 0's pair (every lane of a direct-to-LDS load writes
+  // its 4 bytes)
   const uint8_t* szb;
   int64_t szstride;  // bytes per group
   {
-    const int c0 = n0 + 32 * p;
-    if (lane >= 16 && lane < 20 && a.hasz) {
-      const int w = min(c0 / 8 + (lane - 16), (a.N - 1) / 8);
+    const int c0 = n0 + 32 * p, l32 = lane & 31;
+    if (l32 >= 16 && l32 < 20 && a.hasz) {
+      const int w = min(c0 / 8 + (l32 - 16), (a.N - 1) / 8);
       szb = reinterpret_cast<const uint8_t*>(a.zeros + w);
       szstride = a.ldz * 4;
     } else {
-      const int c = min(c0 + 2 * (lane < 16 ? lane : 0), a.N - 2);
+      const int c = min(c0 + 2 * (l32 < 16 ? l32 : 0), a.N - 2);
       szb = reinterpret_cast<const uint8_t*>(a.scales + c);
       szstride = a.lds * 2;
     }
   }
-  const int slice0 = kbeg / kPcBK;
-  auto group_of = [&](int t) -> uint32_t {  // group of local slice t (clamped to the last slice)
-    const uint32_t sl = (uint32_t)(slice0 + min(t, nk - 1));
-    return a.gdiv == 0 ? 0u : (a.gdiv == 1 ? sl : __umulhi(sl, a.gmul));
+  // chunks (32 columns) of a local slice's two halves (slices past the last read it again; past K, the last chunk), the
+  // same for the whole wavefront, and the lane's own
+  auto chunk0 = [&](int t) { return (kbeg + min(t, nk - 1) * kPcBK) / 32; };
+  auto chunk1 = [&](int t) { return TAIL ? min(chunk0(t) + 1, a.K / 32 - 1) : chunk0(t) + 1; };
+  auto group_of = [&](int c) -> uint32_t {
+    return a.gdiv == 0 ? 0u : (a.gdiv == 1 ? (uint32_t)c : __umulhi((uint32_t)c, a.gmul));
   };
   // x rows of slice t into a stage's x area
   auto issue_x = [&](int t, uint8_t* dst) __attribute__((always_inline)) {
     const int k0 = kbeg + min(t, nk - 1) * kPcBK;
     dst += p * kPcXI * 1024;
 #pragma unroll
-    for (int i = 0; i < kPcXI; ++i) __builtin_amdgcn_global_load_lds(xr[i] + k0, dst + i * 1024, 16, 0, 0);
+    for (int i = 0; i < kPcXI; ++i) {
+      const uint16_t* src = xr[i] + k0;
+      if (TAIL) src = k0 + lcol < a.K ? src : g_pc_zero;
+      __builtin_amdgcn_global_load_lds(src, dst + i * 1024, 16, 0, 0);
+    }
   };
   // packed weights, scales and zero words of slice t into a stage's staging areas (base: the stage's packed-weight
   // area, the scale area follows it)
   auto issue_q = [&](int t, uint8_t* dst) __attribute__((always_inline)) {
-    const int k0 = kbeg + min(t, nk - 1) * kPcBK;
-    __builtin_amdgcn_global_load_lds(wq + k0 / 8, dst + p * 1024, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds(szb + (int64_t)group_of(t) * szstride, dst + kPcQBytes + p * 256, 4, 0, 0);
+    const int c0 = chunk0(t), c1 = chunk1(t);
+    const uint32_t g0 = group_of(c0), g1 = group_of(c1);
+    __builtin_amdgcn_global_load_lds(wq + 4 * (wh ? c1 : c0), dst + p * 1024, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(szb + (int64_t)(lane < 32 ? g0 : g1) * szstride, dst + kPcQBytes + p * 256, 4, 0, 0);
   };
   uint32_t nmask = 0x0F0F0F0Fu;
   asm("" : "+v"(nmask));  // hidden from known-bits analysis: bytes of masked words convert with v_cvt_f32_ubyte{k}
@@ -264,7 +308,7 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
   // one slice's weights from a stage's staging areas (q) into its weight rows (w)
   auto dequant = [&](const uint8_t* __restrict__ q, uint8_t* __restrict__ w) __attribute__((always_inline)) {
     const uint4 qv = *reinterpret_cast<const uint4*>(q + p * 1024 + lane * 16);
-    const uint8_t* sz = q + kPcQBytes + p * 256;
+    const uint8_t* sz = q + kPcQBytes + p * 256 + wh * 128;
     const uint32_t sraw = *reinterpret_cast<const uint16_t*>(sz + (lane >> 1) * 2);
     const uint32_t zw = (*reinterpret_cast<const uint32_t*>(sz + 64 + ((lane >> 1) >> 3) * 4) & zsel) |
                         (0x88888888u & ~zsel);  // symmetric: zero-point 8
@@ -272,6 +316,26 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
     const float c = -(float)nibble(zw, (lane >> 1) & 7) * sc;
     const uint32_t wd[4] = {qv.x, qv.y, qv.z, qv.w};
     uint8_t* rp = w + wr * kPcRow;
+    if (!XBF16 && !a.sbf16) {
+      // fp16 x and scales: 1024 + q by bits, minus 1024 + z (exact), times s in packed fp16 -- the exact product rounded
+      // once, as the fp32 form rounds it -- in 17 instructions per 8 values instead of 23
+      const uint32_t zb = 0x6400u + nibble(zw, (lane >> 1) & 7);
+      const f16x2_pc_t z2 = __builtin_bit_cast(f16x2_pc_t, zb | zb << 16);
+      const f16x2_pc_t s2 = __builtin_bit_cast(f16x2_pc_t, sraw | sraw << 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t h = wd[i] >> 4;
+        uint32_t o[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {  // byte b: nibbles 2 b and 2 b + 1 into the two halves
+          const uint32_t t = __builtin_amdgcn_perm(h, wd[i], 0x0c040c00u + 0x00010001u * b);
+          const f16x2_pc_t m = __builtin_bit_cast(f16x2_pc_t, (t & 0x000F000Fu) | 0x64006400u);
+          o[b] = __builtin_bit_cast(uint32_t, (m - z2) * s2);
+        }
+        *reinterpret_cast<uint4*>(rp + (((4 * wh + i) ^ (wr & 7)) * 16)) = make_uint4(o[0], o[1], o[2], o[3]);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // word i = columns 8 i .. 8 i + 7 of the lane's 32 = unit 4 wh + i of the row
       const uint32_t lo = wd[i] & nmask, hi = (wd[i] >> 4) & nmask;  // nibbles 0,2,4,6 / 1,3,5,7
@@ -324,34 +388,51 @@ __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // drain before the consumers reuse the ring
 }
 
-bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
-              int sdt, int64_t lds, int64_t N, int64_t K, int gs, int64_t G) {
-  return perm == nullptr && (K % kPcBK) == 0 && ((gs % kPcBK) == 0 || G == 1) && (N % 8) == 0 && N >= 8 &&
-         sdt != FG_F32 && (lds % 2) == 0 && (reinterpret_cast<uintptr_t>(scales) % 4) == 0 && (ldx % 8) == 0 &&
-         (reinterpret_cast<uintptr_t>(x) % 16) == 0 && (ldq % 4) == 0 && (reinterpret_cast<uintptr_t>(qw) % 16) == 0 &&
-         group_div_exact(K, gs, G, kPcBK);
+template <int BM, bool XBF16, bool TAIL>
+__global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) w4_pc_kernel(const PcArgs a) {
+  w4_pc_body<BM, XBF16, TAIL>(a);
 }
 
-// K splits: one when the tiles cover the CUs, else as many as keep the workgroups within one round over the CUs, each
-// at least 512 columns.
-void w4_pc_plan(int M, int N, int K, int split_k, int* splits, int* kchunk) {
-  const int cus = device_cus();
-  const int64_t tiles = (int64_t)((M + kPcBM - 1) / kPcBM) * ((N + kPcBN - 1) / kPcBN);
-  int s = split_k;
-  if (s <= 0) {
-    s = tiles >= cus ? 1 : (int)(cus / tiles);
-    const int max_s = K / 512 > 0 ? K / 512 : 1;
-    s = std::min(std::min(s, max_s), 16);
+bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
+              int sdt, int64_t lds, int64_t N, int64_t K, int gs, int64_t G) {
+  return perm == nullptr && (K % 32) == 0 && ((gs % 32) == 0 || G == 1) && (N % 8) == 0 && N >= 8 &&
+         sdt != FG_F32 && (lds % 2) == 0 && (reinterpret_cast<uintptr_t>(scales) % 4) == 0 && (ldx % 8) == 0 &&
+         (reinterpret_cast<uintptr_t>(x) % 16) == 0 && (ldq % 4) == 0 && (reinterpret_cast<uintptr_t>(qw) % 16) == 0 &&
+         group_div_exact(K, gs, G, 32);
+}
+
+// Row tile (64, 128 or 256) and K splits: the cheapest by a cost in ns fitted to graph replays over five shapes (N =
+// 2048..28672, K = 2048..14336, 5..1500 rows): a launch takes the slices of its workgroups times the tile's time per
+// slice, plus 4.6 us, for every round of workgroups over the CUs; a split launch 2.7 us and 0.42 us per MB of partials
+// more.  The choice lies within 0.5% (geometric mean) of the best of tile and split measured.  The time per slice hardly
+// falls below 128 rows: a producer's chain of staging read, dequantisation and stores is what a slice takes there.
+// Rows of 64 / 128 / 256 measured (us, fp16 x, groups of 64): K=4096, N=28672 M=64 46 / 52 / -, M=128 89 / 53 / 69,
+// M=200 175 / 99 / 71; K=N=2048 M=300 17.8 / 19.2 / 22.7.  The all-rounder, which took these before: M=64 54, M=128 62,
+// M=200 89, and 22.5.
+void w4_pc_plan(int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk) {
+  static const struct { int bm, ns; } kTile[] = {{64, 614}, {128, 726}, {256, 880}};
+  const int64_t cus = device_cus(), slices = (K + kPcBK - 1) / kPcBK;
+  int64_t best = -1;
+  for (const auto& t : kTile) {
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + kPcBN - 1) / kPcBN);
+    const int64_t most = split_k > 0 ? split_k : std::max<int64_t>(1, std::min<int64_t>({16, K / 256, cus / tiles}));
+    for (int64_t s = split_k > 0 ? split_k : 1; s <= most; ++s) {
+      const int64_t per = (slices + s - 1) / s, used = (slices + per - 1) / per;
+      const int64_t rounds = (tiles * used + cus - 1) / cus;
+      const int64_t cost = rounds * (per * t.ns + 4600) + (used > 1 ? 2700 + used * M * (int64_t)N / 600 : 0);
+      if (best < 0 || cost < best) {
+        best = cost;
+        *bm = t.bm;
+        *splits = (int)used;
+        *kchunk = (int)per * kPcBK;
+      }
+    }
   }
-  int kc = (K + s - 1) / s;
-  kc = (kc + kPcBK - 1) / kPcBK * kPcBK;
-  *kchunk = kc;
-  *splits = (K + kc - 1) / kc;
 }
 
 size_t w4_pc_workspace_bytes(int M, int N, int K, int split_k) {
-  int s, kc;
-  w4_pc_plan(M, N, K, split_k, &s, &kc);
+  int bm, s, kc;
+  w4_pc_plan(M, N, K, split_k, &bm, &s, &kc);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -363,8 +444,8 @@ hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* q
                         int sdt, int64_t lds, const int32_t* zeros, int64_t ldz, const void* bias, int bdt, void* y,
                         int64_t ldy, float* ws, int M, int N, int K, int gs, bool single_group, int split_k,
                         hipStream_t s) {
-  int splits, kchunk;
-  w4_pc_plan(M, N, K, split_k, &splits, &kchunk);
+  int bm, splits, kchunk;
+  w4_pc_plan(M, N, K, split_k, &bm, &splits, &kchunk);
   PcArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.ldx = ldx;
@@ -384,19 +465,26 @@ hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* q
   a.N = N;
   a.K = K;
   a.kchunk = kchunk;
-  a.gdiv = single_group ? 0u : (uint32_t)(gs / kPcBK);
+  a.gdiv = single_group ? 0u : (uint32_t)(gs / 32);
   a.gmul = a.gdiv > 1 ? 0xffffffffu / a.gdiv + 1u : 0u;
   a.sbf16 = sdt == FG_BF16;
   if (splits > 1 && ws == nullptr) return hipErrorInvalidValue;
-  auto kern = xbf16 ? w4_pc_kernel<true> : w4_pc_kernel<false>;
-  hipError_t e =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kPcLds);
-  if (e != hipSuccess) return e;
-  const int tiles = ((M + kPcBM - 1) / kPcBM) * ((N + kPcBN - 1) / kPcBN);
-  note_kernel("w4_pc_kernel<%s> 256x128 splits=%d%s", xbf16 ? "bf16" : "f16", splits,
-              splits > 1 ? " + w4_splitk_reduce_kernel" : "");
-  hipLaunchKernelGGL(kern, dim3(tiles, splits), dim3(kPcThreads), kPcLds, s, a);
-  e = hipGetLastError();
+  auto go = [&](auto bm_tag) -> hipError_t {
+    constexpr int BM = decltype(bm_tag)::value;
+    auto kern = K % kPcBK ? (xbf16 ? w4_pc_kernel<BM, true, true> : w4_pc_kernel<BM, false, true>)
+                          : (xbf16 ? w4_pc_kernel<BM, true, false> : w4_pc_kernel<BM, false, false>);
+    const hipError_t err =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, pc_lds(BM));
+    if (err != hipSuccess) return err;
+    const int tiles = ((M + BM - 1) / BM) * ((N + kPcBN - 1) / kPcBN);
+    note_kernel("w4_pc_kernel<%s> %dx128 splits=%d%s", xbf16 ? "bf16" : "f16", BM, splits,
+                splits > 1 ? " + w4_splitk_reduce_kernel" : "");
+    hipLaunchKernelGGL(kern, dim3(tiles, splits), dim3(kPcThreads), pc_lds(BM), s, a);
+    return hipGetLastError();
+  };
+  hipError_t e = bm == 64    ? go(std::integral_constant<int, 64>{})
+                 : bm == 128 ? go(std::integral_constant<int, 128>{})
+                             : go(std::integral_constant<int, 256>{});
   if (e != hipSuccess || splits == 1) return e;
   return xbf16 ? launch_w4_splitk_reduce<true>(ws, splits, M, N, bias, bdt, y, ldy, s)
                : launch_w4_splitk_reduce<false>(ws, splits, M, N, bias, bdt, y, ldy, s);

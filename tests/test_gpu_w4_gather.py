@@ -26,10 +26,10 @@ def test_gather_moves_every_element(m, k, pad):
     assert torch.equal(out.view(torch.int16), x[:, perm.long()].view(torch.int16)) and out.stride(0) % 8 == 0
 
 
-# the GEMV on blocked scales, the CDNA4 copies, the prefill kernels, and (K % 64 != 0) the tiled kernel
+# the GEMV on blocked scales, the CDNA4 copies, the prefill kernels, and (groups of 16) the tiled kernel
 @pytest.mark.parametrize("m,n,k,gs,kernel", [(1, 1024, 2048, 128, "w4_gemv_split"), (16, 1024, 2048, 128, "w4_frag"),
-                                             (100, 1024, 2048, 64, "w4_big"), (300, 1032, 2048, 128, "w4_pc"),
-                                             (9, 520, 1056, 32, "w4_mfma")])
+                                             (100, 1024, 2048, 64, "w4_pc"), (300, 1030, 2048, 128, "w4_big"),
+                                             (9, 520, 1056, 16, "w4_mfma")])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
 def test_act_order_module_reaches_the_policy_kernels(m, n, k, gs, kernel, xdt):
     q, s, z = w4_parts(n, k, gs, False, seed=m)

@@ -1,0 +1,66 @@
+"""The producer / consumer kernel's row tiles, groups and K tails, reached through the policy: 64-, 128- and 256-row tiles
+with and without K splits, groups of 32 / 64 / 96 / one, K that ends inside a 64-column slice, fp16 and bf16 x with scales
+of either type (packed fp16 dequantisation and the fp32 one), against the CPU oracle."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from forge_amd import layouts as L
+from forge_amd import ops_gemm as ops
+from oracle import gemm as og
+from tests._util import assert_close, gen, oracle_packed, to_f32, w4_parts, x_act
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF, HF = torch.bfloat16, torch.float16
+CASES = [  # m, n, k, group, sym, x, scales, bias, tile rows
+    (5, 136, 512, 64, False, HF, HF, None, 64),
+    (17, 1032, 1056, 32, True, BF, HF, BF, 64),       # K % 64 == 32
+    (64, 2048, 96, 96, False, HF, BF, HF, 64),        # one group, one slice and a half
+    (65, 1024, 2048, 64, False, HF, HF, HF, 64),
+    (128, 6144, 4096, 64, True, HF, HF, HF, 128),     # splits
+    (127, 16392, 1056, 32, False, BF, BF, None, 128),
+    (200, 6144, 2048, 32, False, BF, HF, None, 256),
+    (129, 6144, 4128, 96, True, HF, HF, BF, 256),
+    (256, 20488, 544, -1, False, HF, HF, None, 256),
+    (33, 20488, 160, 32, False, HF, HF, None, 64),    # tiles cover the CUs: no split
+]
+
+
+@pytest.mark.parametrize("m,n,k,gs,sym,xdt,sdt,bdt,bm", CASES)
+def test_tiles_groups_and_tails(m, n, k, gs, sym, xdt, sdt, bdt, bm):
+    q, s, z = w4_parts(n, k, gs, sym, seed=m + k, scale_dtype=sdt)
+    p = L.pack_w4(q, s, z, gs).to(DEV)
+    x = x_act(m, k, xdt, seed=m)
+    b = None if bdt is None else torch.randn(n, generator=gen(3)).to(bdt)
+    y = ops.w4a16_linear(x.to(DEV), p, None if b is None else b.to(DEV))
+    kern = ops.last_kernel()
+    assert kern.startswith("w4_pc_kernel") and f" {bm}x128" in kern, kern
+    ref = og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, gs), None if b is None else to_f32(b))
+    assert_close(y.cpu(), ref, "bfloat16" if xdt == BF else "float16", what=kern)
+    assert torch.equal(y, ops.w4a16_linear(x.to(DEV), p, None if b is None else b.to(DEV)))
+
+
+def test_packed_fp16_dequantisation_equals_the_fp32_form():
+    """Every code, zero-point and a spread of fp16 scales (subnormal products among them): x picks single weights, so
+    the outputs are the dequantised weights themselves, equal to ((q - z) * s) rounded once to fp16."""
+    n, k = 256, 64
+    q = torch.arange(16, dtype=torch.uint8).repeat(n, k // 16)
+    z = (torch.arange(n) % 16).to(torch.uint8).view(n, 1)
+    s = torch.exp2(torch.linspace(-24, 10, n)).mul(1 + torch.rand(n, generator=gen(1))).half().view(n, 1)
+    p = L.pack_w4(q, s, z, k).to(DEV)
+    y = ops.w4a16_linear(torch.eye(k).half().to(DEV), p)
+    assert ops.last_kernel().startswith("w4_pc_kernel") or ops.last_kernel().startswith("w4_skinny"), ops.last_kernel()
+    y = ops.w4a16_linear(torch.eye(k).half().to(DEV), p, config={"impl": "prefill", "tile_n": 128})
+    assert ops.last_kernel().startswith("w4_pc_kernel"), ops.last_kernel()
+    want = ((q.float() - z.float()) * s.float()).half()
+    assert torch.equal(y.cpu(), want.t())
+
+
+def test_forced_prefill_still_refuses_what_it_refused():
+    q, s, z = w4_parts(128, 96, 32, False)
+    p = L.pack_w4(q, s, z, 32).to(DEV)
+    from forge_amd import _lib
+    with pytest.raises(_lib.KernelLaunchError, match="K%64"):
+        ops.w4a16_linear(x_act(70, 96).to(DEV), p, config={"impl": "prefill"})
