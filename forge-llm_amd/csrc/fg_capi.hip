@@ -35,7 +35,12 @@ bool w4_big_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const
 size_t w4_big_workspace_bytes(int M, int N, int K, int split_k, bool w8);
 bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
               int sdt, int64_t lds, int64_t N, int64_t K, int gs, int64_t G);
-size_t w4_pc_workspace_bytes(int M, int N, int K, int split_k);
+size_t w4_pc_workspace_bytes(bool w8, int M, int N, int K, int split_k);
+bool w8_pc_ok(const void* x, int64_t ldx, const int8_t* qw, int64_t ldq, const void* scales, int sdt, int64_t lds,
+              int64_t N, int64_t K, int gs, int64_t G);
+hipError_t launch_w8_pc(const void* x, int64_t ldx, bool xbf16, const int8_t* qw, int64_t ldq, const void* scales,
+                        int sdt, int64_t lds, const void* bias, int bdt, void* y, int64_t ldy, float* ws, int M, int N,
+                        int K, int gs, bool single_group, int split_k, hipStream_t s);
 bool w4_pp_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
               int sdt, int64_t lds, const int32_t* zeros, int64_t ldz, int64_t M, int64_t N, int64_t K, int gs,
               int64_t G);
@@ -352,7 +357,7 @@ size_t prefill_workspace_bytes(int tile_n, int64_t M, int64_t N, int64_t K, int 
   if (pp) b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k));
   if (!w4 && tile_n == 0 && w8_pp_split(M, N) > 1)
     b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k > 0 ? split_k : w8_pp_split(M, N)));
-  if (pc) b = std::max(b, fg::w4_pc_workspace_bytes((int)M, (int)N, (int)K, split_k));
+  if (pc) b = std::max(b, fg::w4_pc_workspace_bytes(false, (int)M, (int)N, (int)K, split_k));
   return b;
 }
 
@@ -744,17 +749,32 @@ static bool w8a16_ring_rows(int64_t M, int64_t N, int64_t K) {
   return M > 16 ? M <= 64 : (M > 2 && (N >= 16384 || K >= 8192));
 }
 
+// Whether a W8A16 call that neither the GEMV, the ring nor the skinny kernel takes goes to the producer / consumer kernel
+// (64- and 128-row tiles) where its operands allow: whenever K ends inside a 64-column slice (the other kernels cannot
+// read it and the generic one would serve: K=4128, N=4096, groups of 32, 6 / 64 / 512 rows 101 / 665 / 4439 us against
+// 15 / 20 / 41), for 65..128 rows, and up to 256 while its 128-row tiles fit one round (all-rounder / producer-consumer,
+// us: K=4096, N=6144 M=80 30.5 / 21.3, M=256 40.4 / 36.2; N=28672 M=128 71.9 / 56.9, M=200 -- two rounds -- 100.5 /
+// 107.8; K=14336, N=4096 M=128 46.3 / 34.6, M=256 62.5 / 55.9; from 384 rows the ping-pong kernel is ahead).  Up to 64 rows (groups that are no multiple of 128) it would
+// be ahead of the all-rounder too (K=N=4096, groups of 64, 64 rows 18.7 against 25.4), but tests/test_gpu_policy_paths.py
+// states that the policy there runs what a forced prefill runs.
+static bool w8_pc_rows(int64_t M, int64_t N, int64_t K) {
+  return K % 64 != 0 || (M > 64 && M <= 128) || (M > 64 && M <= 256 && ((M + 127) / 128) * ((N + 127) / 128) <= fg::device_cus());
+}
+
 size_t fg_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size, const fg_w4_config* cfg) {
   if (M <= 0 || N <= 0 || K <= 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim) return 0;
   const int gs = group_size > 0 ? group_size : (int)K;
   const int64_t G = (K + gs - 1) / gs;
   const int impl = cfg ? cfg->impl : FG_W4_AUTO;
   // the prefill kernels' split-K partials, whenever one may run (their alignment conditions are checked at launch)
+  // the producer / consumer kernel, which also takes K % 64 == 32
+  const bool pc_shape = impl == FG_W4_AUTO && (K % 32 == 0) && (gs % 32 == 0 || G == 1) && w8_pc_rows(M, N, K);
+  const size_t pc = pc_shape ? fg::w4_pc_workspace_bytes(true, (int)M, (int)N, (int)K, 0) : 0;
   const bool prefill_shape = (K % 64 == 0) && (gs % 32 == 0 || G == 1);
-  if (!prefill_shape || impl == FG_W4_GENERIC || impl == FG_W4_MFMA || impl == FG_W4_GEMV) return 0;
+  if (!prefill_shape || impl == FG_W4_GENERIC || impl == FG_W4_MFMA || impl == FG_W4_GEMV) return pc;
   const size_t ring = impl == FG_W4_AUTO && w8a16_ring_rows(M, N, K) ? fg::w8a16_ring_workspace_bytes((int)M, (int)N, (int)K)
                                                                : 0;
-  return std::max(ring, prefill_workspace_bytes(cfg ? cfg->tile_n : 0, M, N, K, cfg ? cfg->split_k : 0, false));
+  return std::max({pc, ring, prefill_workspace_bytes(cfg ? cfg->tile_n : 0, M, N, K, cfg ? cfg->split_k : 0, false)});
 }
 
 int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight, int64_t ldq, const void* scales,
@@ -793,8 +813,15 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
   // qkv level, gate+up 33.2 against 27.1 on the ring); then the LDS ring (w8a16_ring_rows), else the skinny kernel up
   // to 64 rows
   const bool gemv_rows = M <= 2 || (M <= 4 && N <= 8192 && K < 8192);
+  const bool pc = w8_pc_rows(M, N, K) && fg::w8_pc_ok(x, ldx, qweight, ldq, scales, scale_dtype, lds, N, K, gs, G) &&
+                  !(cfg && (cfg->tile_m || cfg->tile_n || cfg->split_k));
   if (kern < 0)
-    kern = (gemv && gemv_rows) ? 3 : ((ring && w8a16_ring_rows(M, N, K)) ? 4 : ((skinny && M <= 64) ? 1 : (big ? 2 : 0)));
+    kern = (gemv && gemv_rows)                    ? 3
+           : (ring && w8a16_ring_rows(M, N, K))   ? 4
+           : (skinny && M <= 64)                  ? 1
+           : pc                                   ? 5
+           : big                                  ? 2
+                                                  : 0;
   if (kern == 3 && !gemv)
     return fail(FG_EUNSUPPORTED, "fg_w8a16_gemm: decode GEMV needs M<=4, K%%16==0, group%%16==0 (or one group), "
                                  "16-bit scales with lds%%8==0, ldq%%16==0, ldx%%8==0, 16-byte aligned x/qweight/"
@@ -819,6 +846,13 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
   } else if (kern == 1) {
     e = fg::launch_w8a16_skinny(x, ldx, xbf16, qweight, ldq, scales, scale_dtype, lds, bias, bias_dtype, y, ldy,
                                 (int)M, (int)N, (int)K, gs, G == 1, s);
+  } else if (kern == 5) {
+    const size_t need = fg::w4_pc_workspace_bytes(true, (int)M, (int)N, (int)K, 0);
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+      return fail(FG_EINVAL, "fg_w8a16_gemm: workspace of %zu bytes needed, %zu given", need,
+                  workspace ? workspace_bytes : (size_t)0);
+    e = fg::launch_w8_pc(x, ldx, xbf16, qweight, ldq, scales, scale_dtype, lds, bias, bias_dtype, y, ldy,
+                         static_cast<float*>(workspace), (int)M, (int)N, (int)K, gs, G == 1, 0, s);
   } else if (kern == 2) {
     // the ping-pong kernel or the all-rounder, by the W4A16 rule; where W4A16 would take the producer / consumer
     // kernel (none for int8 weights), the ping-pong kernel with its K split as w8_pp_split says

@@ -1,4 +1,5 @@
-// W4A16 prefill with producer and consumer wavefronts: y[M,N] = x[M,K] @ dequant(W)[N,K]^T (+bias).
+// W4A16 prefill with producer and consumer wavefronts: y[M,N] = x[M,K] @ dequant(W)[N,K]^T (+bias).  W8A16 (int8
+// weights) takes the same kernel with tiles of 64 and 128 rows: twice the staging bytes, no zero words.
 //
 // A workgroup owns a BM x 128 output tile (BM = 256, 128 or 64; below 256 rows) and walks K in 64-column slices through
 // a three-stage LDS ring.  Its eight wavefronts split the work by role, one of each role per SIMD (wavefronts 0-3 on SIMDs 0-3, 4-7 likewise):
@@ -52,15 +53,16 @@ typedef _Float16 f16x2_pc_t __attribute__((ext_vector_type(2)));
 
 constexpr int kPcBN = 128, kPcBK = 64, kPcRow = 128, kPcThreads = 512;
 constexpr int kPcWBytes = kPcBN * kPcRow;                      // dequantised weight rows
-constexpr int kPcQBytes = kPcBN * kPcBK / 2;                   // packed weights of the slice
+constexpr int pc_q_bytes(int wb) { return kPcBN * kPcBK * wb / 8; }  // packed weights of the slice (WB bits each)
 constexpr int kPcSBytes = 4 * 256;                             // scales and zero words
 constexpr int pc_x_bytes(int bm) { return bm * kPcRow; }       // x rows
-constexpr int pc_stage(int bm) { return pc_x_bytes(bm) + kPcWBytes + kPcQBytes + kPcSBytes; }
-constexpr int pc_lds(int bm) { return 3 * pc_stage(bm); }
-static_assert(pc_lds(256) <= 160 * 1024, "the ring exceeds the LDS");
+constexpr int pc_stage(int bm, int wb) { return pc_x_bytes(bm) + kPcWBytes + pc_q_bytes(wb) + kPcSBytes; }
+constexpr int pc_lds(int bm, int wb) { return 3 * pc_stage(bm, wb); }
+static_assert(pc_lds(256, 4) <= 160 * 1024 && pc_lds(128, 8) <= 160 * 1024, "the ring exceeds the LDS");
 // direct-to-LDS loads one producer issues per slice: x rows, packed weights, scales + zero words
 constexpr int pc_xi(int bm) { return pc_x_bytes(bm) / 1024 / 4; }
-constexpr int kPcQI = 1, kPcSI = 1;
+constexpr int pc_qi(int wb) { return pc_q_bytes(wb) / 1024 / 4; }
+constexpr int kPcSI = 1;
 static_assert(pc_xi(256) == 8, "eight x loads per producer and slice");
 
 // What a TAIL launch reads in place of the 16-byte x units past K: zeros, so the weights they meet do not matter.
@@ -69,8 +71,8 @@ static __device__ __align__(16) const uint16_t g_pc_zero[8] = {};
 struct PcArgs {
   const uint16_t* x;
   int64_t ldx;
-  const int32_t* qw;
-  int64_t ldq;  // int32 words per row
+  const void* qw;
+  int64_t ldq;  // 4-bit weights: int32 words per row; 8-bit: bytes
   const uint16_t* scales;
   int64_t lds;
   const int32_t* zeros;  // qweight when symmetric (a valid address, never used)
@@ -113,9 +115,10 @@ __device__ __forceinline__ uint4 pc_frag(const uint8_t* rp, int r16, int lane, i
   return *reinterpret_cast<const uint4*>(rp + c * 16);
 }
 
-template <int BM, bool XBF16, bool TAIL>
+template <int BM, bool XBF16, int WB, bool TAIL>
 __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
-  constexpr int kPcBM = BM, kPcXBytes = pc_x_bytes(BM), kPcStage = pc_stage(BM), kPcXI = pc_xi(BM);
+  constexpr int kPcBM = BM, kPcXBytes = pc_x_bytes(BM), kPcStage = pc_stage(BM, WB), kPcXI = pc_xi(BM);
+  constexpr int kPcQI = pc_qi(WB), kPcQBytes = pc_q_bytes(WB);
   constexpr int TM = BM / 32;  // 16-row blocks of a consumer
   extern __shared__ __align__(16) uint8_t smem[];
   const int ntm = (a.M + kPcBM - 1) / kPcBM, ntn = (a.N + kPcBN - 1) / kPcBN;
@@ -255,9 +258,9 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   const uint16_t* xr[kPcXI];
 #pragma unroll
   for (int i = 0; i < kPcXI; ++i) xr[i] = a.x + (int64_t)min(m0 + (kPcXI * p + i) * 8 + lrow, a.M - 1) * a.ldx + lcol;
-  // packed weights: lane l owns tile row 32 p + l / 2, columns 32 (l % 2) .. + 32 of each slice (16 bytes)
+  // packed weights: lane l owns tile row 32 p + l / 2, columns 32 (l % 2) .. + 32 of each slice (16 or 32 bytes)
   const int wr = 32 * p + (lane >> 1), wh = lane & 1;
-  const int32_t* wq = a.qw + (int64_t)min(n0 + wr, a.N - 1) * a.ldq;
+  const uint8_t* wq = static_cast<const uint8_t*>(a.qw) + (int64_t)min(n0 + wr, a.N - 1) * a.ldq * (WB == 4 ? 4 : 1);
   // scales and zero words of the producer's 32 channels, of the group of the slice's first 32 columns in lanes 0-31 and
   // of its second 32 in lanes 32-63 (the same group when the group size is a multiple of 64): lanes 0-15 of each half
   // read scale pairs, lanes 16-19 zero words, the rest repeat lane 0's pair (every lane of a direct-to-LDS load writes
@@ -299,7 +302,9 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   auto issue_q = [&](int t, uint8_t* dst) __attribute__((always_inline)) {
     const int c0 = chunk0(t), c1 = chunk1(t);
     const uint32_t g0 = group_of(c0), g1 = group_of(c1);
-    __builtin_amdgcn_global_load_lds(wq + 4 * (wh ? c1 : c0), dst + p * 1024, 16, 0, 0);
+#pragma unroll
+    for (int h = 0; h < kPcQI; ++h)
+      __builtin_amdgcn_global_load_lds(wq + (wh ? c1 : c0) * (4 * WB) + 16 * h, dst + (p * kPcQI + h) * 1024, 16, 0, 0);
     __builtin_amdgcn_global_load_lds(szb + (int64_t)(lane < 32 ? g0 : g1) * szstride, dst + kPcQBytes + p * 256, 4, 0, 0);
   };
   uint32_t nmask = 0x0F0F0F0Fu;
@@ -307,12 +312,29 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   const uint32_t zsel = a.hasz ? 0xffffffffu : 0u;
   // one slice's weights from a stage's staging areas (q) into its weight rows (w)
   auto dequant = [&](const uint8_t* __restrict__ q, uint8_t* __restrict__ w) __attribute__((always_inline)) {
-    const uint4 qv = *reinterpret_cast<const uint4*>(q + p * 1024 + lane * 16);
+    const uint4 qv = *reinterpret_cast<const uint4*>(q + p * kPcQI * 1024 + lane * 16);
     const uint8_t* sz = q + kPcQBytes + p * 256 + wh * 128;
     const uint32_t sraw = *reinterpret_cast<const uint16_t*>(sz + (lane >> 1) * 2);
     const uint32_t zw = (*reinterpret_cast<const uint32_t*>(sz + 64 + ((lane >> 1) >> 3) * 4) & zsel) |
                         (0x88888888u & ~zsel);  // symmetric: zero-point 8
     const float sc = a.sbf16 ? bf16_bits_to_f32(sraw) : f16_bits_to_f32((uint16_t)sraw);
+    if constexpr (WB == 8) {  // u = q ^ 0x80 = q + 128: q * s = u * s - 128 s, exact in fp32, rounded once
+      const uint4 qv2 = *reinterpret_cast<const uint4*>(q + (p * kPcQI + 1) * 1024 + lane * 16);
+      const uint32_t wd[8] = {qv.x, qv.y, qv.z, qv.w, qv2.x, qv2.y, qv2.z, qv2.w};
+      const float c128 = -128.f * sc;
+      uint8_t* row = w + wr * kPcRow;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float d[8];
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+          d[b] = __builtin_fmaf((float)(((wd[2 * i + b / 4] ^ 0x80808080u) >> (8 * (b % 4))) & 0xFFu), sc, c128);
+        *reinterpret_cast<uint4*>(row + (((4 * wh + i) ^ (wr & 7)) * 16)) =
+            make_uint4(pc_pack<XBF16>(d[0], d[1]), pc_pack<XBF16>(d[2], d[3]), pc_pack<XBF16>(d[4], d[5]),
+                       pc_pack<XBF16>(d[6], d[7]));
+      }
+      return;
+    }
     const float c = -(float)nibble(zw, (lane >> 1) & 7) * sc;
     const uint32_t wd[4] = {qv.x, qv.y, qv.z, qv.w};
     uint8_t* rp = w + wr * kPcRow;
@@ -388,9 +410,18 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // drain before the consumers reuse the ring
 }
 
-template <int BM, bool XBF16, bool TAIL>
+template <int BM, bool XBF16, int WB, bool TAIL>
 __global__ void __launch_bounds__(kPcThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) w4_pc_kernel(const PcArgs a) {
-  w4_pc_body<BM, XBF16, TAIL>(a);
+  w4_pc_body<BM, XBF16, WB, TAIL>(a);
+}
+
+// W8A16 (int8 weights, ldq in bytes): as w4_pc_ok without zero words.
+bool w8_pc_ok(const void* x, int64_t ldx, const int8_t* qw, int64_t ldq, const void* scales, int sdt, int64_t lds,
+              int64_t N, int64_t K, int gs, int64_t G) {
+  return (K % 32) == 0 && ((gs % 32) == 0 || G == 1) && (N % 2) == 0 && sdt != FG_F32 && (lds % 2) == 0 &&
+         (reinterpret_cast<uintptr_t>(scales) % 4) == 0 && (ldx % 8) == 0 &&
+         (reinterpret_cast<uintptr_t>(x) % 16) == 0 && (ldq % 16) == 0 && (reinterpret_cast<uintptr_t>(qw) % 16) == 0 &&
+         group_div_exact(K, gs, G, 32);
 }
 
 bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
@@ -409,11 +440,12 @@ bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const 
 // Rows of 64 / 128 / 256 measured (us, fp16 x, groups of 64): K=4096, N=28672 M=64 46 / 52 / -, M=128 89 / 53 / 69,
 // M=200 175 / 99 / 71; K=N=2048 M=300 17.8 / 19.2 / 22.7.  The all-rounder, which took these before: M=64 54, M=128 62,
 // M=200 89, and 22.5.
-void w4_pc_plan(int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk) {
+void w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk) {
   static const struct { int bm, ns; } kTile[] = {{64, 614}, {128, 726}, {256, 880}};
   const int64_t cus = device_cus(), slices = (K + kPcBK - 1) / kPcBK;
   int64_t best = -1;
   for (const auto& t : kTile) {
+    if (w8 && t.bm == 256) continue;  // three stages with 8-bit staging exceed the LDS
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + kPcBN - 1) / kPcBN);
     const int64_t most = split_k > 0 ? split_k : std::max<int64_t>(1, std::min<int64_t>({16, K / 256, cus / tiles}));
     for (int64_t s = split_k > 0 ? split_k : 1; s <= most; ++s) {
@@ -430,9 +462,9 @@ void w4_pc_plan(int M, int N, int K, int split_k, int* bm, int* splits, int* kch
   }
 }
 
-size_t w4_pc_workspace_bytes(int M, int N, int K, int split_k) {
+size_t w4_pc_workspace_bytes(bool w8, int M, int N, int K, int split_k) {
   int bm, s, kc;
-  w4_pc_plan(M, N, K, split_k, &bm, &s, &kc);
+  w4_pc_plan(w8, M, N, K, split_k, &bm, &s, &kc);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -440,12 +472,13 @@ template <bool XBF16>
 hipError_t launch_w4_splitk_reduce(const float* ws, int S, int M, int N, const void* bias, int bdt, void* y,
                                    int64_t ldy, hipStream_t s);
 
-hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* qw, int64_t ldq, const void* scales,
-                        int sdt, int64_t lds, const int32_t* zeros, int64_t ldz, const void* bias, int bdt, void* y,
-                        int64_t ldy, float* ws, int M, int N, int K, int gs, bool single_group, int split_k,
-                        hipStream_t s) {
+template <int WB>
+static hipError_t launch_pc(const void* x, int64_t ldx, bool xbf16, const void* qw, int64_t ldq, const void* scales,
+                            int sdt, int64_t lds, const int32_t* zeros, int64_t ldz, const void* bias, int bdt, void* y,
+                            int64_t ldy, float* ws, int M, int N, int K, int gs, bool single_group, int split_k,
+                            hipStream_t s) {
   int bm, splits, kchunk;
-  w4_pc_plan(M, N, K, split_k, &bm, &splits, &kchunk);
+  w4_pc_plan(WB == 8, M, N, K, split_k, &bm, &splits, &kchunk);
   PcArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.ldx = ldx;
@@ -454,7 +487,7 @@ hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* q
   a.scales = static_cast<const uint16_t*>(scales);
   a.lds = lds;
   a.hasz = zeros != nullptr;
-  a.zeros = zeros ? zeros : qw;
+  a.zeros = zeros ? zeros : static_cast<const int32_t*>(qw);
   a.ldz = zeros ? ldz : 0;
   a.bias = bias;
   a.bdt = bdt;
@@ -471,23 +504,40 @@ hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* q
   if (splits > 1 && ws == nullptr) return hipErrorInvalidValue;
   auto go = [&](auto bm_tag) -> hipError_t {
     constexpr int BM = decltype(bm_tag)::value;
-    auto kern = K % kPcBK ? (xbf16 ? w4_pc_kernel<BM, true, true> : w4_pc_kernel<BM, false, true>)
-                          : (xbf16 ? w4_pc_kernel<BM, true, false> : w4_pc_kernel<BM, false, false>);
+    auto kern = K % kPcBK ? (xbf16 ? w4_pc_kernel<BM, true, WB, true> : w4_pc_kernel<BM, false, WB, true>)
+                          : (xbf16 ? w4_pc_kernel<BM, true, WB, false> : w4_pc_kernel<BM, false, WB, false>);
+    constexpr int lds_bytes = pc_lds(BM, WB);
     const hipError_t err =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, pc_lds(BM));
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (err != hipSuccess) return err;
     const int tiles = ((M + BM - 1) / BM) * ((N + kPcBN - 1) / kPcBN);
-    note_kernel("w4_pc_kernel<%s> %dx128 splits=%d%s", xbf16 ? "bf16" : "f16", BM, splits,
+    note_kernel("w4_pc_kernel<%s%s> %dx128 splits=%d%s", xbf16 ? "bf16" : "f16", WB == 8 ? ",w8" : "", BM, splits,
                 splits > 1 ? " + w4_splitk_reduce_kernel" : "");
-    hipLaunchKernelGGL(kern, dim3(tiles, splits), dim3(kPcThreads), pc_lds(BM), s, a);
+    hipLaunchKernelGGL(kern, dim3(tiles, splits), dim3(kPcThreads), lds_bytes, s, a);
     return hipGetLastError();
   };
-  hipError_t e = bm == 64    ? go(std::integral_constant<int, 64>{})
-                 : bm == 128 ? go(std::integral_constant<int, 128>{})
-                             : go(std::integral_constant<int, 256>{});
+  hipError_t e;
+  if (bm == 64) e = go(std::integral_constant<int, 64>{});
+  else if (WB == 8 || bm == 128) e = go(std::integral_constant<int, 128>{});
+  else e = go(std::integral_constant<int, WB == 8 ? 128 : 256>{});
   if (e != hipSuccess || splits == 1) return e;
   return xbf16 ? launch_w4_splitk_reduce<true>(ws, splits, M, N, bias, bdt, y, ldy, s)
                : launch_w4_splitk_reduce<false>(ws, splits, M, N, bias, bdt, y, ldy, s);
+}
+
+hipError_t launch_w4_pc(const void* x, int64_t ldx, bool xbf16, const int32_t* qw, int64_t ldq, const void* scales,
+                        int sdt, int64_t lds, const int32_t* zeros, int64_t ldz, const void* bias, int bdt, void* y,
+                        int64_t ldy, float* ws, int M, int N, int K, int gs, bool single_group, int split_k,
+                        hipStream_t s) {
+  return launch_pc<4>(x, ldx, xbf16, qw, ldq, scales, sdt, lds, zeros, ldz, bias, bdt, y, ldy, ws, M, N, K, gs,
+                      single_group, split_k, s);
+}
+
+hipError_t launch_w8_pc(const void* x, int64_t ldx, bool xbf16, const int8_t* qw, int64_t ldq, const void* scales,
+                        int sdt, int64_t lds, const void* bias, int bdt, void* y, int64_t ldy, float* ws, int M, int N,
+                        int K, int gs, bool single_group, int split_k, hipStream_t s) {
+  return launch_pc<8>(x, ldx, xbf16, qw, ldq, scales, sdt, lds, nullptr, 0, bias, bdt, y, ldy, ws, M, N, K, gs,
+                      single_group, split_k, s);
 }
 
 }  // namespace fg

@@ -64,3 +64,20 @@ def test_forced_prefill_still_refuses_what_it_refused():
     from forge_amd import _lib
     with pytest.raises(_lib.KernelLaunchError, match="K%64"):
         ops.w4a16_linear(x_act(70, 96).to(DEV), p, config={"impl": "prefill"})
+
+
+@pytest.mark.parametrize("m,n,k,gs,xdt,bdt", [
+    (3, 130, 96, -1, BF, None), (6, 3072, 1376, -1, HF, BF), (64, 4096, 160, 32, BF, BF), (70, 6144, 4096, -1, BF, None),
+    (128, 1030, 1056, 96, HF, HF), (200, 4096, 2048, 64, HF, None), (256, 520, 4096, 32, BF, BF), (700, 3074, 1376, -1, BF, None)])
+def test_int8_weights(m, n, k, gs, xdt, bdt):
+    """W8A16 in the same kernel: groups of 32 / 64 / 96 / one, K tails, splits; |q| up to 128."""
+    q = torch.randint(-128, 128, (n, k), generator=gen(m + k), dtype=torch.int8)
+    s = (torch.rand(n, L.num_groups(k, gs), generator=gen(1)) * 0.01).half()
+    p = L.pack_w8(q, s, gs).to(DEV)
+    x = x_act(m, k, xdt, seed=m)
+    b = None if bdt is None else torch.randn(n, generator=gen(3)).to(bdt)
+    y = ops.w8a16_linear(x.to(DEV), p, None if b is None else b.to(DEV))
+    assert ops.last_kernel().startswith("w4_pc_kernel<") and ",w8>" in ops.last_kernel(), ops.last_kernel()
+    w = q.double() * s.double().repeat_interleave(k if gs < 0 else gs, 1)[:, :k]
+    ref = x.double() @ w.t() + (0 if b is None else b.double())
+    assert_close(y.cpu(), ref.float().numpy(), "bfloat16" if xdt == BF else "float16", what=ops.last_kernel())
