@@ -957,7 +957,7 @@ int fg_fp8_gemm(const uint8_t* a, int64_t lda, const float* sa, int64_t sa_sm, i
                                    "both 16-byte aligned operands; tile_n (32, 64, 128 for tile_m=64, 128 for "
                                    "tile_m=128) the same");
     if (ring) {
-        return hip_status(fg::launch_fp8_gemm_ring(a, lda, sa, sa_sm, b, ldb, sb, sb_sn, bias, bias_dtype, y, ldy,
+      return hip_status(fg::launch_fp8_gemm_ring(a, lda, sa, sa_sm, b, ldb, sb, sb_sn, bias, bias_dtype, y, ldy,
                                                  y_dtype, (int)M, (int)N, (int)K, tile, ring, s),
                         "fg_fp8_gemm launch");
     }

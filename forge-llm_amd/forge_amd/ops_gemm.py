@@ -943,6 +943,12 @@ class _PackedLinear(nn.Module):
     def _linear(self, x: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
         raise NotImplementedError
 
+    def _tensor(self, name: str) -> torch.Tensor | None:
+        """Buffer ``name`` past nn.Module.__getattr__, whose search every forward would pay; a tensor that a program has
+        put in the buffer's place (a Parameter, a parametrisation) is found as any attribute is."""
+        buffers = self._buffers
+        return buffers[name] if name in buffers else getattr(self, name)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         bias = self.bias
         return self._linear(x, None if bias is None else bias.to(x.dtype))
@@ -1011,9 +1017,8 @@ class KernelW4A16Linear(_PackedLinear):
         return cls.from_packed(pack_w4(q, s, z, group_size, layout), b)
 
     def packed(self) -> PackedW4:
-        buf = self._buffers  # past nn.Module.__getattr__, which looks a buffer up in four dicts (every forward)
-        return PackedW4(buf["qweight"], buf["scales"], buf["zeros"], self.layout, self.out_features, self.in_features,
-                        self.group_size, buf["g_idx"], self._meta)
+        return PackedW4(self._tensor("qweight"), self._tensor("scales"), self._tensor("zeros"), self.layout,
+                        self.out_features, self.in_features, self.group_size, self._tensor("g_idx"), self._meta)
 
     def prepare(self) -> KernelW4A16Linear:
         """Host-synchronising preparation (repack, act-order sort) done now, so forward never syncs; runs after
@@ -1096,8 +1101,8 @@ class KernelW8A16Linear(_PackedLinear):
         return cls.from_packed(pack_w8(q, s, group_size), b)
 
     def packed(self) -> PackedW8:
-        buf = self._buffers
-        return PackedW8(buf["qweight"], buf["scales"], PORTABLE_W8, self.out_features, self.in_features, self.group_size)
+        return PackedW8(self._tensor("qweight"), self._tensor("scales"), PORTABLE_W8, self.out_features, self.in_features,
+                        self.group_size)
 
     def dequantize(self, dtype: torch.dtype | None = None) -> torch.Tensor:
         return self.packed().dequantize(dtype or torch.float32)

@@ -62,3 +62,11 @@ def test_stamp_changes_with_every_tensor(sym, act_order):
     p.scales = p.scales.clone()
     seen.add(ops._stamp(p))
     assert len(seen) == len(p.tensors()) + 2
+
+
+@pytest.mark.parametrize("name", ["qweight", "scales"])
+@pytest.mark.parametrize("cls", [ops.KernelW4A16Linear, ops.KernelW8A16Linear])
+def test_packed_follows_a_parameter_in_a_buffers_place(cls, name):
+    mod = cls.from_dense(torch.nn.Linear(64, 16, bias=False))
+    setattr(mod, name, torch.nn.Parameter(getattr(mod, name).clone(), requires_grad=False))
+    assert getattr(mod.packed(), name) is getattr(mod, name) is mod._parameters[name]
