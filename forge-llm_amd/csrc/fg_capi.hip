@@ -324,39 +324,54 @@ bool ring_policy(const fg_w4_config* cfg, int64_t M, int64_t N, int64_t K) {
 // follow M (w4_pc_plan), ahead of the all-rounder on every shape measured; that one where neither's conditions hold.
 constexpr int64_t kPpMinTiles = 160;
 int64_t pp_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
-int prefill_kernel(int tile_n, int64_t M, int64_t N, bool pp, bool pc, bool big, bool skinny_first) {
+// W4: whether the ping-pong kernel, its K split three ways, is ahead of the producer / consumer kernel below kPpMinTiles:
+// with more than a quarter and at most a third of the CUs in tiles the three splits fit one round, while the other kernel's
+// 256-row tiles fill only half to two thirds of one and its 128-row tiles exceed it.  Below K = 4096 the partials cost what
+// the shorter slices save.  (us, producer-consumer / ping-pong, 80 tiles, M=1111, N=4096: K=4096 65.7 / 57.1, K=14336 184.6 /
+// 146.4; outside, M=512: 48 tiles, N=6144, K=4096 50.4 / 53.0, 32 tiles, N=4096, K=14336 75.0 / 87.4.)
+bool w4_pp_thirds(int64_t M, int64_t N, int64_t K) {
+  const int64_t t = pp_tiles(M, N), cus = fg::device_cus();
+  return M >= 256 && K >= 4096 && 4 * t > cus && 3 * t <= cus && ((M + 127) / 128) * ((N + 127) / 128) > cus;
+}
+// `pp_below`: the ping-pong kernel also below kPpMinTiles
+int prefill_kernel(int tile_n, int64_t M, int64_t N, bool pp, bool pc, bool big, bool skinny_first, bool pp_below) {
   if (tile_n == 256 && pp) return 5;
   if (tile_n == 128 && pc) return 4;
   if (tile_n == 64 && big) return 2;
   if (skinny_first) return 1;
-  if (M >= 256 && pp && pp_tiles(M, N) >= kPpMinTiles) return 5;
+  if (M >= 256 && pp && (pp_below || pp_tiles(M, N) >= kPpMinTiles)) return 5;
   if (pc) return 4;
   return big ? 2 : 0;
 }
 
-// W8A16 has no producer / consumer kernel.  Below kPpMinTiles tiles from 256 rows, the ping-pong kernel with its K
-// split two or four ways (the fewest that bring tiles x splits to kPpMinTiles) still beats the all-rounder; where four
-// ways stay short of it, the all-rounder wins (graph replays over four distinct weights, us, all-rounder / ping-pong
-// split 2 / split 4: qkv M = 512 65.7 / 66.3 / 51.2, M = 1024 86.9 / 77.8 / 90.9; o_proj M = 512 44.8 / 62.8 / 46.0,
-// M = 1024 67.1 / 70.4 / 61.3, M = 2048 96.4 / 93.8 / 114.2; down M = 512 95.4 / 163.8 / 98.9, M = 1024 159.0 /
-// 174.9 / 133.7, M = 2048 262.8 / 228.5 / 243.6).  Returns that split, 1 from kPpMinTiles tiles, 0 for the
+// W8A16 has no producer / consumer kernel from 384 rows.  Below kPpMinTiles tiles from 256 rows the ping-pong kernel, its
+// K split up to four ways, beats the all-rounder down to 40 tiles (graph replays over four distinct weights, us, all-rounder
+// / ping-pong split 2 / split 4: qkv M = 512 65.7 / 66.3 / 51.2, M = 1024 86.9 / 77.8 / 90.9; o_proj M = 512 44.8 / 62.8 /
+// 46.0, M = 1024 67.1 / 70.4 / 61.3, M = 2048 96.4 / 93.8 / 114.2; down M = 512 95.4 / 163.8 / 98.9, M = 1024 159.0 / 174.9 /
+// 133.7, M = 2048 262.8 / 228.5 / 243.6).  As many splits of at least 512 columns as one round over the CUs holds (splits of
+// 1 / 2 / 3 / 4: 144 tiles, K=4096 96.4 / 129.1 / 114.4 / 137.6, K=14336 300.8 / 351.8 / 275.9 / 310.2; 96 tiles, K=4096
+// 95.1 / 71.5 / 92.9 / 91.7; 80 tiles, K=4096 94.7 / 65.0 / 58.5 / 80.4, K=14336 297 / 168 / 152 / 195; 72 tiles, K=4096
+// 94.1 / 63.5 / 53.6 / 76.2, K=8192 175.6 / 106.4 / 95.5 / 127.9).  Returns that number, 1 from kPpMinTiles tiles, 0 for the
 // all-rounder.
-int w8_pp_split(int64_t M, int64_t N) {
+int w8_pp_split(int64_t M, int64_t N, int64_t K) {
   if (M < 256) return 0;
   const int64_t t = pp_tiles(M, N);
-  return t >= kPpMinTiles ? 1 : (2 * t >= kPpMinTiles ? 2 : (4 * t >= kPpMinTiles ? 4 : 0));
+  if (t >= kPpMinTiles) return 1;
+  if (4 * t < kPpMinTiles) return 0;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({4, fg::device_cus() / t, K / 512}));
 }
 
 // Split-K workspace of the prefill kernel prefill_kernel picks for this shape and tile_n (for W8A16 also the split
 // ping-pong launch w8_pp_split picks), and of those it falls back to when the operands rule a kernel out at launch
 // (the ping-pong kernel falls back to the producer / consumer kernel, W4 only, and both to the all-rounder).
 size_t prefill_workspace_bytes(int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool w4) {
-  const bool pp = tile_n == 256 || (tile_n == 0 && M >= 256 && pp_tiles(M, N) >= kPpMinTiles);
+  const bool pp = tile_n == 256 || (tile_n == 0 && M >= 256 && (pp_tiles(M, N) >= kPpMinTiles ||
+                                                                 (w4 && w4_pp_thirds(M, N, K))));
   const bool pc = w4 && tile_n != 64;
   size_t b = fg::w4_big_workspace_bytes((int)M, (int)N, (int)K, split_k, !w4);
   if (pp) b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k));
-  if (!w4 && tile_n == 0 && w8_pp_split(M, N) > 1)
-    b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k > 0 ? split_k : w8_pp_split(M, N)));
+  if (!w4 && tile_n == 0 && w8_pp_split(M, N, K) > 0)
+    b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k > 0 ? split_k : w8_pp_split(M, N, K)));
   if (pc) b = std::max(b, fg::w4_pc_workspace_bytes(false, (int)M, (int)N, (int)K, split_k));
   return b;
 }
@@ -535,7 +550,7 @@ int w4a16_run(const void* x, int64_t ldx, int x_dtype, const int32_t* qweight, i
     int kern = 0;
     if (p.impl == FG_W4_PREFILL)
       kern = prefill_kernel(cfg ? cfg->tile_n : 0, M, N, pp, pc, big,
-                            auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096);
+                            auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096, w4_pp_thirds(M, N, K));
     else
       kern = skinny ? 1 : ((auto_impl && pc) ? 4 : ((auto_impl && big) ? 2 : 0));
     if (ring_policy(cfg, M, N, K) && perm == nullptr &&
@@ -854,16 +869,16 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
     e = fg::launch_w8_pc(x, ldx, xbf16, qweight, ldq, scales, scale_dtype, lds, bias, bias_dtype, y, ldy,
                          static_cast<float*>(workspace), (int)M, (int)N, (int)K, gs, G == 1, 0, s);
   } else if (kern == 2) {
-    // the ping-pong kernel or the all-rounder, by the W4A16 rule; where W4A16 would take the producer / consumer
-    // kernel (none for int8 weights), the ping-pong kernel with its K split as w8_pp_split says
+    // the ping-pong kernel or the all-rounder, by the W4A16 rule; below its tile count the ping-pong kernel with its K
+    // split as w8_pp_split says
     const bool pp = fg::w8_pp_ok(x, ldx, qweight, ldq, scales, scale_dtype, lds, M, N, K, gs, G) &&
                     !(cfg && cfg->tile_m);
     const int tn = cfg ? cfg->tile_n : 0;
-    int pk = prefill_kernel(tn, M, N, pp, false, big, false);
+    int pk = prefill_kernel(tn, M, N, pp, false, big, false, false);
     int split = cfg ? cfg->split_k : 0;
-    if (pk != 5 && pp && tn == 0 && w8_pp_split(M, N) > 1) {
+    if (pk != 5 && pp && tn == 0 && w8_pp_split(M, N, K) > 0) {
       pk = 5;
-      if (split <= 0) split = w8_pp_split(M, N);
+      if (split <= 0) split = w8_pp_split(M, N, K);
     }
     const size_t need = pk == 5 ? fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split)
                                 : fg::w4_big_workspace_bytes((int)M, (int)N, (int)K, split, true);
