@@ -119,7 +119,8 @@ __global__ void __launch_bounds__(256) quant_fp8_rowwise_kernel(const void* __re
 // in 1 x 128 blocks (a workgroup per block).  Here a row is read once, 8 values per lane and 16-byte load, and stays in
 // registers; the absolute maximum is a packed 16-bit integer maximum of the bit patterns (their order is the order of
 // magnitudes, a NaN above every number); and the quotient by the row's scale is exact with five multiply-adds.  The same
-// four calls: 4.8, 18.9 (5.3 TB/s), 9.5 and 7.3 us (kernel trace).
+// four calls: 4.8, 18.9 (5.3 TB/s), 10.0 and 7.3 us (kernel trace; the third with the norm's sum in the element-wise
+// kernel's order, which costs 0.5 us of it: row_sum_sq).
 
 // RN(a / b) from y = RN(1 / b): q0 = a y is within two units in the last place, one correction brings it within one,
 // and the second correction of a quotient that close is the correctly rounded one (Markstein, "Computation of
@@ -223,12 +224,46 @@ __device__ __forceinline__ float pattern_f(uint32_t b) {
 }
 __device__ __forceinline__ bool pattern_nan(bool bf16, uint32_t b) { return b > (bf16 ? 0x7f80u : 0x7c00u); }
 
-// One workgroup per row; thread t holds the row's 16-byte units t, t + T, .. (C of them at most, T threads).
+// Sum of squares of a row of K 16-bit values that lies in LDS as pairs, in the order of quant_fp8_rowwise_kernel's 256
+// threads (thread v sums columns v, v + 256, .. in turn, then wave_sum, then the four wavefronts in turn), so that the
+// normed values and their codes are the same bytes whichever kernel a row takes.  A thread of the first two wavefronts
+// (with one wavefront, each thread twice) stands for two neighbours v = 2 t, 2 t + 1, whose columns are one pair.  (us,
+// graph replays, element-wise kernel / this one / each thread summing the units it holds: 32 x 4096 13.3 / 3.8 / 3.3,
+// 1024 x 4096 18.7 / 7.0 / 6.5, 1024 x 14336 77.4 / 17.1 / 16.4.)
+template <bool BF16>
+__device__ __forceinline__ float row_sum_sq(const uint32_t* pairs, int K, int T, float* red) {
+  const auto lo = [](uint32_t w) { return BF16 ? __uint_as_float(w << 16) : f16_bits_to_f32((uint16_t)w); };
+  const auto hi = [](uint32_t w) { return BF16 ? __uint_as_float(w & 0xffff0000u) : f16_bits_to_f32((uint16_t)(w >> 16)); };
+  if (threadIdx.x < 128) {
+    for (int t = threadIdx.x; t < 128; t += T) {  // T is 64 or at least 128
+      float a = 0.f, b = 0.f;
+#pragma unroll 4
+      for (int p = t; p < K / 2; p += 128) {
+        const uint32_t w = pairs[p];
+        a = __builtin_fmaf(lo(w), lo(w), a);
+        b = __builtin_fmaf(hi(w), hi(w), b);
+      }
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) {  // wave_sum's exchanges over 32, 16, .., 2 columns' threads
+        a += __shfl_xor(a, off, kWave);
+        b += __shfl_xor(b, off, kWave);
+      }
+      if ((t & 31) == 0) red[t >> 5] = a + b;  // ... and over neighbours
+    }
+  }
+  __syncthreads();
+  return ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+// One workgroup per row; thread t holds the row's 16-byte units t, t + T, .. (C of them at most, T threads).  With the norm
+// the row also goes through LDS (2 K bytes), for the order of the sum above.
 template <int C, bool BF16, bool FP8, bool RMS>
 __global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                           uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ s,
                                                           int K, const void* __restrict__ rms_w, int wdt, float eps) {
-  __shared__ uint32_t red[2][16];
+  extern __shared__ __align__(16) uint4 row_units[];
+  __shared__ uint32_t red[16];
+  __shared__ float red_ss[4];
   const int64_t row = blockIdx.x;
   const int T = blockDim.x, units = K / 8, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = T >> 6;
   const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
@@ -240,21 +275,13 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __rest
   }
   float rs = 1.f;
   if (RMS) {
-    float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      float f[8];
-      unpack8<BF16>(u[c], f);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(f[i], f[i], ss);
+      const int k = threadIdx.x + c * T;
+      if (k < units) row_units[k] = u[c];
     }
-    ss = wave_sum(ss);
-    if (waves > 1) {
-      if (lane == 0) red[0][wave] = __float_as_uint(ss);
-      __syncthreads();
-      ss = 0.f;
-      for (int w = 0; w < waves; ++w) ss += __uint_as_float(red[0][w]);
-    }
+    __syncthreads();
+    const float ss = row_sum_sq<BF16>(reinterpret_cast<const uint32_t*>(row_units), K, T, red_ss);
     rs = __fdiv_rn(1.f, __fsqrt_rn(__fdiv_rn(ss, (float)K) + eps));
   }
   auto normed = [&](int c, float (&f)[8]) {
@@ -288,9 +315,9 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __rest
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, kWave));
   if (waves > 1) {
-    if (lane == 0) red[1][wave] = m;
+    if (lane == 0) red[wave] = m;
     __syncthreads();
-    for (int w = 0; w < waves; ++w) m = max(m, red[1][w]);
+    for (int w = 0; w < waves; ++w) m = max(m, red[w]);
   }
   const bool nan = RMS ? m > 0x7f800000u : pattern_nan(BF16, m);
   const float amax = RMS ? __uint_as_float(m) : pattern_f<BF16>(m);
@@ -338,6 +365,8 @@ __global__ void __launch_bounds__(256) quant_row_blocks_kernel(const uint16_t* _
   *reinterpret_cast<uint2*>(q + (int64_t)row * ldq + k) = encode8<true>(f, scale, __fdiv_rn(1.f, scale), fast);
 }
 
+constexpr int kQuantNormMaxK = 32000;
+
 // Whether x and q can be accessed in 16- and 8-byte units: 16-bit values in whole units, aligned rows.
 static bool quant_vec_ok(const void* x, int64_t ldx, int xdt, const void* q, int64_t ldq, int64_t K) {
   return (xdt == FG_BF16 || xdt == FG_F16) && K % 8 == 0 && ldx % 8 == 0 && ldq % 8 == 0 &&
@@ -360,7 +389,7 @@ static hipError_t launch_quant_rows(const void* x, int64_t ldx, int xdt, uint8_t
                                     int K, int T, int C, const void* rms_w, int wdt, float eps, hipStream_t st) {
   auto go = [&](auto c_tag, auto bf_tag) {
     hipLaunchKernelGGL((quant_rows_kernel<decltype(c_tag)::value, decltype(bf_tag)::value, FP8, RMS>), dim3(M), dim3(T),
-                       0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, K, rms_w, wdt, eps);
+                       RMS ? (size_t)K * 2 : 0, st, static_cast<const uint16_t*>(x), ldx, q, ldq, s, K, rms_w, wdt, eps);
     return hipGetLastError();
   };
   auto pick = [&](auto bf_tag) {
@@ -554,7 +583,9 @@ hipError_t launch_quant_fp8(const void* x, int64_t ldx, int xdt, uint8_t* q, int
                             const float* static_scale, const void* rms_w, int wdt, float eps, int fuse,
                             hipStream_t st) {
   int C = 0;
-  const int T = !static_scale && quant_vec_ok(x, ldx, xdt, q, ldq, K) && reinterpret_cast<uintptr_t>(rms_w) % 16 == 0
+  // with the norm a row lies in LDS beside the reductions' words: at most 32000 columns
+  const int T = !static_scale && quant_vec_ok(x, ldx, xdt, q, ldq, K) && !(fuse && K > kQuantNormMaxK) &&
+                        reinterpret_cast<uintptr_t>(rms_w) % 16 == 0
                     ? quant_rows_plan(M, K, &C)
                     : 0;
   if (T && fuse) return launch_quant_rows<true, true>(x, ldx, xdt, q, ldq, s, M, K, T, C, rms_w, wdt, eps, st);
