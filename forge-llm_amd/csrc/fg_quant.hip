@@ -302,6 +302,7 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(const uint16_t* __rest
   if (RMS) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
+      if (threadIdx.x + c * T >= units) continue;  // zeros past the row, which an infinite rs would turn into NaN
       float f[8];
       normed(c, f);
 #pragma unroll

@@ -75,3 +75,15 @@ def test_norm_rowwise_equals_elementwise(m, k, dt, wdt):
     w = None if wdt is None else (1 + 0.1 * torch.randn(k, generator=gen(1))).to(wdt).to(DEV)
     _same(ops.quantize_act_fp8(x, rms_weight=w, rms_eps=1e-5),
           ops.quantize_act_fp8(_strided(x), rms_weight=w, rms_eps=1e-5))
+
+
+@pytest.mark.parametrize("wdt", [None, torch.bfloat16])
+@pytest.mark.parametrize("m,k", [(8, 504), (9, 520), (600, 1032), (9, 8192)])
+def test_norm_of_rows_whose_squares_underflow(m, k, wdt):
+    """eps = 0 and a row whose mean square is zero: the row is multiplied by infinity, and the threads that hold no unit
+    of it must not add a NaN of their own."""
+    x = _values(m, k, torch.bfloat16, m + k)
+    w = None if wdt is None else (1 + 0.1 * torch.randn(k, generator=gen(1))).to(wdt).to(DEV)
+    a = ops.quantize_act_fp8(x, rms_weight=w, rms_eps=0.0)
+    _same(a, ops.quantize_act_fp8(_strided(x), rms_weight=w, rms_eps=0.0))
+    assert torch.isinf(a[1][7])
