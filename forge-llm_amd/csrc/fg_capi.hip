@@ -333,17 +333,6 @@ bool w4_pp_thirds(int64_t M, int64_t N, int64_t K) {
   const int64_t t = pp_tiles(M, N), cus = fg::device_cus();
   return M >= 256 && K >= 4096 && 4 * t > cus && 3 * t <= cus && ((M + 127) / 128) * ((N + 127) / 128) > cus;
 }
-// `pp_below`: the ping-pong kernel also below kPpMinTiles
-int prefill_kernel(int tile_n, int64_t M, int64_t N, bool pp, bool pc, bool big, bool skinny_first, bool pp_below) {
-  if (tile_n == 256 && pp) return 5;
-  if (tile_n == 128 && pc) return 4;
-  if (tile_n == 64 && big) return 2;
-  if (skinny_first) return 1;
-  if (M >= 256 && pp && (pp_below || pp_tiles(M, N) >= kPpMinTiles)) return 5;
-  if (pc) return 4;
-  return big ? 2 : 0;
-}
-
 // W8A16 has no producer / consumer kernel from 384 rows.  Below kPpMinTiles tiles from 256 rows the ping-pong kernel, its
 // K split up to four ways, beats the all-rounder down to 40 tiles (graph replays over four distinct weights, us, all-rounder
 // / ping-pong split 2 / split 4: qkv M = 512 65.7 / 66.3 / 51.2, M = 1024 86.9 / 77.8 / 90.9; o_proj M = 512 44.8 / 62.8 /
@@ -361,19 +350,70 @@ int w8_pp_split(int64_t M, int64_t N, int64_t K) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({4, fg::device_cus() / t, K / 512}));
 }
 
-// Split-K workspace of the prefill kernel prefill_kernel picks for this shape and tile_n (for W8A16 also the split
-// ping-pong launch w8_pp_split picks), and of those it falls back to when the operands rule a kernel out at launch
-// (the ping-pong kernel falls back to the producer / consumer kernel, W4 only, and both to the all-rounder).
-size_t prefill_workspace_bytes(int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool w4) {
-  const bool pp = tile_n == 256 || (tile_n == 0 && M >= 256 && (pp_tiles(M, N) >= kPpMinTiles ||
-                                                                 (w4 && w4_pp_thirds(M, N, K))));
-  const bool pc = w4 && tile_n != 64;
-  size_t b = fg::w4_big_workspace_bytes((int)M, (int)N, (int)K, split_k, !w4);
-  if (pp) b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k));
-  if (!w4 && tile_n == 0 && w8_pp_split(M, N, K) > 0)
-    b = std::max(b, fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split_k > 0 ? split_k : w8_pp_split(M, N, K)));
-  if (pc) b = std::max(b, fg::w4_pc_workspace_bytes(false, (int)M, (int)N, (int)K, split_k));
-  return b;
+// A kernel of a W4A16 / W8A16 call on MFMA tiles, numbered as in the launch switches, and the K splits its launch asks for
+// (0: its own plan's).
+struct TileRun {
+  int kern, split;
+};
+
+// fg_w4_config.tile_n as the tile kernels read it: 256 / 128 / 64, else 0 (the policy chooses).
+int prefill_tile_n(const fg_w4_config* cfg) {
+  const int t = cfg ? cfg->tile_n : 0;
+  return t == 256 || t == 128 || t == 64 ? t : 0;
+}
+
+// The one choice among the prefill kernels whose conditions hold, by the rules above: asked with the operands' conditions
+// for a launch, and with every combination of them for the size of its workspace.
+TileRun prefill_run(bool w4, int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool pp, bool pc, bool big,
+                    bool skinny_first) {
+  if (tile_n == 256 && pp) return {5, split_k};
+  if (tile_n == 128 && pc) return {4, split_k};
+  if (tile_n == 64 && big) return {2, split_k};
+  if (skinny_first) return {1, 0};
+  if (pp && M >= 256 && pp_tiles(M, N) >= kPpMinTiles) return {5, split_k};
+  if (pp && w4 && w4_pp_thirds(M, N, K)) return {5, split_k};
+  if (pp && !w4 && tile_n == 0 && w8_pp_split(M, N, K) > 0) return {5, split_k > 0 ? split_k : w8_pp_split(M, N, K)};
+  if (pc) return {4, split_k};
+  return {big ? 2 : 0, split_k};
+}
+
+// W4A16 on MFMA tiles (`use` FG_W4_PREFILL or FG_W4_MFMA).
+TileRun w4_tile_run(int use, bool auto_impl, int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool skinny, bool pp,
+                    bool pc, bool big) {
+  if (use == FG_W4_PREFILL)
+    return prefill_run(true, tile_n, M, N, K, split_k, pp, pc, big,
+                       auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096);
+  if (skinny) return {1, 0};
+  return auto_impl ? prefill_run(true, tile_n, M, N, K, split_k, false, pc, big, false) : TileRun{0, split_k};
+}
+
+// Split-K partials a TileRun writes.
+size_t tile_run_bytes(bool w4, TileRun r, int64_t M, int64_t N, int64_t K, int tile_m) {
+  const int m = (int)M, n = (int)N, k = (int)K;
+  if (r.kern == 5) return fg::w4_pp_workspace_bytes(m, n, k, r.split);
+  if (r.kern == 4) return fg::w4_pc_workspace_bytes(!w4, m, n, k, r.split);
+  if (r.kern == 2) return fg::w4_big_workspace_bytes(m, n, k, r.split, !w4);
+  if (r.kern != 0 || !w4) return 0;
+  int kchunk = 0, used = 1;
+  fg::w4_mfma_split_plan(m, n, k, tile_m, r.split, &kchunk, &used);
+  return used > 1 ? (size_t)used * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+// The largest of them over the operands a launch of this shape can meet.  big_shape / pc_shape: the all-rounder's and the
+// producer / consumer kernel's conditions on sizes hold.  On operands, the ping-pong kernel's conditions include the
+// producer / consumer kernel's, and those the all-rounder's.
+size_t w4_tile_bytes(int use, bool auto_impl, int tile_n, int tile_m, int64_t M, int64_t N, int64_t K, int split_k,
+                     bool big_shape, bool pc_shape) {
+  size_t most = 0;
+  int last = -1;
+  // none of them (an act-order perm, or a tile_m), the all-rounder, the producer / consumer kernel too, all three
+  for (int ok = 0; ok < (tile_m ? 1 : 4); ++ok) {
+    const bool big = ok >= 1 && big_shape, pc = ok >= 2 && pc_shape, pp = ok >= 3 && big_shape && pc_shape;
+    const TileRun r = w4_tile_run(use, auto_impl, tile_n, M, N, K, split_k, false, pp, pc, big);
+    if (r.kern != last) most = std::max(most, tile_run_bytes(true, r, M, N, K, tile_m));
+    last = r.kern;
+  }
+  return most;
 }
 
 // Kernel choice and launch shape for one W4A16 call; fg_w4a16_workspace_bytes and fg_w4a16_gemm share it so the
@@ -432,17 +472,10 @@ int plan_w4(int64_t M, int64_t N, int64_t K, int32_t group_size, bool x_aligned,
     p->max_blocks = cfg ? cfg->max_blocks : 0;
   } else if (use == FG_W4_MFMA || use == FG_W4_PREFILL) {
     p->tile_m = cfg ? cfg->tile_m : 0;
-    int kchunk = 0, used = 1;
-    fg::w4_mfma_split_plan((int)M, (int)N, (int)K, p->tile_m, cfg ? cfg->split_k : 0, &kchunk, &used);
     p->splits = cfg && cfg->split_k ? cfg->split_k : 0;
-    const size_t wm = used > 1 ? (size_t)used * (size_t)M * (size_t)N * sizeof(float) : 0;
-    if (wm > p->ws_bytes) p->ws_bytes = wm;
-    // the launch picks among the skinny, prefill and tiled MFMA kernels once the operand addresses are known (an
-    // act-order perm or misaligned operands rule some out): size the workspace for either split-K kernel
-    if (prefill_ok || (pc_shape && impl == FG_W4_AUTO)) {
-      const size_t wb = prefill_workspace_bytes(cfg ? cfg->tile_n : 0, M, N, K, p->splits, true);
-      if (wb > p->ws_bytes) p->ws_bytes = wb;
-    }
+    // the launch picks among the skinny, prefill and tiled MFMA kernels once the operand addresses are known
+    p->ws_bytes = w4_tile_bytes(use, impl == FG_W4_AUTO, prefill_tile_n(cfg), p->tile_m, M, N, K, p->splits, prefill_ok,
+                                pc_shape);
     // ... and for the LDS-ring kernel when the policy sends the call there
     if (ring_policy(cfg, M, N, K)) {
       const size_t wr = fg::w4_ring_workspace_bytes(true, (int)M, (int)N, (int)K);
@@ -542,23 +575,26 @@ int w4a16_run(const void* x, int64_t ldx, int x_dtype, const int32_t* qweight, i
     const bool big = fg::w4_big_ok(x, ldx, qweight, ldq, perm, K, gs, G) && !(cfg && cfg->tile_m);
     const bool pc = fg::w4_pc_ok(x, ldx, qweight, ldq, perm, scales, scale_dtype, lds, N, K, gs, G) &&
                     !(cfg && cfg->tile_m);
-    const bool pp = fg::w4_pp_ok(x, ldx, qweight, ldq, perm, scales, scale_dtype, lds, zeros, zeros ? ldz : 0, M, N,
-                                 K, gs, G) &&
-                    !(cfg && cfg->tile_m);
+    const bool pp = pc && fg::w4_pp_ok(x, ldx, qweight, ldq, perm, scales, scale_dtype, lds, zeros, zeros ? ldz : 0, M, N,
+                                       K, gs, G);
     // 0: LDS-tiled MFMA, 1: skinny, 2: all-round prefill, 3: LDS ring, 4: producer / consumer prefill, 5: ping-pong
     // prefill
-    int kern = 0;
-    if (p.impl == FG_W4_PREFILL)
-      kern = prefill_kernel(cfg ? cfg->tile_n : 0, M, N, pp, pc, big,
-                            auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096, w4_pp_thirds(M, N, K));
-    else
-      kern = skinny ? 1 : ((auto_impl && pc) ? 4 : ((auto_impl && big) ? 2 : 0));
+    const TileRun run = w4_tile_run(p.impl, auto_impl, prefill_tile_n(cfg), M, N, K, p.splits, skinny, pp, pc, big);
+    int kern = run.kern;
+    size_t need = tile_run_bytes(true, run, M, N, K, p.tile_m);
     if (ring_policy(cfg, M, N, K) && perm == nullptr &&
         fg::w4_ring_ok(true, x, ldx, qweight, ldq, scales, scale_dtype, lds, zeros, zeros ? ldz : 0, (int)M, N, K, gs,
-                       G) &&
-        (fg::w4_ring_workspace_bytes(true, (int)M, (int)N, (int)K) == 0 ||
-         (workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0)))
-      kern = 3;
+                       G)) {
+      const size_t wr = fg::w4_ring_workspace_bytes(true, (int)M, (int)N, (int)K);
+      if (wr == 0 || (workspace && workspace_bytes >= wr && reinterpret_cast<uintptr_t>(workspace) % 16 == 0)) {
+        kern = 3;
+        need = wr;
+      }
+    }
+    // the plan above covers every kernel a launch can take; a launch that it did not cover ends here
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+      return fail(FG_EINVAL, "fg_w4a16_gemm: kernel %d writes a workspace of %zu bytes, %zu given", kern, need,
+                  workspace ? workspace_bytes : (size_t)0);
     if (kern == 3)
       e = fg::launch_w4_ring(true, x, ldx, xbf16, qweight, ldq, scales, scale_dtype, lds, zeros, ldz, bias,
                              bias_dtype, y, ldy, (int)M, (int)N, (int)K, gs, G == 1, (int)G, workspace,
@@ -789,7 +825,12 @@ size_t fg_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_s
   if (!prefill_shape || impl == FG_W4_GENERIC || impl == FG_W4_MFMA || impl == FG_W4_GEMV) return pc;
   const size_t ring = impl == FG_W4_AUTO && w8a16_ring_rows(M, N, K) ? fg::w8a16_ring_workspace_bytes((int)M, (int)N, (int)K)
                                                                : 0;
-  return std::max({pc, ring, prefill_workspace_bytes(cfg ? cfg->tile_n : 0, M, N, K, cfg ? cfg->split_k : 0, false)});
+  const int tn = prefill_tile_n(cfg), split = cfg ? cfg->split_k : 0;
+  size_t most = std::max(pc, ring);
+  for (const bool pp : {false, true})
+    most = std::max(most, tile_run_bytes(false, prefill_run(false, tn, M, N, K, split, pp && !(cfg && cfg->tile_m), false,
+                                                            true, false), M, N, K, 0));
+  return most;
 }
 
 int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight, int64_t ldq, const void* scales,
@@ -873,15 +914,9 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
     // split as w8_pp_split says
     const bool pp = fg::w8_pp_ok(x, ldx, qweight, ldq, scales, scale_dtype, lds, M, N, K, gs, G) &&
                     !(cfg && cfg->tile_m);
-    const int tn = cfg ? cfg->tile_n : 0;
-    int pk = prefill_kernel(tn, M, N, pp, false, big, false, false);
-    int split = cfg ? cfg->split_k : 0;
-    if (pk != 5 && pp && tn == 0 && w8_pp_split(M, N, K) > 0) {
-      pk = 5;
-      if (split <= 0) split = w8_pp_split(M, N, K);
-    }
-    const size_t need = pk == 5 ? fg::w4_pp_workspace_bytes((int)M, (int)N, (int)K, split)
-                                : fg::w4_big_workspace_bytes((int)M, (int)N, (int)K, split, true);
+    const TileRun run = prefill_run(false, prefill_tile_n(cfg), M, N, K, cfg ? cfg->split_k : 0, pp, false, big, false);
+    const int pk = run.kern, split = run.split;
+    const size_t need = tile_run_bytes(false, run, M, N, K, 0);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
       return fail(FG_EINVAL, "fg_w8a16_gemm: workspace of %zu bytes needed, %zu given", need,
                   workspace ? workspace_bytes : (size_t)0);

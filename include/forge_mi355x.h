@@ -56,7 +56,8 @@ typedef struct fg_w4_config {
                            the LDS-tiled MFMA kernel over the register-resident split-K kernel used for M <= 64 */
   int32_t split_k;      /* MFMA / PREFILL: K splits (fp32 partials in the workspace, reduced in fixed order) */
   int32_t tile_n;       /* GEMV tile kernel: output channels per workgroup tile (rounded up to a multiple of 8);
-                           PREFILL: 256 / 128 / 64 = ping-pong / producer-consumer / all-round kernel */
+                           PREFILL: 256 / 128 / 64 = ping-pong / producer-consumer / all-round kernel (any other
+                           value leaves the choice to the policy) */
   int32_t gemv_kernel;  /* GEMV: FG_GEMV_SPLIT = split-K register kernel (M <= 4, K <= 65536), FG_GEMV_TILE = LDS-tiled
                            kernel, FG_GEMV_WAVE = one-wavefront-per-row-block kernel; AUTO = split when it fits,
                            else tile, else wave.  Setting rows_per_wave implies WAVE, tile_n implies TILE. */
