@@ -431,12 +431,16 @@ def _gather_columns(x2: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
     return out[:, :k]
 
 
+def _x_aligned(x2: torch.Tensor) -> bool:
+    return _ld(x2) % 8 == 0 and x2.data_ptr() % 16 == 0
+
+
 def _w4_call(x2: torch.Tensor, ops_: _W4Operands, bias: torch.Tensor | None, y: torch.Tensor,
              cfg: _lib.W4Config | None) -> None:
     L = _lib.lib()
     w = ops_.weight
     m, k = x2.shape
-    x_ok = int(_ld(x2) % 8 == 0 and x2.data_ptr() % 16 == 0)
+    x_ok = int(_x_aligned(x2))
     q_ok = int(_ld(w.qweight) % 4 == 0 and w.qweight.data_ptr() % 16 == 0)
     ws_bytes = L.fg_w4a16_workspace_bytes(m, w.n, k, w.group_size, x_ok, q_ok, int(ops_.g_idx is not None),
                                           _cfg_ref(cfg))
@@ -536,11 +540,13 @@ def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = 
         if packed.g_idx is None or packed.layout.kind == KIND_CDNA4:
             _w4_dispatch(x2, packed, b, y, config)
         else:
-            ops_ = _w4_operands(packed, x2)
-            if ops_.perm is not None:  # regular act order: x in the sorted weight's column order, then any kernel
+            ops_, cfg = _w4_operands(packed, x2), _w4_config(config)
+            # regular act order: x in the sorted weight's column order, then any kernel.  A configuration meets x as it
+            # lies where x is unaligned: the gather's aligned copy would pass what the kernel it names refuses
+            if ops_.perm is not None and (cfg is None or _x_aligned(x2)):
                 _w4_dispatch(_gather_columns(x2, ops_.perm), ops_.weight, b, y, config)
             else:
-                _w4_call(x2, ops_, b, y, _w4_config(config))
+                _w4_call(x2, ops_, b, y, cfg)
     _done("w4a16_linear")
     return y if x.dim() == 2 else y.reshape(*x.shape[:-1], packed.n)
 

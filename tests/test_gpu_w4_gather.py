@@ -5,6 +5,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from forge_amd import _lib
 from forge_amd import layouts as L
 from forge_amd import ops_gemm as ops
 from oracle import gemm as og
@@ -42,3 +43,19 @@ def test_act_order_module_reaches_the_policy_kernels(m, n, k, gs, kernel, xdt):
     assert_close(y.cpu(), ref, "bfloat16" if xdt == torch.bfloat16 else "float16", what=f"act-order {kernel}")
     mod.scales.mul_(2)  # the copies of the sorted weight follow the weight's own tensors
     assert_close(mod(x.to(DEV)).cpu(), 2 * ref, "bfloat16" if xdt == torch.bfloat16 else "float16", what="scaled")
+
+
+def test_a_forced_kernel_still_refuses_unaligned_rows():
+    """config names a kernel that needs 16-byte aligned x: refused on an act-order weight as on a plain one, not served by
+    the gather's aligned copy; the policy serves both."""
+    m, n, k = 20, 512, 1024
+    q, s, z = w4_parts(n, k, 128, False, seed=1)
+    g_idx = (torch.arange(k) // 128)[torch.randperm(k, generator=gen(2))].to(torch.int32)
+    x = x_act(m, k + 1, torch.bfloat16, seed=3).to(DEV)[:, 1:]
+    for packed in (L.pack_w4(q, s, z, 128).to(DEV), L.pack_w4(q, s, z, 128, g_idx=g_idx).to(DEV)):
+        for impl in ("mfma", "prefill", "dequant_gemm"):
+            with pytest.raises(_lib.KernelLaunchError, match="aligned"):
+                ops.w4a16_linear(x, packed, config={"impl": impl})
+    y = ops.w4a16_linear(x, packed)
+    ref = og.w4a16_gemm_ref(to_f32(x.cpu()), oracle_packed(q, s, z, 128, g_idx))
+    assert_close(y.cpu(), ref, "bfloat16", what="act-order, unaligned x")
