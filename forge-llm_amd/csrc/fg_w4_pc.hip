@@ -33,7 +33,7 @@
 // Split-K (gridDim.y > 1): each split covers `kchunk` columns and writes fp32 partials [S, M, N] to the caller's
 // workspace; w4_splitk_reduce_kernel (fg_w4_mfma.hip) sums them in a fixed order and adds the bias.
 //
-// A K that ends inside a slice (K % 64 == 32; TAIL) reads zeros in place of x past K.
+// A K that ends inside a slice (K % 64 == 32; TAIL) reads zeros in place of x past K and scales the weights there by zero.
 //
 // Requirements (w4_pc_ok): K % 32 == 0, group a multiple of 32 (or one group), N % 8 == 0, 16-bit scales with an even
 // row stride, 16-byte aligned x (ldx % 8 == 0) and qweight (ldq % 4 == 0), 4-byte aligned scales, no act-order perm.
@@ -65,7 +65,7 @@ constexpr int pc_qi(int wb) { return pc_q_bytes(wb) / 1024 / 4; }
 constexpr int kPcSI = 1;
 static_assert(pc_xi(256) == 8, "eight x loads per producer and slice");
 
-// What a TAIL launch reads in place of the 16-byte x units past K: zeros, so the weights they meet do not matter.
+// What a TAIL launch reads in place of the 16-byte x units past K: zeros, which meet weights scaled to zero.
 static __device__ __align__(16) const uint16_t g_pc_zero[8] = {};
 
 struct PcArgs {
@@ -310,11 +310,13 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   uint32_t nmask = 0x0F0F0F0Fu;
   asm("" : "+v"(nmask));  // hidden from known-bits analysis: bytes of masked words convert with v_cvt_f32_ubyte{k}
   const uint32_t zsel = a.hasz ? 0xffffffffu : 0u;
-  // one slice's weights from a stage's staging areas (q) into its weight rows (w)
-  auto dequant = [&](const uint8_t* __restrict__ q, uint8_t* __restrict__ w) __attribute__((always_inline)) {
+  // one slice's weights from a stage's staging areas (q) into its weight rows (w).  Past K (TAIL) they take a scale of
+  // zero: a weight that overflows 16 bits, times the zeros read for x there, would be a NaN
+  auto dequant = [&](int t, const uint8_t* __restrict__ q, uint8_t* __restrict__ w) __attribute__((always_inline)) {
+    const bool past = TAIL && wh && chunk0(t) + 1 >= a.K / 32;
     const uint4 qv = *reinterpret_cast<const uint4*>(q + p * kPcQI * 1024 + lane * 16);
     const uint8_t* sz = q + kPcQBytes + p * 256 + wh * 128;
-    const uint32_t sraw = *reinterpret_cast<const uint16_t*>(sz + (lane >> 1) * 2);
+    const uint32_t sraw = past ? 0u : *reinterpret_cast<const uint16_t*>(sz + (lane >> 1) * 2);
     const uint32_t zw = (*reinterpret_cast<const uint32_t*>(sz + 64 + ((lane >> 1) >> 3) * 4) & zsel) |
                         (0x88888888u & ~zsel);  // symmetric: zero-point 8
     const float sc = a.sbf16 ? bf16_bits_to_f32(sraw) : f16_bits_to_f32((uint16_t)sraw);
@@ -381,7 +383,7 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
     issue_q(t + 3, q_dst);
     // slice t + 1's staging landed (issued two iterations ago; everything after it may still be in flight)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPcXI + 2 * (kPcQI + kPcSI)) : "memory");
-    dequant(q_rd, w_wr);
+    dequant(t + 1, q_rd, w_wr);
     // slice t + 1's x rows landed and this wave's weight stores are done; then the barrier publishes stage t + 1
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPcXI + 2 * (kPcQI + kPcSI)) : "memory");
   };
@@ -396,7 +398,7 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
   issue_x(1, s1);
   issue_q(2, s2 + kQ);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPcXI + 2 * (kPcQI + kPcSI)) : "memory");  // slice 0's staging
-  dequant(s0 + kQ, s0 + kPcXBytes);
+  dequant(0, s0 + kQ, s0 + kPcXBytes);
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPcXI + 2 * (kPcQI + kPcSI)) : "memory");
   // stage of slice t: t % 3; rotate (a, b, c) = stages of (t, t + 1, t + 2)
   uint8_t *sa = s0, *sb = s1, *sc = s2;

@@ -81,3 +81,24 @@ def test_int8_weights(m, n, k, gs, xdt, bdt):
     w = q.double() * s.double().repeat_interleave(k if gs < 0 else gs, 1)[:, :k]
     ref = x.double() @ w.t() + (0 if b is None else b.double())
     assert_close(y.cpu(), ref.float().numpy(), "bfloat16" if xdt == BF else "float16", what=ops.last_kernel())
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m", [20, 100])
+@pytest.mark.parametrize("k,gs", [(1056, 32), (96, 96), (4128, -1)])
+def test_overflowing_weights_before_a_k_tail_give_infinity(m, k, gs, bits):
+    """Weights of the last 32 columns that round to an fp16 infinity: the columns past K hold nothing, so y is infinite (x
+    is positive) and not a NaN."""
+    n = 136
+    g = 1 if gs < 0 else k // gs
+    s = torch.full((n, g), 0.01).half()
+    s[:, -1] = 8000.0
+    q = torch.full((n, k), 9 if bits == 4 else 1, dtype=torch.uint8 if bits == 4 else torch.int8)
+    q[:, -32:] = 15 if bits == 4 else 100
+    x = torch.ones(m, k).half().to(DEV)
+    if bits == 4:
+        y = ops.w4a16_linear(x, L.pack_w4(q, s, torch.full((n, g), 1, dtype=torch.uint8), gs).to(DEV))
+    else:
+        y = ops.w8a16_linear(x, L.pack_w8(q, s, gs).to(DEV))
+    assert ops.last_kernel().startswith("w4_pc_kernel"), ops.last_kernel()
+    assert torch.isposinf(y).all()
