@@ -184,15 +184,12 @@ namespace fg {
 
 namespace {
 thread_local char g_kernel[160];
-thread_local bool g_gathered;  // the launch to come reads x as fg_w4_gather_columns left it
 }
 
 void note_kernel(const char* fmt, ...) {
-  const int at = g_gathered ? snprintf(g_kernel, sizeof(g_kernel), "gather_columns + ") : 0;
-  g_gathered = false;
   va_list ap;
   va_start(ap, fmt);
-  vsnprintf(g_kernel + at, sizeof(g_kernel) - at, fmt, ap);
+  vsnprintf(g_kernel, sizeof(g_kernel), fmt, ap);
   va_end(ap);
 }
 
@@ -209,7 +206,6 @@ int fail(int code, const char* fmt, ...) {
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
   g_err = buf;
-  fg::g_gathered = false;
   return code;
 }
 
@@ -768,10 +764,8 @@ int fg_w4_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* 
   if (!x || !perm || !out) return fail(FG_EINVAL, "fg_w4_gather_columns: null tensor");
   if (ldx < K || ldo < (K + 7) / 8 * 8 || ldo % 8 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0)
     return fail(FG_EINVAL, "fg_w4_gather_columns: out needs 16-byte aligned rows of at least K rounded up to 8");
-  const int rc = hip_status(fg::launch_gather(x, ldx, perm, out, ldo, (int)M, (int)K, static_cast<hipStream_t>(stream)),
-                            "fg_w4_gather_columns launch");
-  fg::g_gathered = rc == FG_OK;
-  return rc;
+  return hip_status(fg::launch_gather(x, ldx, perm, out, ldo, (int)M, (int)K, static_cast<hipStream_t>(stream)),
+                    "fg_w4_gather_columns launch");
 }
 
 int fg_w4_dequant(const int32_t* qweight, int64_t ldq, const void* scales, int scale_dtype, int64_t lds,

@@ -95,6 +95,7 @@ hipError_t launch_gather(const void* x, int64_t ldx, const int32_t* perm, void* 
   const uint16_t* xi = static_cast<const uint16_t*>(x);
   uint16_t* o = static_cast<uint16_t*>(out);
   const int units = (K + 7) / 8, c = (units + kGatherThreads - 1) / kGatherThreads;
+  note_kernel("gather_columns");
   const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(perm) % 16 == 0;  // whole units of perm ...
   if (M <= kGatherDirectM || K > kGatherMaxK) {
     auto k = vec ? gather_direct_kernel<true> : gather_direct_kernel<false>;

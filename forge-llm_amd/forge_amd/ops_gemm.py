@@ -62,6 +62,13 @@ _ONCE: set[str] = set()
 _ONCE_LOCK = threading.Lock()
 
 
+class _Thread(threading.local):
+    gathered = False  # this thread's last op gathered x's columns
+
+
+_THREAD = _Thread()
+
+
 # ================================================================================================ switches
 def _env_reader(name: str) -> Callable[[], str]:
     """A function that reads environment variable ``name`` ("" when unset) as it is now.  Every op asks for several:
@@ -100,9 +107,10 @@ def last_path(op: str) -> str | None:
 
 
 def last_kernel() -> str:
-    """The kernel, with its launch form, that this thread's last op ran (``fg_last_kernel``): finer than
-    :func:`last_path`, which names the path only."""
-    return _lib.last_kernel()
+    """The kernel, with its launch form, that this thread's last op ran (``fg_last_kernel``), behind the column gather
+    where the op put one in front: finer than :func:`last_path`, which names the path only."""
+    kernel = _lib.last_kernel()
+    return f"gather_columns + {kernel}" if _THREAD.gathered and kernel != "gather_columns" else kernel
 
 
 def reset_failure_memo() -> None:
@@ -167,6 +175,7 @@ def _on_gpu(t: torch.Tensor, op: str) -> None:
     if force_ref():
         raise HardwareUnsupported(f"{op}: FORGE_FORCE_REF=1 asks for the torch reference path, which forge_amd does "
                                   "not include (run the reference implementation for that)")
+    _THREAD.gathered = False
     _lib.require_device(t, op)
     if not _SELFTEST.passed(t.get_device()):
         _SELFTEST.ensure(t)
@@ -428,6 +437,7 @@ def _gather_columns(x2: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
     out = torch.empty((m, (k + 7) // 8 * 8), dtype=x2.dtype, device=x2.device)
     _check(_lib.lib().fg_w4_gather_columns(_lib.ptr(x2), _ld(x2), _lib.ptr(perm), _lib.ptr(out), out.stride(0), m, k,
                                            _lib.stream_of(x2)), "fg_w4_gather_columns")
+    _THREAD.gathered = True
     return out[:, :k]
 
 

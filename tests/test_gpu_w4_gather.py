@@ -59,3 +59,13 @@ def test_a_forced_kernel_still_refuses_unaligned_rows():
     y = ops.w4a16_linear(x, packed)
     ref = og.w4a16_gemm_ref(to_f32(x.cpu()), oracle_packed(q, s, z, 128, g_idx))
     assert_close(y.cpu(), ref, "bfloat16", what="act-order, unaligned x")
+
+
+def test_the_gathers_label_ends_with_its_op():
+    """A gather that no product followed (a failed allocation in between) does not name the next op's kernel."""
+    x = x_act(20, 512, torch.bfloat16, seed=1).to(DEV)
+    ops._gather_columns(x, torch.randperm(512, generator=gen(1)).to(torch.int32).to(DEV))
+    assert ops.last_kernel() == "gather_columns"
+    a = torch.ones(64, 256, dtype=torch.int8, device=DEV)
+    ops.int8_gemm(a, None, a, None, out_dtype=torch.int32)
+    assert "gather" not in ops.last_kernel(), ops.last_kernel()
