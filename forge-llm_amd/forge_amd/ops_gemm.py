@@ -74,10 +74,11 @@ def _env_reader(name: str) -> Callable[[], str]:
     """A function that reads environment variable ``name`` ("" when unset) as it is now.  Every op asks for several:
     ``os.environ.get`` encodes the name and decodes the value each time (0.8 us), the mapping behind it holds both as
     bytes."""
-    data, key = getattr(os.environ, "_data", None), os.fsencode(name)
-    if not isinstance(data, dict):
-        return lambda: os.environ.get(name, "")
+    key = os.fsencode(name)
     def read() -> str:
+        data = getattr(os.environ, "_data", None)  # looked up each time: a program may put another mapping in its place
+        if type(data) is not dict:
+            return os.environ.get(name, "")
         value = data.get(key)
         return "" if value is None else os.fsdecode(value)
     return read

@@ -24,6 +24,13 @@ def test_switches_follow_the_environment(monkeypatch):
     assert not ops.force_ref()
 
 
+def test_switches_follow_an_environment_put_in_its_place(monkeypatch):
+    monkeypatch.setattr(os, "environ", {**os.environ, "FORGE_FORCE_REF": "1", "FORGE_W4_IMPL": "gemv"})
+    assert ops.force_ref() and ops.forced_impl() == "gemv" and not ops.kernel_debug()
+    monkeypatch.undo()
+    assert not ops.force_ref() and ops.forced_impl() is None
+
+
 def _view(side, strides, i, kb):
     return side.as_strided((1,), (1,), side.storage_offset() + i * strides[0] + kb * strides[1]).item()
 
