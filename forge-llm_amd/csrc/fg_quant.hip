@@ -511,10 +511,11 @@ __global__ void __launch_bounds__(256) quant_fp8_tile_encode_kernel(const void* 
   }
 }
 
-// One row per block, 16-byte accesses, several blocks per wavefront: units a power of two of lanes holds.
+// One row per block, 16-byte accesses, several blocks per wavefront: units a power of two of lanes holds.  A launch has
+// fewer than 2^32 threads, one per unit here.
 static bool quant_row_blocks_ok(const void* x, int64_t ldx, int xdt, const void* q, int64_t ldq, int64_t M, int64_t K,
                                 int64_t bk) {
-  return bk >= 8 && bk <= 512 && (bk & (bk - 1)) == 0 && M * ((K + bk - 1) / bk) < (1LL << 31) &&
+  return bk >= 8 && bk <= 512 && (bk & (bk - 1)) == 0 && M * ((K + bk - 1) / bk) * (bk / 8) < (1LL << 32) - 256 &&
          quant_vec_ok(x, ldx, xdt, q, ldq, K);
 }
 
