@@ -572,9 +572,11 @@ static hipError_t launch_ring_t(const uint8_t* A, int64_t lda, const uint8_t* B,
   return hipGetLastError();
 }
 
-// Instances (BM x BN, wavefronts, stages), each the fastest of those measured for its size: 64 x 32 with 2 x 2
-// wavefronts and 5 stages (two workgroups per CU; 8 stages, one per CU, level in the first round of workgroups and 20-30%
-// slower past it), 64 x 64 with 2 x 4 and 6, or 4 once there is more than one workgroup per CU (two are then resident:
+// Instances (BM x BN, wavefronts, stages), each the fastest of those measured for its size: 64 x 32 with 2 x 2 wavefronts
+// and 6 stages (the policy takes that tile where its workgroups are one per CU or fewer; us at 5 / 6 / 8 stages: fp8
+// N=8192, M=17 K=28672 61.1 / 57.2 / 56.5, K=8192 17.9 / 17.2 / 17.4; int8 N=4096, K=14336, M=64 29.5 / 29.5 / 30.2;
+// K=N=4096, M=33 fp8 10.1 / 10.3 / 10.4, int8 11.2 / 11.2 / 11.4: five leave too few loads in flight over long K, eight take
+// longer to fill), 64 x 64 with 2 x 4 and 6, or 4 once there is more than one workgroup per CU (two are then resident:
 // fp8 K=N=8192, M=256 39 us against 43), 64 x 128 with 2 x 4 and 4, 128 x 64 with 4 x 2 and 4, 128 x 128 with 2 x 4 and
 // 3, 192 x 64 with 4 x 2 and 4, 192 x 128 and 256 x 128 with 4 x 2 and 3.
 template <class Mma, class Epi>
@@ -586,7 +588,7 @@ static hipError_t launch_ring(const uint8_t* A, int64_t lda, const uint8_t* B, i
   if (bm == 128 && bn == 64) return launch_ring_t<Mma, 128, 64, 4, 2, 4>(A, lda, B, ldb, M, N, K, epi, s);
   if (bm == 128) return launch_ring_t<Mma, 128, 128, 2, 4, 3>(A, lda, B, ldb, M, N, K, epi, s);
   if (bn == 128) return launch_ring_t<Mma, 64, 128, 2, 4, 4>(A, lda, B, ldb, M, N, K, epi, s);
-  if (bn == 32) return launch_ring_t<Mma, 64, 32, 2, 2, 5>(A, lda, B, ldb, M, N, K, epi, s);
+  if (bn == 32) return launch_ring_t<Mma, 64, 32, 2, 2, 6>(A, lda, B, ldb, M, N, K, epi, s);
   return mm_tiles(M, N, 64, 64) > device_cus() ? launch_ring_t<Mma, 64, 64, 2, 4, 4>(A, lda, B, ldb, M, N, K, epi, s)
                                                : launch_ring_t<Mma, 64, 64, 2, 4, 6>(A, lda, B, ldb, M, N, K, epi, s);
 }
