@@ -36,6 +36,8 @@ size_t w4_big_workspace_bytes(int M, int N, int K, int split_k, bool w8);
 bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const int32_t* perm, const void* scales,
               int sdt, int64_t lds, int64_t N, int64_t K, int gs, int64_t G);
 size_t w4_pc_workspace_bytes(bool w8, int M, int N, int K, int split_k);
+int64_t w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk);
+int64_t w4_big_cost(int M, int N, int K, bool xbf16);
 bool w8_pc_ok(const void* x, int64_t ldx, const int8_t* qw, int64_t ldq, const void* scales, int sdt, int64_t lds,
               int64_t N, int64_t K, int gs, int64_t G);
 hipError_t launch_w8_pc(const void* x, int64_t ldx, bool xbf16, const int8_t* qw, int64_t ldq, const void* scales,
@@ -316,8 +318,9 @@ bool ring_policy(const fg_w4_config* cfg, int64_t M, int64_t N, int64_t K) {
 // weights, us, ping-pong / producer-consumer with 256-row tiles / all-rounder: M = 512 qkv 53.0 / 50.4 / 60.5, o_proj 48.1 / 36.9 / 40.9,
 // gate+up 114.6 / 138.6 / 135.1, down 87.4 / 75.0 / 96.9; M = 2048 qkv 108.9 / 135.2 / 131.0, o_proj 98.3 / 78.4 /
 // 93.4, gate+up 449.5 / 501.7 / 502.3, down 234.8 / 232.5 / 297.4; M = 8192 qkv 367 / 434 / 413, o_proj 246 / 294 /
-// 273, gate+up 1624 / 1916 / 1799, down 779 / 894 / 878).  Below 256 rows the producer / consumer kernel, whose row tiles
-// follow M (w4_pc_plan), ahead of the all-rounder on every shape measured; that one where neither's conditions hold.
+// 273, gate+up 1624 / 1916 / 1799, down 779 / 894 / 878).  Below 256 rows, and with groups that are no
+// multiple of 64, the producer / consumer kernel, whose row tiles follow M, or the all-rounder, by cost (w4_big_ahead);
+// the all-rounder where neither's conditions hold.
 constexpr int64_t kPpMinTiles = 160;
 int64_t pp_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
 // W4: whether the ping-pong kernel, its K split three ways, is ahead of the producer / consumer kernel below kPpMinTiles:
@@ -346,6 +349,19 @@ int w8_pp_split(int64_t M, int64_t N, int64_t K) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({4, fg::device_cus() / t, K / 512}));
 }
 
+// W4: whether the all-rounder is ahead of the producer / consumer kernel where both can run and the ping-pong kernel cannot.
+// Its 256-column tiles split a wide output with few rows into more K splits than one round of 128-column tiles leaves room
+// for, and take wide outputs in fewer rounds (us, producer-consumer / all-rounder, bf16: groups of 64, 16 rows, N=20480, K=8192
+// 87.8 / 58.1, K=4096 46.5 / 33.5, N=43008, K=4096 91.4 / 73.6; groups of 32, 512 rows, N=28672, K=4096 133.2 / 123.0, 300
+// rows, N=20480, K=2048 55.1 / 45.1; the other way: groups of 64, 16 rows, N=4096, K=8192 18.4 / 20.3, 100 rows, N=6144,
+// K=4096 23.9 / 28.2).
+bool w4_big_ahead(int64_t M, int64_t N, int64_t K, int gs, int64_t G, bool xbf16) {
+  if (M >= 256 && (gs % 64 == 0 || G == 1)) return false;
+  int bm, splits, kchunk;
+  return fg::w4_big_cost((int)M, (int)N, (int)K, xbf16) <
+         fg::w4_pc_plan(false, (int)M, (int)N, (int)K, 0, &bm, &splits, &kchunk);
+}
+
 // A kernel of a W4A16 / W8A16 call on MFMA tiles, numbered as in the launch switches, and the K splits its launch asks for
 // (0: its own plan's).
 struct TileRun {
@@ -359,9 +375,10 @@ int prefill_tile_n(const fg_w4_config* cfg) {
 }
 
 // The one choice among the prefill kernels whose conditions hold, by the rules above: asked with the operands' conditions
-// for a launch, and with every combination of them for the size of its workspace.
+// for a launch, and with every combination of them for the size of its workspace.  big_first: the all-rounder before the
+// producer / consumer kernel.
 TileRun prefill_run(bool w4, int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool pp, bool pc, bool big,
-                    bool skinny_first) {
+                    bool skinny_first, bool big_first) {
   if (tile_n == 256 && pp) return {5, split_k};
   if (tile_n == 128 && pc) return {4, split_k};
   if (tile_n == 64 && big) return {2, split_k};
@@ -369,18 +386,18 @@ TileRun prefill_run(bool w4, int tile_n, int64_t M, int64_t N, int64_t K, int sp
   if (pp && M >= 256 && pp_tiles(M, N) >= kPpMinTiles) return {5, split_k};
   if (pp && w4 && w4_pp_thirds(M, N, K)) return {5, split_k};
   if (pp && !w4 && tile_n == 0 && w8_pp_split(M, N, K) > 0) return {5, split_k > 0 ? split_k : w8_pp_split(M, N, K)};
-  if (pc) return {4, split_k};
+  if (pc && !(big && big_first)) return {4, split_k};
   return {big ? 2 : 0, split_k};
 }
 
 // W4A16 on MFMA tiles (`use` FG_W4_PREFILL or FG_W4_MFMA).
 TileRun w4_tile_run(int use, bool auto_impl, int tile_n, int64_t M, int64_t N, int64_t K, int split_k, bool skinny, bool pp,
-                    bool pc, bool big) {
+                    bool pc, bool big, bool big_first) {
   if (use == FG_W4_PREFILL)
     return prefill_run(true, tile_n, M, N, K, split_k, pp, pc, big,
-                       auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096);
+                       auto_impl && skinny && M <= 64 && N <= 4096 && K <= 4096, big_first);
   if (skinny) return {1, 0};
-  return auto_impl ? prefill_run(true, tile_n, M, N, K, split_k, false, pc, big, false) : TileRun{0, split_k};
+  return auto_impl ? prefill_run(true, tile_n, M, N, K, split_k, false, pc, big, false, big_first) : TileRun{0, split_k};
 }
 
 // Split-K partials a TileRun writes.
@@ -397,7 +414,8 @@ size_t tile_run_bytes(bool w4, TileRun r, int64_t M, int64_t N, int64_t K, int t
 
 // The largest of them over the operands a launch of this shape can meet.  big_shape / pc_shape: the all-rounder's and the
 // producer / consumer kernel's conditions on sizes hold.  On operands, the ping-pong kernel's conditions include the
-// producer / consumer kernel's, and those the all-rounder's.
+// producer / consumer kernel's, and those the all-rounder's; each is asked for without those before it, so the order of the
+// last two does not matter.
 size_t w4_tile_bytes(int use, bool auto_impl, int tile_n, int tile_m, int64_t M, int64_t N, int64_t K, int split_k,
                      bool big_shape, bool pc_shape) {
   size_t most = 0;
@@ -405,7 +423,7 @@ size_t w4_tile_bytes(int use, bool auto_impl, int tile_n, int tile_m, int64_t M,
   // none of them (an act-order perm, or a tile_m), the all-rounder, the producer / consumer kernel too, all three
   for (int ok = 0; ok < (tile_m ? 1 : 4); ++ok) {
     const bool big = ok >= 1 && big_shape, pc = ok >= 2 && pc_shape, pp = ok >= 3 && big_shape && pc_shape;
-    const TileRun r = w4_tile_run(use, auto_impl, tile_n, M, N, K, split_k, false, pp, pc, big);
+    const TileRun r = w4_tile_run(use, auto_impl, tile_n, M, N, K, split_k, false, pp, pc, big, false);
     if (r.kern != last) most = std::max(most, tile_run_bytes(true, r, M, N, K, tile_m));
     last = r.kern;
   }
@@ -575,7 +593,9 @@ int w4a16_run(const void* x, int64_t ldx, int x_dtype, const int32_t* qweight, i
                                        K, gs, G);
     // 0: LDS-tiled MFMA, 1: skinny, 2: all-round prefill, 3: LDS ring, 4: producer / consumer prefill, 5: ping-pong
     // prefill
-    const TileRun run = w4_tile_run(p.impl, auto_impl, prefill_tile_n(cfg), M, N, K, p.splits, skinny, pp, pc, big);
+    const bool big_first = pc && big && p.splits == 0 && w4_big_ahead(M, N, K, gs, G, xbf16);
+    const TileRun run = w4_tile_run(p.impl, auto_impl, prefill_tile_n(cfg), M, N, K, p.splits, skinny, pp, pc, big,
+                                    big_first);
     int kern = run.kern;
     size_t need = tile_run_bytes(true, run, M, N, K, p.tile_m);
     if (ring_policy(cfg, M, N, K) && perm == nullptr &&
@@ -823,7 +843,7 @@ size_t fg_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_s
   size_t most = std::max(pc, ring);
   for (const bool pp : {false, true})
     most = std::max(most, tile_run_bytes(false, prefill_run(false, tn, M, N, K, split, pp && !(cfg && cfg->tile_m), false,
-                                                            true, false), M, N, K, 0));
+                                                            true, false, false), M, N, K, 0));
   return most;
 }
 
@@ -908,7 +928,7 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
     // split as w8_pp_split says
     const bool pp = fg::w8_pp_ok(x, ldx, qweight, ldq, scales, scale_dtype, lds, M, N, K, gs, G) &&
                     !(cfg && cfg->tile_m);
-    const TileRun run = prefill_run(false, prefill_tile_n(cfg), M, N, K, cfg ? cfg->split_k : 0, pp, false, big, false);
+    const TileRun run = prefill_run(false, prefill_tile_n(cfg), M, N, K, cfg ? cfg->split_k : 0, pp, false, big, false, false);
     const int pk = run.kern, split = run.split;
     const size_t need = tile_run_bytes(false, run, M, N, K, 0);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))

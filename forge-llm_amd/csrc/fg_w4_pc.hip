@@ -442,18 +442,23 @@ bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const 
 // Rows of 64 / 128 / 256 measured (us, fp16 x, groups of 64): K=4096, N=28672 M=64 46 / 52 / -, M=128 89 / 53 / 69,
 // M=200 175 / 99 / 71; K=N=2048 M=300 17.8 / 19.2 / 22.7.  The all-rounder, which took these before: M=64 54, M=128 62,
 // M=200 89, and 22.5.
-void w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk) {
+// Returns that cost.
+int64_t w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk) {
   static const struct { int bm, ns; } kTile[] = {{64, 614}, {128, 726}, {256, 880}};
-  const int64_t cus = device_cus(), slices = (K + kPcBK - 1) / kPcBK;
+  const uint32_t cus = (uint32_t)device_cus(), slices = ((uint32_t)K + kPcBK - 1) / kPcBK;
   int64_t best = -1;
   for (const auto& t : kTile) {
     if (w8 && t.bm == 256) continue;  // three stages with 8-bit staging exceed the LDS
-    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + kPcBN - 1) / kPcBN);
-    const int64_t most = split_k > 0 ? split_k : std::max<int64_t>(1, std::min<int64_t>({16, K / 256, cus / tiles}));
-    for (int64_t s = split_k > 0 ? split_k : 1; s <= most; ++s) {
-      const int64_t per = (slices + s - 1) / s, used = (slices + per - 1) / per;
-      const int64_t rounds = (tiles * used + cus - 1) / cus;
-      const int64_t cost = rounds * (per * t.ns + 4600) + (used > 1 ? 2700 + used * M * (int64_t)N / 600 : 0);
+    const uint32_t tiles = (uint32_t)((M + t.bm - 1) / t.bm) * (uint32_t)((N + kPcBN - 1) / kPcBN);
+    const uint32_t most = split_k > 0 ? (uint32_t)split_k
+                                      : std::max(1u, std::min(std::min(16u, (uint32_t)K / 256), cus / tiles));
+    uint32_t last = 0;
+    for (uint32_t s = split_k > 0 ? most : 1; s <= most; ++s) {
+      const uint32_t per = (slices + s - 1) / s;
+      if (per == last) continue;  // one split more, no shorter ones
+      last = per;
+      const uint32_t used = (slices + per - 1) / per, rounds = (tiles * used + cus - 1) / cus;
+      const int64_t cost = (int64_t)rounds * ((int64_t)per * t.ns + 4600) + (used > 1 ? 2700 + (int64_t)used * M * N / 600 : 0);
       if (best < 0 || cost < best) {
         best = cost;
         *bm = t.bm;
@@ -462,6 +467,7 @@ void w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits,
       }
     }
   }
+  return best;
 }
 
 size_t w4_pc_workspace_bytes(bool w8, int M, int N, int K, int split_k) {

@@ -102,3 +102,22 @@ def test_overflowing_weights_before_a_k_tail_give_infinity(m, k, gs, bits):
         y = ops.w8a16_linear(x, L.pack_w8(q, s, gs).to(DEV))
     assert ops.last_kernel().startswith("w4_pc_kernel"), ops.last_kernel()
     assert torch.isposinf(y).all()
+
+
+@pytest.mark.parametrize("m,n,k,gs,xdt,expect", [
+    (16, 20480, 2048, 64, BF, "w4_big_kernel<64"),    # 80 wide tiles: three K splits in a round, against one
+    (5, 43016, 1024, 32, BF, "w4_big_kernel<64"),
+    (16, 4096, 2048, 64, BF, "w4_pc_kernel"),
+    (300, 20480, 576, 32, BF, "w4_big_kernel<128"),
+    (509, 28680, 1024, 32, BF, "w4_big_kernel<256"),
+    (513, 4104, 1152, 96, HF, "w4_pc_kernel"),
+    (300, 20480, 576, 64, BF, "w4_pp_kernel"),        # groups of 64 from 256 rows: by the other rules
+])
+def test_all_rounder_where_it_costs_less(m, n, k, gs, xdt, expect):
+    q, s, z = w4_parts(n, k, gs, False, seed=m)
+    p = L.pack_w4(q, s, z, gs).to(DEV)
+    x = x_act(m, k, xdt, seed=m)
+    y = ops.w4a16_linear(x.to(DEV), p)
+    assert ops.last_kernel().startswith(expect), ops.last_kernel()
+    ref = og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, gs))
+    assert_close(y.cpu(), ref, "bfloat16" if xdt == BF else "float16", what=expect)
