@@ -37,7 +37,7 @@ bool w4_pc_ok(const void* x, int64_t ldx, const int32_t* qw, int64_t ldq, const 
               int sdt, int64_t lds, int64_t N, int64_t K, int gs, int64_t G);
 size_t w4_pc_workspace_bytes(bool w8, int M, int N, int K, int split_k);
 int64_t w4_pc_plan(bool w8, int M, int N, int K, int split_k, int* bm, int* splits, int* kchunk);
-int64_t w4_big_cost(int M, int N, int K, bool xbf16);
+int64_t w4_big_cost(int M, int N, int K, bool xbf16, bool w8);
 bool w8_pc_ok(const void* x, int64_t ldx, const int8_t* qw, int64_t ldq, const void* scales, int sdt, int64_t lds,
               int64_t N, int64_t K, int gs, int64_t G);
 hipError_t launch_w8_pc(const void* x, int64_t ldx, bool xbf16, const int8_t* qw, int64_t ldq, const void* scales,
@@ -358,7 +358,7 @@ int w8_pp_split(int64_t M, int64_t N, int64_t K) {
 bool w4_big_ahead(int64_t M, int64_t N, int64_t K, int gs, int64_t G, bool xbf16) {
   if (M >= 256 && (gs % 64 == 0 || G == 1)) return false;
   int bm, splits, kchunk;
-  return fg::w4_big_cost((int)M, (int)N, (int)K, xbf16) <
+  return fg::w4_big_cost((int)M, (int)N, (int)K, xbf16, false) <
          fg::w4_pc_plan(false, (int)M, (int)N, (int)K, 0, &bm, &splits, &kchunk);
 }
 
@@ -814,16 +814,24 @@ static bool w8a16_ring_rows(int64_t M, int64_t N, int64_t K) {
   return M > 16 ? M <= 64 : (M > 2 && (N >= 16384 || K >= 8192));
 }
 
-// Whether a W8A16 call that neither the GEMV, the ring nor the skinny kernel takes goes to the producer / consumer kernel
-// (64- and 128-row tiles) where its operands allow: whenever K ends inside a 64-column slice (the other kernels cannot
-// read it and the generic one would serve: K=4128, N=4096, groups of 32, 6 / 64 / 512 rows 101 / 665 / 4439 us against
-// 15 / 20 / 41), for 65..128 rows, and up to 256 while its 128-row tiles fit one round (all-rounder / producer-consumer,
-// us: K=4096, N=6144 M=80 30.5 / 21.3, M=256 40.4 / 36.2; N=28672 M=128 71.9 / 56.9, M=200 -- two rounds -- 100.5 /
-// 107.8; K=14336, N=4096 M=128 46.3 / 34.6, M=256 62.5 / 55.9; from 384 rows the ping-pong kernel is ahead).  Up to 64 rows (groups that are no multiple of 128) it would
-// be ahead of the all-rounder too (K=N=4096, groups of 64, 64 rows 18.7 against 25.4), but tests/test_gpu_policy_paths.py
-// states that the policy there runs what a forced prefill runs.
+// Whether a W8A16 call that neither the GEMV, the ring nor the skinny kernel takes may go to the producer / consumer kernel
+// (64- and 128-row tiles): whenever K ends inside a 64-column slice (the other kernels cannot read it and the generic one
+// would serve: K=4128, N=4096, groups of 32, 6 / 64 / 512 rows 101 / 665 / 4439 us against 15 / 20 / 41), for 65..128 rows,
+// and up to 256 while its 128-row tiles fit one round (all-rounder / producer-consumer, us: K=4096, N=6144 M=80 30.5 / 21.3,
+// M=256 40.4 / 36.2; N=28672 M=128 71.9 / 56.9, M=200 -- two rounds -- 100.5 / 107.8; K=14336, N=4096 M=128 46.3 / 34.6,
+// M=256 62.5 / 55.9; from 384 rows the ping-pong kernel is ahead).  Up to 64 rows (groups that are no multiple of 128) it
+// would be ahead of the all-rounder too (K=N=4096, groups of 64, 64 rows 18.7 against 25.4), but
+// tests/test_gpu_policy_paths.py states that the policy there runs what a forced prefill runs.
 static bool w8_pc_rows(int64_t M, int64_t N, int64_t K) {
   return K % 64 != 0 || (M > 64 && M <= 128) || (M > 64 && M <= 256 && ((M + 127) / 128) * ((N + 127) / 128) <= fg::device_cus());
+}
+
+// ... unless the all-rounder, whose wider tiles leave room for more K splits, costs less there (all-rounder /
+// producer-consumer, us: M=130, N=10752, K=12544 94.7 / 144.6; M=129, N=K=8192 53.0 / 59.6; M=129, N=5120, K=13824 59.5 / 64.7).
+static bool w8_big_ahead(int64_t M, int64_t N, int64_t K, bool xbf16) {
+  int bm, splits, kchunk;
+  return M < 256 && fg::w4_big_cost((int)M, (int)N, (int)K, xbf16, true) <
+                        fg::w4_pc_plan(true, (int)M, (int)N, (int)K, 0, &bm, &splits, &kchunk);
 }
 
 size_t fg_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size, const fg_w4_config* cfg) {
@@ -886,12 +894,12 @@ int fg_w8a16_gemm(const void* x, int64_t ldx, int x_dtype, const int8_t* qweight
   const bool pc = w8_pc_rows(M, N, K) && fg::w8_pc_ok(x, ldx, qweight, ldq, scales, scale_dtype, lds, N, K, gs, G) &&
                   !(cfg && (cfg->tile_m || cfg->tile_n || cfg->split_k));
   if (kern < 0)
-    kern = (gemv && gemv_rows)                    ? 3
-           : (ring && w8a16_ring_rows(M, N, K))   ? 4
-           : (skinny && M <= 64)                  ? 1
-           : pc                                   ? 5
-           : big                                  ? 2
-                                                  : 0;
+    kern = (gemv && gemv_rows)                              ? 3
+           : (ring && w8a16_ring_rows(M, N, K))             ? 4
+           : (skinny && M <= 64)                            ? 1
+           : (pc && !(big && w8_big_ahead(M, N, K, xbf16))) ? 5
+           : big                                            ? 2
+                                                            : 0;
   if (kern == 3 && !gemv)
     return fail(FG_EUNSUPPORTED, "fg_w8a16_gemm: decode GEMV needs M<=4, K%%16==0, group%%16==0 (or one group), "
                                  "16-bit scales with lds%%8==0, ldq%%16==0, ldx%%8==0, 16-byte aligned x/qweight/"

@@ -394,17 +394,19 @@ void w4_big_plan(int M, int N, int K, int split_k, int* bm, int* splits, int* kc
   *splits = (K + kc - 1) / kc;
 }
 
-// Cost in ns of the automatic plan on int4 weights, in the form of w4_pc_plan's and made to be compared with it: workgroup
-// rounds times (64-column slices times a time per slice and row tile, plus a start), plus the partials.  The times are
-// those whose comparison picks the faster kernel over 767 calls (graph replays; N = 512..60000, K = 128..16384, groups of 32 /
-// 64 / 96 / 128, 5..255 rows, and 256..4096 rows with groups that are no multiple of 64): 0.16% (geometric mean) slower
-// than the faster of the two, where the producer / consumer kernel alone is at 2.6% and up to 55%.
-int64_t w4_big_cost(int M, int N, int K, bool xbf16) {
+// Cost in ns of the automatic plan, in the form of w4_pc_plan's and made to be compared with it: workgroup rounds times
+// (64-column slices times a time per slice and row tile, plus a start), plus the partials.  The times are those whose
+// comparison picks the faster kernel (graph replays; N = 512..60000, K = 128..16384): over 767 calls on int4 weights (groups
+// of 32 / 64 / 96 / 128, 5..255 rows, and 256..4096 rows with groups that are no multiple of 64) it is 0.16% (geometric
+// mean) behind the faster of the two, where the producer / consumer kernel alone is at 2.6% and up to 55%; over 248 on int8
+// weights (65..255 rows) 0.08%, against 1.2% and up to 53%.
+int64_t w4_big_cost(int M, int N, int K, bool xbf16, bool w8) {
   int bm, splits, kchunk;
-  w4_big_plan(M, N, K, 0, &bm, &splits, &kchunk, false);
+  w4_big_plan(M, N, K, 0, &bm, &splits, &kchunk, w8);
   const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + kW4BigBN - 1) / kW4BigBN), cus = device_cus();
-  const int64_t ns = bm == 64 ? 1025 : (bm == 128 ? 1275 : 1500), start = bm == 64 ? 6000 : (bm == 128 ? 2000 : 9000);
-  const int64_t slice = xbf16 ? ns : ns * 13 / 10;  // fp16 takes more instructions to round to
+  const int64_t ns = bm == 64 ? 1025 : (bm == 128 ? 1275 : (w8 ? 1800 : 1500));
+  const int64_t start = bm == 64 ? 6000 : (bm == 128 ? (w8 ? 15000 : 2000) : (w8 ? 2000 : 9000));
+  const int64_t slice = xbf16 ? ns : ns * (w8 ? 11 : 13) / 10;  // fp16 takes more instructions to round to
   return (tiles * splits + cus - 1) / cus * (kchunk / kW4BigBK * slice + start) +
          (splits > 1 ? 3000 + (int64_t)splits * M * N / 500 : 0);
 }

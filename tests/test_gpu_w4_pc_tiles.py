@@ -121,3 +121,16 @@ def test_all_rounder_where_it_costs_less(m, n, k, gs, xdt, expect):
     assert ops.last_kernel().startswith(expect), ops.last_kernel()
     ref = og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, gs))
     assert_close(y.cpu(), ref, "bfloat16" if xdt == BF else "float16", what=expect)
+
+
+@pytest.mark.parametrize("m,n,k,gs,xdt,expect", [
+    (129, 8192, 2048, -1, BF, "w4_pc_kernel"), (129, 5120, 8192, 64, BF, "w4_big_kernel"), (70, 4096, 4096, -1, BF, "w4_pc_kernel"),
+    (173, 9608, 8192, -1, HF, "w4_big_kernel"), (256, 2048, 8192, -1, BF, "w4_pc_kernel")])
+def test_all_rounder_on_int8_weights_where_it_costs_less(m, n, k, gs, xdt, expect):
+    q = torch.randint(-128, 128, (n, k), generator=gen(m + k), dtype=torch.int8)
+    s = (torch.rand(n, L.num_groups(k, gs), generator=gen(1)) * 0.01).half()
+    x = x_act(m, k, xdt, seed=m)
+    y = ops.w8a16_linear(x.to(DEV), L.pack_w8(q, s, gs).to(DEV))
+    assert ops.last_kernel().startswith(expect), ops.last_kernel()
+    ref = x.double() @ (q.double() * s.double().repeat_interleave(k if gs < 0 else gs, 1)).t()
+    assert_close(y.cpu(), ref.float().numpy(), "bfloat16" if xdt == BF else "float16", what=ops.last_kernel())
