@@ -332,21 +332,38 @@ bool w4_pp_thirds(int64_t M, int64_t N, int64_t K) {
   const int64_t t = pp_tiles(M, N), cus = fg::device_cus();
   return M >= 256 && K >= 4096 && 4 * t > cus && 3 * t <= cus && ((M + 127) / 128) * ((N + 127) / 128) > cus;
 }
-// W8A16 has no producer / consumer kernel from 384 rows.  Below kPpMinTiles tiles from 256 rows the ping-pong kernel, its
-// K split up to four ways, beats the all-rounder down to 40 tiles (graph replays over four distinct weights, us, all-rounder
+// W8A16 has no producer / consumer kernel from 384 rows.  Below kPpMinTiles tiles from 256 rows the ping-pong kernel, its K
+// split up to four ways, beats the all-rounder down to 40 tiles (graph replays over four distinct weights, us, all-rounder
 // / ping-pong split 2 / split 4: qkv M = 512 65.7 / 66.3 / 51.2, M = 1024 86.9 / 77.8 / 90.9; o_proj M = 512 44.8 / 62.8 /
 // 46.0, M = 1024 67.1 / 70.4 / 61.3, M = 2048 96.4 / 93.8 / 114.2; down M = 512 95.4 / 163.8 / 98.9, M = 1024 159.0 / 174.9 /
-// 133.7, M = 2048 262.8 / 228.5 / 243.6).  As many splits of at least 512 columns as one round over the CUs holds (splits of
-// 1 / 2 / 3 / 4: 144 tiles, K=4096 96.4 / 129.1 / 114.4 / 137.6, K=14336 300.8 / 351.8 / 275.9 / 310.2; 96 tiles, K=4096
-// 95.1 / 71.5 / 92.9 / 91.7; 80 tiles, K=4096 94.7 / 65.0 / 58.5 / 80.4, K=14336 297 / 168 / 152 / 195; 72 tiles, K=4096
-// 94.1 / 63.5 / 53.6 / 76.2, K=8192 175.6 / 106.4 / 95.5 / 127.9).  Returns that number, 1 from kPpMinTiles tiles, 0 for the
-// all-rounder.
+// 133.7, M = 2048 262.8 / 228.5 / 243.6).  As many splits of at least 512 columns as one round over the CUs
+// holds (splits of 1 / 2 / 3 / 4: 144 tiles, K=4096 96.4 / 129.1 / 114.4 / 137.6; 96 tiles, K=4096 95.1 / 71.5 / 92.9 / 91.7;
+// 80 tiles, K=4096 94.7 / 65.0 / 58.5 / 80.4, K=14336 297 / 168 / 152 / 195; 72 tiles, K=4096 94.1 / 63.5 / 53.6 / 76.2,
+// K=8192 175.6 / 106.4 / 95.5 / 127.9).  That rule is behind in two places: 144 tiles, K=14336 300.8 / 351.8 / 275.9 / 310.2
+// (one split runs), and 32 tiles, K=14336, which the all-rounder keeps at 94.2, where six splits take 78.4.
+// From 40 to 64 tiles, where four splits fit a round, and K < 2048, where they are shorter than 512 columns, the cheapest of
+// 1..4: 1274 ns per 64-column slice, and for the partials 5 us, 0.12 us per MB, and 0.35 us per MB past 45 MB, which the
+// caches no longer hold (four splits / splits of at least 512 columns: 48 tiles, 600 x 4096, K=1024 28.4 / 31.7, K=1280 29.4
+// / 33.8, K=512 27.8 / 22.4; 64 tiles, K=1024 39.5 / 32.4, K=768 38.0 / 28.3).
+// Returns that number, 1 from kPpMinTiles tiles, 0 for the all-rounder.
 int w8_pp_split(int64_t M, int64_t N, int64_t K) {
   if (M < 256) return 0;
-  const int64_t t = pp_tiles(M, N);
+  const int64_t t = pp_tiles(M, N), cus = fg::device_cus();
   if (t >= kPpMinTiles) return 1;
   if (4 * t < kPpMinTiles) return 0;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({4, fg::device_cus() / t, K / 512}));
+  if (4 * t > cus || K >= 2048) return (int)std::max<int64_t>(1, std::min<int64_t>({4, cus / t, K / 512}));
+  int64_t best = -1;
+  int splits = 1;
+  for (int s = 1; s <= 4; ++s) {
+    const int64_t kb = s * M * N * 4 / 1000;
+    const int64_t cost = ((K + 63) / 64 + s - 1) / s * 1274 +
+                         (s > 1 ? 5000 + kb * 12 / 100 + std::max<int64_t>(0, kb - 45000) * 35 / 100 : 0);
+    if (best < 0 || cost < best) {
+      best = cost;
+      splits = s;
+    }
+  }
+  return splits;
 }
 
 // W4: whether the all-rounder is ahead of the producer / consumer kernel where both can run and the ping-pong kernel cannot.

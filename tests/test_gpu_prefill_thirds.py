@@ -47,3 +47,10 @@ def test_int8_weights(m, n, k, gs, xdt, split):
     ref = og.w8a16_gemm_ref(to_f32(x), og.pack_w8(q.numpy(), s.float().numpy(), gs))
     assert_close(y.cpu(), ref, "bfloat16" if xdt == BF else "float16", what=f"w8a16 m={m} n={n} k={k}")
     assert torch.equal(y, ops.w8a16_linear(x.to(DEV), p))
+
+
+@pytest.mark.parametrize("m,n,k,gs,xdt,split", [
+    (600, 4096, 1024, -1, BF, 4), (600, 4096, 512, 128, HF, 1), (1024, 4096, 1024, -1, BF, 2), (1024, 4096, 1984, 64, BF, 3),
+    (700, 3592, 1088, -1, HF, 4)])
+def test_int8_weights_of_40_to_64_tiles(m, n, k, gs, xdt, split):
+    test_int8_weights(m, n, k, gs, xdt, split)
