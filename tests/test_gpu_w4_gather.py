@@ -69,3 +69,40 @@ def test_the_gathers_label_ends_with_its_op():
     a = torch.ones(64, 256, dtype=torch.int8, device=DEV)
     ops.int8_gemm(a, None, a, None, out_dtype=torch.int32)
     assert "gather" not in ops.last_kernel(), ops.last_kernel()
+
+
+def _act_order(m, n, k, gs, xdt, seed):
+    q, s, z = w4_parts(n, k, gs, False, seed=seed)
+    g_idx = (torch.arange(k) // gs)[torch.randperm(k, generator=gen(seed))].to(torch.int32)
+    x = x_act(m, k, xdt, seed=seed + 1)
+    return q, s, z, g_idx, x, og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, gs, g_idx))
+
+
+# the kernels that read the permutation themselves, which a C caller may hand over with the sorted weight
+@pytest.mark.parametrize("m,n,k,gs,gemv,kernel", [
+    (1, 1024, 2048, 128, "split", "w4_gemv_split"), (4, 1024, 2048, 64, "tile", "w4_gemv_tile"), (2, 1024, 2048, 128, "wave", "w4_gemv"),
+    (1, 4096, 4096, 128, None, "w4_gemv"), (4, 4096, 4096, 128, None, "w4_"), (16, 1024, 2048, 128, None, "w4_mfma"),
+    (128, 520, 1024, 64, None, "w4_mfma"), (9, 520, 1056, 16, None, "w4_mfma"), (9, 520, 1056, 16, "unaligned", "w4_generic")])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_permutation_in_the_kernel(m, n, k, gs, gemv, kernel, xdt):
+    q, s, z, g_idx, x, ref = _act_order(m, n, k, gs, xdt, m + n)
+    packed = L.pack_w4(q, s, z, gs, g_idx=g_idx).to(DEV)
+    w, perm = L.cached_group_sort(packed, compute=True)
+    xd, y = x.to(DEV), torch.empty(m, n, dtype=xdt, device=DEV)
+    if gemv == "unaligned":
+        xd, gemv = torch.nn.functional.pad(xd, (1, 0))[:, 1:], None
+    config = None if gemv is None else {"impl": "gemv", "gemv_kernel": gemv}
+    ops._w4_call(xd, ops._W4Operands(w, perm=perm), None, y, ops._w4_config(config))
+    assert _lib.last_kernel().startswith(kernel), _lib.last_kernel()
+    assert_close(y.cpu(), ref, "bfloat16" if xdt == torch.bfloat16 else "float16", what=_lib.last_kernel())
+
+
+@pytest.mark.parametrize("m", [1, 16, 100])
+def test_act_order_weight_in_the_cdna4_layout(m):
+    """Its portable_row copy, sorted, serves it, the permutation read in the kernel."""
+    n, k = 1024, 2048
+    q, s, z, g_idx, x, ref = _act_order(m, n, k, 128, torch.bfloat16, m)
+    packed = L.pack_w4(q, s, z, 128, L.CDNA4_W4, g_idx=g_idx).to(DEV)
+    y = ops.w4a16_linear(x.to(DEV), packed)
+    assert "gather" not in ops.last_kernel()
+    assert_close(y.cpu(), ref, "bfloat16", what=f"cdna4 act-order {ops.last_kernel()}")

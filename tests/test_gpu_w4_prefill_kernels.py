@@ -2,11 +2,11 @@
 (forge/kernels/triton/gemm_w4_dequant.py:194-256 w4_dequant_matmul, gemm_w4a16.py:69-153): the ping-pong kernel
 (256 x 256 tiles, fg_w4_pp.hip), the producer / consumer kernel (256 x 128, fg_w4_pc.hip) and the all-rounder
 (fg_w4_big.hip).  Cases: the policy's choice from 256 rows (ping-pong once a problem has >= 160 tiles of 256 x 256,
-else producer / consumer) on Llama-3-8B shapes; each kernel forced (tile_n = 256 / 128 / 64) on ragged shapes (M and N
+or 65..85 of them and K >= 4096, else producer / consumer) on Llama-3-8B shapes; each kernel forced (tile_n = 256 / 128 / 64) on ragged shapes (M and N
 not multiples of the tile, one row, bias in x's dtype / fp32 / none, symmetric and asymmetric weights, one group and
 groups of 64 / 128, fp16 and bf16 x and scales) and with forced K splits; "dequant_gemm" (the reference's
-dequant_matmul) giving the same bits as "prefill"; act-order weights, fp32 scales and unaligned x leaving the fast
-kernels; graph replays; run-to-run reproducibility.
+dequant_matmul) giving the same bits as "prefill"; act-order weights behind the column gather, fp32 scales and unaligned x
+leaving the fast kernels; graph replays; run-to-run reproducibility.
 
 Bar: max|y - ref| / max|ref| <= 1e-2 of the fp32 oracle (oracle/gemm.py) plus the reference's compare() rule.
 """
@@ -86,7 +86,7 @@ def test_forced_k_splits(tile_n, split):
     assert torch.equal(y, ops.w4a16_linear(x, p, bd, config={"impl": "prefill", "tile_n": tile_n, "split_k": split}))
 
 
-def test_act_order_and_fp32_scales_leave_the_fast_kernels():
+def test_act_order_reaches_the_fast_kernels_behind_the_gather_and_fp32_scales_leave_them():
     n, k, m = 1024, 2048, 1024
     q, s, z = w4_parts(n, k, 128, False, seed=31)
     g_idx = torch.from_numpy(np.random.default_rng(32).permutation(k) // 128).int()
@@ -94,7 +94,7 @@ def test_act_order_and_fp32_scales_leave_the_fast_kernels():
     x = x_act(m, k, torch.bfloat16, seed=33)
     y = ops.w4a16_linear(x.to(DEV), p)
     kern = ops.last_kernel()
-    assert not kern.startswith(("w4_pp_kernel", "w4_pc_kernel")), kern  # the sorted weight comes with a column perm
+    assert kern.startswith("gather_columns + w4_pc_kernel"), kern  # the sorted weight, x gathered into its column order
     ref = og.w4a16_gemm_ref(to_f32(x), oracle_packed(q, s, z, 128, g_idx=g_idx))
     assert_close(y.cpu(), ref, "bfloat16", what="act-order m=1024")
     y, ref, kern, _ = _run(1024, 4096, 4096, torch.bfloat16, None, seed=34, sdt=torch.float32)

@@ -1,8 +1,7 @@
 """GPU parity of the W8A16 prefill kernels (the reference's w8a16_linear at large M, forge/kernels/ops_gemm.py:320-346
 -> gemm_wq.py:138-205 with bits=8): the ping-pong kernel's int8 form (256 x 256 tiles, fg_w4_pp.hip) and the
 all-rounder's (fg_w4_big.hip).  Cases: the policy's choice from 256 rows (ping-pong once a problem has >= 160 tiles of
-256 x 256; below that ping-pong with K split 2 or 4 ways when that reaches 160 tiles x splits, else the all-rounder) on
-Llama-3-8B shapes; each kernel forced (tile_n = 256 / 64) on ragged shapes (one
+256 x 256; from 40 tiles ping-pong with K split up to four ways, below that the all-rounder) on Llama-3-8B shapes; each kernel forced (tile_n = 256 / 64) on ragged shapes (one
 row, M and N not multiples of the tile, bias in x's dtype / fp32 / none, per-channel and grouped fp16 / bf16 scales,
 fp16 and bf16 x) and with forced K splits; "dequant_gemm" giving the same bits as "prefill"; fp32 scales and unaligned
 x leaving the ping-pong kernel; graph replays; run-to-run reproducibility.

@@ -1,8 +1,9 @@
 """GPU parity of the skinny W8A8 kernel (fg_w8_skinny.hip, M <= 64, register-resident split-K): INT8 accumulator and
 fp32 / bf16 / fp16 epilogues bit-exact against the CPU oracle (the int32 partials of the K slices sum exactly), FP8
 within the north-star bar, as is the 64-row kernel on the same inputs; forced with tile_m=16, and the policy's own choice
-(the skinny kernel for M <= 16 at K >= 16384 and for M <= 32 where the ring's 64 x 32 tiles would not cover the CUs,
-the ring kernel for the other aligned shapes) held to the same bar."""
+(the skinny kernel for M <= 16 at K >= 16384, and where the ring's 64 x 32 tiles would leave CUs idle: up to 8 rows if
+they cover them once, 16 below that, 32 while they cover half; the ring kernel for the other aligned shapes) held to the
+same bar."""
 from __future__ import annotations
 
 import numpy as np

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from forge_amd import ops_gemm as ops
-from tests._util import gen
+from tests._util import assert_close, gen
 from tests.test_isa_waits import _check_ring_loops, kernels  # noqa: F401  (fixture)
 
 DEV = "cuda"
@@ -39,7 +39,7 @@ def test_fp8_tiles(m, n, tile, k):
     b = torch.randn(n, generator=gen(3)).to(torch.bfloat16).to(DEV)
     for odt, bias in ((torch.bfloat16, b), (torch.float32, None)):
         y = ops.fp8_linear(a, w, sw, bias, x_scale=sx, out_dtype=odt)
-        assert tile in ops.last_kernel() or k % 256 == 0, ops.last_kernel()
+        assert tile in ops.last_kernel(), ops.last_kernel()
         ref = ops.fp8_linear(_off(a), _off(w), sw, bias, x_scale=sx, out_dtype=odt)
         assert ops.last_kernel().startswith("mm_kernel") and torch.equal(y, ref)
 
@@ -70,11 +70,30 @@ def test_fp8_block_scale_tiles(m, n, tile, k, per_row_weight):
 def test_int8_tiles(m, n, tile, k):
     a, w = _codes(m, k, torch.int8, m + k), _codes(n, k, torch.int8, n + k)
     acc = ops.int8_gemm(a, None, w, None, out_dtype=torch.int32)
-    assert tile in ops.last_kernel() or k % 256 == 0, ops.last_kernel()
+    assert tile in ops.last_kernel(), ops.last_kernel()
     assert torch.equal(acc.double(), a.double() @ w.double().t())
     sx, sw = torch.rand(m, generator=gen(1)).to(DEV), torch.rand(n, generator=gen(2)).to(DEV)
     y = ops.int8_gemm(a, sx, w, sw, out_dtype=torch.float16)
     assert torch.equal(y, ((acc.float() * sx.view(-1, 1)) * sw).half())
+
+
+# K of whole 256-column steps: the skinny kernel's lines on both sides (256 CUs: 8192 channels are one 64 x 32 tile each)
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,expect", [
+    (8, 8192, 256, "w8_skinny"), (8, 8224, 256, "mm_ring"), (9, 8192, 1024, "mm_ring"), (9, 8160, 1024, "w8_skinny"),
+    (16, 8160, 256, "w8_skinny"), (17, 8160, 256, "mm_ring"), (17, 4096, 1024, "w8_skinny"), (32, 4096, 256, "w8_skinny"),
+    (32, 4128, 256, "mm_ring"), (33, 4096, 1024, "mm_ring"), (16, 8224, 16384, "w8_skinny"), (17, 8224, 16384, "mm_ring")])
+def test_skinny_kernel_lines(m, n, k, expect):
+    a, w = _codes(m, k, torch.int8, m + k), _codes(n, k, torch.int8, n + k)
+    acc = ops.int8_gemm(a, None, w, None, out_dtype=torch.int32)
+    assert ops.last_kernel().startswith(expect), ops.last_kernel()
+    assert torch.equal(acc.double(), a.double() @ w.double().t())
+    a, w = _codes(m, k, torch.float8_e4m3fn, m + k), _codes(n, k, torch.float8_e4m3fn, n + k)
+    sx, sw = torch.rand(m, generator=gen(1)).to(DEV), torch.rand(n, generator=gen(2)).to(DEV)
+    y = ops.fp8_linear(a, w, sw, x_scale=sx, out_dtype=torch.float32)
+    assert ops.last_kernel().startswith(expect), ops.last_kernel()
+    ref = (a.double() @ w.double().t()) * sx.double().view(-1, 1) * sw.double()
+    assert_close(y.cpu(), ref.cpu().float().numpy(), "float32", what=ops.last_kernel())
 
 
 @pytest.mark.gpu
