@@ -327,7 +327,9 @@ int64_t pp_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) /
 // with more than a quarter and at most a third of the CUs in tiles the three splits fit one round, while the other kernel's
 // 256-row tiles fill only half to two thirds of one and its 128-row tiles exceed it.  Below K = 4096 the partials cost what
 // the shorter slices save.  (us, producer-consumer / ping-pong, 80 tiles, M=1111, N=4096: K=4096 65.7 / 57.1, K=14336 184.6 /
-// 146.4; outside, M=512: 48 tiles, N=6144, K=4096 50.4 / 53.0, 32 tiles, N=4096, K=14336 75.0 / 87.4.)
+// 146.4; outside, M=512: 48 tiles, N=6144, K=4096 50.4 / 53.0, 32 tiles, N=4096, K=14336 75.0 / 87.4.  66, 72, 78 and 85 tiles
+// over K = 4096..14336 measured no slower than the producer / consumer kernel.  Left on the other side of the line: 48 tiles
+// at K=14336, 112.5 against 103.3 / 100.2 with four / five splits.)
 bool w4_pp_thirds(int64_t M, int64_t N, int64_t K) {
   const int64_t t = pp_tiles(M, N), cus = fg::device_cus();
   return M >= 256 && K >= 4096 && 4 * t > cus && 3 * t <= cus && ((M + 127) / 128) * ((N + 127) / 128) > cus;

@@ -1,5 +1,5 @@
-// Shared pieces of the W8A8 GEMM kernels (fg_mm.hip: 128-row tiles and the K-blocked FP8 mode; fg_mm_big.hip:
-// 256 x 256 tiles fed by direct global->LDS loads): MFMA wrappers and epilogues.
+// Shared pieces of the W8A8 GEMM kernels (fg_mm_big.hip: tiles fed by direct global->LDS loads, K-blocked FP8 scales among
+// them; fg_mm.hip: register-staged tiles for operands those cannot read): MFMA wrappers and epilogues.
 //
 // MFMA register layouts (16x16 tiles): operand lane l holds row/column (l % 16) and the K sub-slice (l / 16); the
 // result lane l holds column (l % 16), rows 4*(l/16) + i, i = 0..3.  A and B use the same K sub-slice mapping, so the

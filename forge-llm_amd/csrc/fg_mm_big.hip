@@ -15,11 +15,13 @@
 // to a per-wavefront LDS buffer, then stored as 16-byte row segments (row scales read once per row, column scales and
 // bias once per column).  32-bit outputs are stored element by element.
 //
-// mm_ring_kernel (below) is the same design for small M: 64- or 128-row tiles, an S-stage ring with S - 1 slices in
-// flight.
+// mm_ring_kernel (below) is the same design with smaller tiles (64 x 32 .. 256 x 128) and an S-stage ring with S - 1 slices
+// in flight; mm_blk_kernel is its form for FP8 with K-blocked scales, which has a 256 x 256 tile too.
 //
-// Requirements (checked by mm_big_ok, for both kernels): K % 128 == 0, 16-byte aligned A and B with lda, ldb multiples
-// of 16.  Rows of A or B past M or N are read from row M-1 or N-1 (valid memory) and their results are not stored.
+// Requirements (mm_tail_ok): K % 16 == 0, 16-byte aligned A and B with lda, ldb multiples of 16; a K that ends inside a
+// 128-byte slice takes the TAIL instances, which read zeros past it.  A tile that a configuration names also needs
+// K % 128 == 0 (mm_big_ok).  Rows of A or B past M or N are read from row M-1 or N-1 (valid memory) and their results are
+// not stored.
 #include "fg_mm.h"
 
 namespace fg {

@@ -19,7 +19,7 @@
 //     zero words of slice t + 3 -> the staging areas of stage t % 3 (read by the producers in t - 1); wait until
 //     slice t + 1's staging loads have landed, dequantise slice t + 1 into stage (t + 1) % 3's weight rows (consumed
 //     in t - 2); wait until slice t + 1's x rows have landed; barrier.
-//   consumers, iteration t: 64 MFMAs per k-step pair over stage t % 3; barrier.
+//   consumers, iteration t: BM / 4 MFMAs (64 at 256 rows) over the two k-steps of stage t % 3; barrier.
 // Every producer issues the same loads in the same order each iteration (slices past the end re-read the last one,
 // into areas no one reads again), so `s_waitcnt vmcnt(N)` with a constant N is exactly "these loads have landed"
 // (loads complete in issue order); the direct-to-LDS loads are invisible to the compiler's wait analysis, so those

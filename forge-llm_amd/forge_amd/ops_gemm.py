@@ -368,8 +368,6 @@ SZ8_ROWS = 2
 _SZ8_KEY = "hip.sz8"  # p.meta entry: (tensor stamp, scales8, zeros8)
 
 
-
-
 def prepare_w4_sz8(packed: PackedW4) -> bool:
     """Keep ``packed``'s scales and zero words re-blocked by 8 channels (``layouts.sz8_blocks``) in ``packed.meta``
     for the 1..2-row decode GEMV; True when made (a portable_row weight on the GPU with N % 8 == 0, K % 32 == 0, a
@@ -529,10 +527,13 @@ def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = 
     """``y = x @ dequant(W)^T (+ bias)`` for bf16 / fp16 ``x [..., K]`` on a gfx950 GPU; returns ``x.dtype``.
 
     The C library picks the kernel per shape (``config={"impl": "gemv" | "mfma" | "prefill" | "generic", ...}`` or
-    ``FORGE_W4_IMPL`` overrides it): split-K register GEMV for 1-2 rows (and small weights at 3-4), the skinny MFMA
-    kernel up to 32 rows, dequantise-to-LDS MFMA tiles beyond, a per-element kernel for irregular act order or
-    unaligned weights.  A weight in the ``cdna4_mfma`` layout (``prepare_w4(p, CDNA4_W4)``) runs its own MFMA kernels
-    for 1..64 rows (a register ring, or an LDS ring with a K-split reduce for 33..64 rows and long K) and a
+    ``FORGE_W4_IMPL`` overrides it): split-K register GEMV for 1-2 rows (and small weights at 3-4), the LDS-ring kernel
+    for 17..64 rows and fewer over wide or long weights, the skinny MFMA kernel for other few rows, dequantise-to-LDS
+    MFMA tiles beyond and for groups those do not take, a per-element kernel for irregular act order or unaligned
+    weights.  A regular act-order weight has x gathered into its column order first and then runs as a plain one (in
+    the ``cdna4_mfma`` layout the kernel reads the permutation).  The copies that ``KernelW4A16Linear.prepare`` keeps
+    serve 1..2 and 3..64 rows.  A weight in the ``cdna4_mfma`` layout (``prepare_w4(p, CDNA4_W4)``) runs its own MFMA
+    kernels for 1..64 rows (a register ring, or an LDS ring with a K-split reduce for 33..64 rows and long K) and a
     portable_row copy beyond.  Every kernel reduces in a fixed order, so results are run-to-run reproducible whatever
     ``deterministic`` says.
     """

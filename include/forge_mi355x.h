@@ -38,9 +38,12 @@ enum { FG_W4_AUTO = 0, FG_W4_GEMV = 1, FG_W4_MFMA = 2, FG_W4_GENERIC = 3, FG_W4_
 /* FG_W4_PREFILL: the prefill kernels, x straight to LDS, weights dequantised tile by tile and fed to bf16 / fp16 MFMA
    (large M x N; needs K % 64 == 0, group % 32 == 0 or one group, aligned x / qweight, no act-order perm): from 256
    rows the ping-pong kernel (256 x 256 tiles, two teams of wavefronts alternating MFMA and dequantisation; group %
-   64 == 0, N % 8 == 0, 16-bit scales) once the problem has >= 160 such tiles, else the producer / consumer kernel
-   (256 x 128 tiles), else the all-rounder (128 / 256 x 256 tiles, split-K).  fg_w4_config.tile_n = 256 / 128 / 64
-   forces one of them where its conditions hold.
+   64 == 0, N % 8 == 0, 16-bit scales) once the problem has >= 160 such tiles, and with its K split three ways over
+   K >= 4096 where 65..85 of them fit one round; else the producer / consumer kernel (64 / 128 / 256 x 128 tiles,
+   split-K; N % 8 == 0, 16-bit scales) or the all-rounder (64 / 128 / 256 x 256 tiles, split-K): below 256 rows, and
+   with groups that are no multiple of 64, whichever of the two costs less, otherwise the first where its conditions
+   hold.  fg_w4_config.tile_n = 256 / 128 / 64 forces one of them where its conditions hold.  The automatic choice
+   also gives the producer / consumer kernel a K with K % 64 == 32.
    FG_W4_DEQUANT_GEMM: the reference's dequant_matmul route (forge/kernels/triton/gemm_w4_dequant.py:194-256,
    dequantise then a library GEMM); here a name for FG_W4_PREFILL, whose kernels fuse the two steps. */
 
@@ -185,9 +188,10 @@ int fg_w4_dequant(const int32_t* qweight, int64_t ldq, const void* scales, int s
  *   scales   fp16|bf16|fp32 [G, N] (row stride lds);  group_size <= 0: one group per row (per-channel)
  *   cfg      NULL (policy: decode GEMV for 1..2 rows and 3..4 over N <= 8192 and K < 8192; LDS-ring kernel for
  *            17..64 rows and for 3..16 over N >= 16384 or K >= 8192; skinny kernel for the other rows up to 64;
- *            then the prefill kernels: from 256 rows the ping-pong kernel once the problem has >= 160 tiles of
- *            256 x 256, below that the ping-pong kernel with K split 2 or 4 ways when tiles x splits reaches 160,
- *            else the all-rounder) or impl FG_W4_GEMV (split-K decode GEMV, M <= 4), FG_W4_MFMA (skinny
+ *            then the prefill kernels: from 256 rows the ping-pong kernel once the problem has >= 40 tiles of
+ *            256 x 256 (below 160 with K split up to four ways); for 65..128 rows, up to 256 while its tiles fit one
+ *            round, and wherever K % 64 == 32, the producer / consumer kernel, or the all-rounder where that costs
+ *            less; else the all-rounder) or impl FG_W4_GEMV (split-K decode GEMV, M <= 4), FG_W4_MFMA (skinny
  *            kernel, M <= 64), FG_W4_PREFILL / FG_W4_DEQUANT_GEMM (the prefill kernels; tile_n = 256 / 64 forces
  *            the ping-pong / all-round kernel), FG_W4_GENERIC (any shape); split_k for the prefill kernels
  *   workspace  fg_w8a16_workspace_bytes bytes (split-K partials of the prefill kernels or, under the policy, of the
