@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(256) quant_fp8_rowwise_kernel(const void* __re
 // in 1 x 128 blocks (a workgroup per block).  Here a row is read once, 8 values per lane and 16-byte load, and stays in
 // registers; the absolute maximum is a packed 16-bit integer maximum of the bit patterns (their order is the order of
 // magnitudes, a NaN above every number); and the quotient by the row's scale is exact with five multiply-adds.  The same
-// four calls: 4.8, 18.9 (5.3 TB/s), 10.0 and 7.3 us (kernel trace; the third with the norm's sum in the element-wise
+// four calls: 4.8, 18.9 (5.3 TB/s), 8.3 and 7.3 us (kernel trace; the third with the norm's sum in the element-wise
 // kernel's order, which costs 0.5 us of it: row_sum_sq).
 
 // RN(a / b) from y = RN(1 / b): q0 = a y is within two units in the last place, one correction brings it within one,
