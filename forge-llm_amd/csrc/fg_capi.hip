@@ -835,7 +835,7 @@ static bool w8a16_ring_rows(int64_t M, int64_t N, int64_t K) {
 
 // Whether a W8A16 call that neither the GEMV, the ring nor the skinny kernel takes may go to the producer / consumer kernel
 // (64- and 128-row tiles): whenever K ends inside a 64-column slice (the other kernels cannot read it and the generic one
-// would serve: K=4128, N=4096, groups of 32, 6 / 64 / 512 rows 101 / 665 / 4439 us against 15 / 20 / 41), for 65..128 rows,
+// would serve: K=4128, N=4096, groups of 32, 6 / 64 / 512 rows 101 / 665 / 4439 us against 16 / 20 / 48), for 65..128 rows,
 // and up to 256 while its 128-row tiles fit one round (all-rounder / producer-consumer, us: K=4096, N=6144 M=80 30.5 / 21.3,
 // M=256 40.4 / 36.2; N=28672 M=128 71.9 / 56.9, M=200 -- two rounds -- 100.5 / 107.8; K=14336, N=4096 M=128 46.3 / 34.6,
 // M=256 62.5 / 55.9; from 384 rows the ping-pong kernel is ahead).  Up to 64 rows (groups that are no multiple of 128) it

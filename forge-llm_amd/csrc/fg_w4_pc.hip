@@ -1,5 +1,9 @@
 // W4A16 prefill with producer and consumer wavefronts: y[M,N] = x[M,K] @ dequant(W)[N,K]^T (+bias).  W8A16 (int8
-// weights) takes the same kernel with tiles of 64 and 128 rows: twice the staging bytes, no zero words.
+// weights) takes the same kernel with tiles of 64 and 128 rows: twice the staging bytes, no zero words.  Its instances for a
+// K that ends inside a slice (pc_exact) keep the weights exact: the integers are the MFMA operands and each 32-column
+// product takes its fp32 scale as it joins the sum, since the kernel that reads such a K otherwise multiplies in fp32 (error
+// against 64 bits, bf16 x, K=4128: 1.66e-3 in both, 2.32e-3 with the scaled weight rounded to bf16, which took 39 us at 512
+// rows of N=4096, groups of 32, against 48).
 //
 // A workgroup owns a BM x 128 output tile (BM = 256, 128 or 64; below 256 rows) and walks K in 64-column slices through
 // a three-stage LDS ring.  Its eight wavefronts split the work by role, one of each role per SIMD (wavefronts 0-3 on SIMDs 0-3, 4-7 likewise):
@@ -28,7 +32,8 @@
 // LDS per stage: x BM rows x 128 B (16-byte unit c of row r at c ^ (r & 7): conflict-free fragment reads), weight
 // rows 128 x 128 B (same swizzle), packed-weight staging 4 KiB (producer p's lane l at p * 1024 + 16 l), scale and
 // zero staging 1 KiB (producer p: 32 fp16 scales at p * 256, its 4 zero words at p * 256 + 64, and 128 bytes further the
-// same of the group of the slice's second 32 columns).  Three stages: 162816 bytes at BM = 256, 113664 and 89088 below.
+// same of the group of the slice's second 32 columns); with pc_exact the fp32 scales of the two halves, 1 KiB, which the
+// consumers read beside the weight rows.  Three stages: 162816 bytes at BM = 256, 113664 and 89088 below.
 //
 // Split-K (gridDim.y > 1): each split covers `kchunk` columns and writes fp32 partials [S, M, N] to the caller's
 // workspace; w4_splitk_reduce_kernel (fg_w4_mfma.hip) sums them in a fixed order and adds the bias.
@@ -56,9 +61,13 @@ constexpr int kPcWBytes = kPcBN * kPcRow;                      // dequantised we
 constexpr int pc_q_bytes(int wb) { return kPcBN * kPcBK * wb / 8; }  // packed weights of the slice (WB bits each)
 constexpr int kPcSBytes = 4 * 256;                             // scales and zero words
 constexpr int pc_x_bytes(int bm) { return bm * kPcRow; }       // x rows
-constexpr int pc_stage(int bm, int wb) { return pc_x_bytes(bm) + kPcWBytes + pc_q_bytes(wb) + kPcSBytes; }
-constexpr int pc_lds(int bm, int wb) { return 3 * pc_stage(bm, wb); }
-static_assert(pc_lds(256, 4) <= 160 * 1024 && pc_lds(128, 8) <= 160 * 1024, "the ring exceeds the LDS");
+constexpr bool pc_exact(int wb, bool tail) { return wb == 8 && tail; }
+constexpr int kPcFBytes = 2 * kPcBN * 4;                       // fp32 scales of the slice's two 32-column halves (pc_exact)
+constexpr int pc_stage(int bm, int wb, bool exact) {
+  return pc_x_bytes(bm) + kPcWBytes + pc_q_bytes(wb) + kPcSBytes + (exact ? kPcFBytes : 0);
+}
+constexpr int pc_lds(int bm, int wb, bool exact) { return 3 * pc_stage(bm, wb, exact); }
+static_assert(pc_lds(256, 4, false) <= 160 * 1024 && pc_lds(128, 8, true) <= 160 * 1024, "the ring exceeds the LDS");
 // direct-to-LDS loads one producer issues per slice: x rows, packed weights, scales + zero words
 constexpr int pc_xi(int bm) { return pc_x_bytes(bm) / 1024 / 4; }
 constexpr int pc_qi(int wb) { return pc_q_bytes(wb) / 1024 / 4; }
@@ -117,8 +126,10 @@ __device__ __forceinline__ uint4 pc_frag(const uint8_t* rp, int r16, int lane, i
 
 template <int BM, bool XBF16, int WB, bool TAIL>
 __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
-  constexpr int kPcBM = BM, kPcXBytes = pc_x_bytes(BM), kPcStage = pc_stage(BM, WB), kPcXI = pc_xi(BM);
+  constexpr bool kExact = pc_exact(WB, TAIL);
+  constexpr int kPcBM = BM, kPcXBytes = pc_x_bytes(BM), kPcStage = pc_stage(BM, WB, kExact), kPcXI = pc_xi(BM);
   constexpr int kPcQI = pc_qi(WB), kPcQBytes = pc_q_bytes(WB);
+  constexpr int kF = kPcWBytes + kPcQBytes + kPcSBytes;  // offset of a stage's fp32 scales from its weight rows
   constexpr int TM = BM / 32;  // 16-row blocks of a consumer
   extern __shared__ __align__(16) uint8_t smem[];
   const int ntm = (a.M + kPcBM - 1) / kPcBM, ntn = (a.N + kPcBN - 1) / kPcBN;
@@ -137,6 +148,7 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
     // (lane / 16) .. + 3 of channel lane % 16): the other order measured 3-5% slower at row counts that leave most of the
     // last tile empty (K=14336, N=4096, M=300 62.1 -> 64.4).
     constexpr bool kWFirst = BM < 256;
+    static_assert(kWFirst || !kExact, "the scales of a lane's results are those of four channels in a row");
     const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15;
     f32x4_pc_t acc[TM][4];
 #pragma unroll
@@ -149,32 +161,52 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
     // eight MFMAs of slice t (whose fragments are already in registers) run, so a consumer -- the only MFMA issuer of
     // its SIMD -- does not sit out the LDS latency at the top of every slice.
     uint4 fa0[TM], fb0[4], fa1[TM], fb1[4];
-    auto read_ks = [&](const uint8_t* st, int s, uint4 (&fa)[TM], uint4 (&fb)[4]) __attribute__((always_inline)) {
+    f32x4_pc_t sc0[4], sc1[4];  // pc_exact: scales of the lane's four channels of each column block
+    auto read_ks = [&](const uint8_t* st, int s, uint4 (&fa)[TM], uint4 (&fb)[4], f32x4_pc_t (&sc)[4])
+                       __attribute__((always_inline)) {
       const uint8_t* sA = st + (wm * (BM / 2) + r16) * kPcRow;
       const uint8_t* sB = st + kPcXBytes + (wn * 64 + r16) * kPcRow;
 #pragma unroll
       for (int j = 0; j < 4; ++j) fb[j] = pc_frag(sB + j * 16 * kPcRow, r16, lane, s);
 #pragma unroll
       for (int i = 0; i < TM; ++i) fa[i] = pc_frag(sA + i * 16 * kPcRow, r16, lane, s);
+      if constexpr (kExact) {
+        const float* f = reinterpret_cast<const float*>(st + kPcXBytes + kF) + s * kPcBN + wn * 64 + 4 * (lane >> 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sc[j] = *reinterpret_cast<const f32x4_pc_t*>(f + j * 16);
+      }
     };
-    auto mfma_rows = [&](int i0, int i1, const uint4 (&fa)[TM], const uint4 (&fb)[4]) __attribute__((always_inline)) {
+    auto mfma_rows = [&](int i0, int i1, const uint4 (&fa)[TM], const uint4 (&fb)[4], const f32x4_pc_t (&sc)[4])
+                         __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = i0; i < i1; ++i)
+      for (int i = i0; i < i1; ++i) {
+        if constexpr (kExact) {
+          f32x4_pc_t part[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = kWFirst ? pc_mfma<XBF16>(fb[j], fa[i], acc[i][j]) : pc_mfma<XBF16>(fa[i], fb[j], acc[i][j]);
+          for (int j = 0; j < 4; ++j) part[j] = pc_mfma<XBF16>(fb[j], fa[i], f32x4_pc_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[j][e], sc[j][e], acc[i][j][e]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = kWFirst ? pc_mfma<XBF16>(fb[j], fa[i], acc[i][j]) : pc_mfma<XBF16>(fa[i], fb[j], acc[i][j]);
+        }
+      }
     };
     const uint8_t* st = smem;
-    read_ks(st, 0, fa0, fb0);
+    read_ks(st, 0, fa0, fb0, sc0);
     for (int t = 0; t < nk; ++t) {
-      read_ks(st, 1, fa1, fb1);
-      mfma_rows(0, TM, fa0, fb0);
-      mfma_rows(0, TM - 2, fa1, fb1);
+      read_ks(st, 1, fa1, fb1, sc1);
+      mfma_rows(0, TM, fa0, fb0, sc0);
+      mfma_rows(0, TM - 2, fa1, fb1, sc1);
       // this stage's fragments are in registers before the barrier lets the producers refill it
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       st = st == smem + 2 * kPcStage ? smem : st + kPcStage;
-      read_ks(st, 0, fa0, fb0);  // slice t + 1 (past the last slice: a stage no one writes any more, unused)
+      read_ks(st, 0, fa0, fb0, sc0);  // slice t + 1 (past the last slice: a stage no one writes any more, unused)
       __builtin_amdgcn_sched_barrier(0);
-      mfma_rows(TM - 2, TM, fa1, fb1);
+      mfma_rows(TM - 2, TM, fa1, fb1, sc1);
       __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_barrier" ::: "memory");  // the producers' last loads have drained: the ring is free
@@ -320,17 +352,18 @@ __device__ __forceinline__ void w4_pc_body(const PcArgs& a) {
     const uint32_t zw = (*reinterpret_cast<const uint32_t*>(sz + 64 + ((lane >> 1) >> 3) * 4) & zsel) |
                         (0x88888888u & ~zsel);  // symmetric: zero-point 8
     const float sc = a.sbf16 ? bf16_bits_to_f32(sraw) : f16_bits_to_f32((uint16_t)sraw);
-    if constexpr (WB == 8) {  // u = q ^ 0x80 = q + 128: q * s = u * s - 128 s, exact in fp32, rounded once
+    if constexpr (WB == 8) {  // u = q ^ 0x80 = q + 128: q * s = u * s - 128 s, exact in fp32, rounded once (pc_exact: s = 1)
       const uint4 qv2 = *reinterpret_cast<const uint4*>(q + (p * kPcQI + 1) * 1024 + lane * 16);
       const uint32_t wd[8] = {qv.x, qv.y, qv.z, qv.w, qv2.x, qv2.y, qv2.z, qv2.w};
-      const float c128 = -128.f * sc;
+      if constexpr (kExact) *reinterpret_cast<float*>(w + kF + (wh * kPcBN + wr) * 4) = sc;
+      const float ws = kExact ? 1.f : sc, c128 = -128.f * ws;
       uint8_t* row = w + wr * kPcRow;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float d[8];
 #pragma unroll
         for (int b = 0; b < 8; ++b)
-          d[b] = __builtin_fmaf((float)(((wd[2 * i + b / 4] ^ 0x80808080u) >> (8 * (b % 4))) & 0xFFu), sc, c128);
+          d[b] = __builtin_fmaf((float)(((wd[2 * i + b / 4] ^ 0x80808080u) >> (8 * (b % 4))) & 0xFFu), ws, c128);
         *reinterpret_cast<uint4*>(row + (((4 * wh + i) ^ (wr & 7)) * 16)) =
             make_uint4(pc_pack<XBF16>(d[0], d[1]), pc_pack<XBF16>(d[2], d[3]), pc_pack<XBF16>(d[4], d[5]),
                        pc_pack<XBF16>(d[6], d[7]));
@@ -514,7 +547,7 @@ static hipError_t launch_pc(const void* x, int64_t ldx, bool xbf16, const void* 
     constexpr int BM = decltype(bm_tag)::value;
     auto kern = K % kPcBK ? (xbf16 ? w4_pc_kernel<BM, true, WB, true> : w4_pc_kernel<BM, false, WB, true>)
                           : (xbf16 ? w4_pc_kernel<BM, true, WB, false> : w4_pc_kernel<BM, false, WB, false>);
-    constexpr int lds_bytes = pc_lds(BM, WB);
+    const int lds_bytes = pc_lds(BM, WB, pc_exact(WB, K % kPcBK != 0));
     const hipError_t err =
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (err != hipSuccess) return err;

@@ -134,3 +134,17 @@ def test_all_rounder_on_int8_weights_where_it_costs_less(m, n, k, gs, xdt, expec
     assert ops.last_kernel().startswith(expect), ops.last_kernel()
     ref = x.double() @ (q.double() * s.double().repeat_interleave(k if gs < 0 else gs, 1)).t()
     assert_close(y.cpu(), ref.float().numpy(), "bfloat16" if xdt == BF else "float16", what=ops.last_kernel())
+
+
+@pytest.mark.parametrize("xdt", [BF, HF])
+@pytest.mark.parametrize("m,n,k,gs", [(6, 1032, 4128, 32), (40, 264, 1056, 96), (100, 1024, 4128, -1), (513, 520, 1376, 32)])
+def test_int8_weights_stay_exact_before_a_k_tail(m, n, k, gs, xdt):
+    """No weight is rounded to 16 bits: the distance to the 64-bit product is that of its rounding to x's type, and the
+    fp32 sum's, K terms of 2^-24 at most, here within a hundredth of the former."""
+    q = torch.randint(-128, 128, (n, k), generator=gen(m + k), dtype=torch.int8)
+    s = (torch.rand(n, L.num_groups(k, gs), generator=gen(1)) * 0.002 + 0.0002).half()
+    x = x_act(m, k, xdt, seed=m)
+    y = ops.w8a16_linear(x.to(DEV), L.pack_w8(q, s, gs).to(DEV)).cpu().double()
+    assert ops.last_kernel().startswith("w4_pc_kernel<") and ",w8>" in ops.last_kernel(), ops.last_kernel()
+    ref = x.double() @ (q.double() * s.double().repeat_interleave(k if gs < 0 else gs, 1)).t()
+    assert (y - ref).norm() <= 1.01 * (ref.to(xdt).double() - ref).norm()
