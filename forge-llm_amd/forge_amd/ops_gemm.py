@@ -553,9 +553,10 @@ def w4a16_linear(x: torch.Tensor, packed: PackedW4, bias: torch.Tensor | None = 
             _w4_dispatch(x2, packed, b, y, config)
         else:
             ops_, cfg = _w4_operands(packed, x2), _w4_config(config)
-            # regular act order: x in the sorted weight's column order, then any kernel.  A configuration meets x as it
-            # lies where x is unaligned: the gather's aligned copy would pass what the kernel it names refuses
-            if ops_.perm is not None and (cfg is None or _x_aligned(x2)):
+            # regular act order: x in the sorted weight's column order, then any kernel.  Unaligned rows are read as they
+            # lie: the gather's aligned copy would pass what a named kernel refuses, and reach kernels that round the
+            # weights to 16 bits where the kernels for such rows keep them in 32
+            if ops_.perm is not None and _x_aligned(x2):
                 _w4_dispatch(_gather_columns(x2, ops_.perm), ops_.weight, b, y, config)
             else:
                 _w4_call(x2, ops_, b, y, cfg)

@@ -61,6 +61,20 @@ def test_a_forced_kernel_still_refuses_unaligned_rows():
     assert_close(y.cpu(), ref, "bfloat16", what="act-order, unaligned x")
 
 
+@pytest.mark.parametrize("m", [2, 9, 100])
+def test_unaligned_rows_keep_fp32_weights(m):
+    """The kernels for rows that are not 16-byte aligned multiply dequantised weights in fp32, with act order as without:
+    the distance to the 64-bit product is that of its rounding to bf16 (and a hundredth for the fp32 sum)."""
+    n, k = 520, 1024
+    q, s, z = w4_parts(n, k, 128, False, seed=1)
+    g_idx = (torch.arange(k) // 128)[torch.randperm(k, generator=gen(2))].to(torch.int32)
+    x = x_act(m, k + 1, torch.bfloat16, seed=3)[:, 1:]
+    y = ops.w4a16_linear(torch.nn.functional.pad(x, (1, 0)).to(DEV)[:, 1:], L.pack_w4(q, s, z, 128, g_idx=g_idx).to(DEV))
+    w = (q.double() - z.double()[:, g_idx.long()]) * s.double()[:, g_idx.long()]
+    ref = x.double() @ w.t()
+    assert (y.cpu().double() - ref).norm() <= 1.01 * (ref.bfloat16().double() - ref).norm(), ops.last_kernel()
+
+
 def test_the_gathers_label_ends_with_its_op():
     """A gather that no product followed (a failed allocation in between) does not name the next op's kernel."""
     x = x_act(20, 512, torch.bfloat16, seed=1).to(DEV)
