@@ -67,6 +67,7 @@ class _Thread(threading.local):
 
 
 _THREAD = _Thread()
+_gathers = False  # whether any op ever did: a thread-local store costs every op 0.1 us
 
 
 # ================================================================================================ switches
@@ -74,10 +75,11 @@ def _env_reader(name: str) -> Callable[[], str]:
     """A function that reads environment variable ``name`` ("" when unset) as it is now.  Every op asks for several:
     ``os.environ.get`` encodes the name and decodes the value each time (0.8 us), the mapping behind it holds both as
     bytes."""
-    key = os.fsencode(name)
+    env, data, key = os.environ, getattr(os.environ, "_data", None), os.fsencode(name)
+    if not isinstance(data, dict):
+        return lambda: os.environ.get(name, "")
     def read() -> str:
-        data = getattr(os.environ, "_data", None)  # looked up each time: a program may put another mapping in its place
-        if type(data) is not dict:
+        if os.environ is not env:  # a program put another mapping in its place
             return os.environ.get(name, "")
         value = data.get(key)
         return "" if value is None else os.fsdecode(value)
@@ -176,7 +178,8 @@ def _on_gpu(t: torch.Tensor, op: str) -> None:
     if force_ref():
         raise HardwareUnsupported(f"{op}: FORGE_FORCE_REF=1 asks for the torch reference path, which forge_amd does "
                                   "not include (run the reference implementation for that)")
-    _THREAD.gathered = False
+    if _gathers:
+        _THREAD.gathered = False
     _lib.require_device(t, op)
     if not _SELFTEST.passed(t.get_device()):
         _SELFTEST.ensure(t)
@@ -432,11 +435,12 @@ def _w4_operands(packed: PackedW4, x: torch.Tensor) -> _W4Operands:
 
 def _gather_columns(x2: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
     """``x2[:, perm]``, in rows that start on 16 bytes: the activations in a sorted act-order weight's column order."""
+    global _gathers
     m, k = x2.shape
     out = torch.empty((m, (k + 7) // 8 * 8), dtype=x2.dtype, device=x2.device)
     _check(_lib.lib().fg_w4_gather_columns(_lib.ptr(x2), _ld(x2), _lib.ptr(perm), _lib.ptr(out), out.stride(0), m, k,
                                            _lib.stream_of(x2)), "fg_w4_gather_columns")
-    _THREAD.gathered = True
+    _THREAD.gathered = _gathers = True
     return out[:, :k]
 
 
